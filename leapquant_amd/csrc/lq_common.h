@@ -257,6 +257,8 @@ __device__ __forceinline__ char* block_base(const lq_state& st, int slot, int hv
 }
 
 // ---- checks and launches shared by the entry points of different source files (not exported) ----------------------
+// compute units of the current device: what grids and launch rules are sized by
+__attribute__((visibility("hidden"))) int lq_num_cus();
 // the argument checks of lq_gdn_step / lq_kda_step (the KDA step also needs Gbuf and K = V = 128) and of lq_flush
 __attribute__((visibility("hidden"))) int lq_check_step(const lq_state* st, const lq_step_io* io);
 __attribute__((visibility("hidden"))) int lq_check_flush(const lq_state* st, const float* Q0, const int* idx, int N,

@@ -972,6 +972,14 @@ constexpr int FT4 = 256;             // threads per workgroup
 constexpr int NW4 = FT4 / 64;        // waves
 constexpr int HALF = 32;             // window entries staged at once
 constexpr int OPS4 = HALF + 8;       // operand row stride (bf16): 80 B rows, 16-byte aligned, conflict-free b128 reads
+// thread, lane and wave within the 256 threads that work on a head (a workgroup of 512 flushes two heads side by side)
+__device__ __forceinline__ int tid4() {
+  int t = threadIdx.x & (FT4 - 1);
+  asm volatile("" : "+v"(t));
+  return t;
+}
+__device__ __forceinline__ int lane4() { return tid4() & 63; }
+__device__ __forceinline__ int wave4() { return __builtin_amdgcn_readfirstlane(tid4() >> 6); }
 // CF (conflict-free layout): the factor tables [4][128] fp16 are read by the four lane rows of a 16-lane group at once
 // (row l & 3, same column), and rows of 128 halfs all start in the same bank, so each row is padded by 16 halfs (rows
 // then start 8 banks apart); the row-maximum table [16][128] fp32 is written by the four lane groups at once (row
@@ -1027,7 +1035,7 @@ __device__ __forceinline__ void load_half(WinHalf& r, const lq_state& st, int sl
   const bf16_t* Kb = (const bf16_t*)st.Kbuf + ((long long)slot * st.H + hk) * L * K_;
   const bf16_t* Ub = (const bf16_t*)st.Ubuf + ((long long)slot * st.HV + hv) * L * V_;
   const f16_t* Gb = KDA ? (const f16_t*)st.Gbuf + ((long long)slot * st.HV + hv) * L * KD : nullptr;
-  const int t = opaque_tid(), jp = t % 16, c8 = (t / 16) * 8;
+  const int t = tid4(), jp = t % 16, c8 = (t / 16) * 8;
   const uint4 z = make_uint4(0u, 0u, 0u, 0u);        // columns past a K_ / V_ < 128 head: zero operands
 #pragma unroll
   for (int k = 0; k < 2; ++k) {
@@ -1050,7 +1058,7 @@ template <bool KDA = false, bool CF>
 __device__ __forceinline__ void store_half(FlushShared4T<CF>& sh, const WinHalf& r, int h, int hf) {
   // the split is of the fp32-rounded product: no fusing of w u into the lo subtraction (kernels.py:1509-1511)
 #pragma clang fp contract(off)
-  const int t = opaque_tid(), jl = 2 * (t % 16), c8 = (t / 16) * 8;
+  const int t = tid4(), jl = 2 * (t % 16), c8 = (t / 16) * 8;
   const bool rot = CF && ((t / 16) & 1);
   const int j0 = HALF * hf + jl;
   const bool v0 = j0 < h, v1 = j0 + 1 < h;
@@ -1112,7 +1120,7 @@ __device__ __forceinline__ float kda_key_scan4(FlushShared4T<CF>& sh, float dcar
   // the split is of the fp32-rounded product (kernels.py:1456-1463): no fusing into the first subtraction
 #pragma clang fp contract(off)
   static_assert(NT == 2 || NT == 3, "two or three bf16 terms");
-  const int t = opaque_tid(), c = t >> 1, s = t & 1, jb = 16 * s, j0 = HALF * hf + jb;
+  const int t = tid4(), c = t >> 1, s = t & 1, jb = 16 * s, j0 = HALF * hf + jb;
   uint32_t ku[8], eu[8];
 #pragma unroll
   for (int x = 0; x < 2; ++x) {
@@ -1161,7 +1169,7 @@ __device__ __forceinline__ float kda_key_scan4(FlushShared4T<CF>& sh, float dcar
 // us at config 3)
 __device__ __forceinline__ void rebuild_half4x2(Tile4& t, const bf16_t (*A)[OPS4], const bf16_t (*B1)[OPS4],
                                                 const bf16_t (*B2)[OPS4]) {
-  const int l = lane_id(), w = wave_id(), q = l >> 4;
+  const int l = lane4(), w = wave4(), q = l >> 4;
   bf16x8 af[2];
 #pragma unroll
   for (int g = 0; g < 2; ++g) af[g] = *(const bf16x8*)&A[32 * w + 16 * g + (l & 15)][8 * q];
@@ -1191,7 +1199,7 @@ __device__ __forceinline__ void rebuild_half4x2(Tile4& t, const bf16_t (*A)[OPS4
 // accumulator takes its hi term, then its lo term
 __device__ __forceinline__ void rebuild_half4x2a(Tile4& t, const bf16_t (*A1)[OPS4], const bf16_t (*A2)[OPS4],
                                                  const bf16_t (*B)[OPS4]) {
-  const int l = lane_id(), w = wave_id(), q = l >> 4;
+  const int l = lane4(), w = wave4(), q = l >> 4;
   bf16x8 a1[2], a2[2];
 #pragma unroll
   for (int g = 0; g < 2; ++g) {
@@ -1223,7 +1231,7 @@ __device__ __forceinline__ void rebuild_half4x2a(Tile4& t, const bf16_t (*A1)[OP
 }
 // acc[c][v] += sum_j A[c][j] B[v][j] over one staged half, one bf16 term (the prefill dequant's third key term)
 __device__ __forceinline__ void rebuild_half4x1(Tile4& t, const bf16_t (*A)[OPS4], const bf16_t (*B)[OPS4]) {
-  const int l = lane_id(), w = wave_id(), q = l >> 4;
+  const int l = lane4(), w = wave4(), q = l >> 4;
   bf16x8 af[2];
 #pragma unroll
   for (int g = 0; g < 2; ++g) af[g] = *(const bf16x8*)&A[32 * w + 16 * g + (l & 15)][8 * q];
@@ -1242,7 +1250,7 @@ __device__ __forceinline__ void rebuild_half4x1(Tile4& t, const bf16_t (*A)[OPS4
 // lane group j needs, so a 4 x 4 transpose over the lane groups (two swap32, two swap16) delivers it.
 template <int K_, int V_>
 __device__ __forceinline__ void load_code_words4(uint32_t wds[2][8], const int8_t* Sq) {
-  const int l = lane_id(), w = wave_id(), q = l >> 4;
+  const int l = lane4(), w = wave4(), q = l >> 4;
   if constexpr (K_ == KD && V_ == VD) {
     const int l16 = l & 15;
     uint4 x[4];
@@ -1279,7 +1287,7 @@ __device__ __forceinline__ void load_code_words4(uint32_t wds[2][8], const int8_
 __device__ __forceinline__ void tile_add_words4(Tile4& t, const uint32_t wds[2][8], const float* svr,
                                                 const float* skl) {
 #pragma clang fp contract(off)
-  const int l = lane_id(), w = wave_id(), q = l >> 4;
+  const int l = lane4(), w = wave4(), q = l >> 4;
 #pragma unroll
   for (int g = 0; g < 2; ++g) {
     const int c0 = 32 * w + 16 * g + 4 * q;
@@ -1300,8 +1308,8 @@ __device__ __forceinline__ void tile_add_words4(Tile4& t, const uint32_t wds[2][
 // instructions where sixteen readlanes were VALU ones
 template <bool CF>
 __device__ __forceinline__ void bcast4x4(const FlushShared4T<CF>& sh, const f32x4& acc, float M[4][4]) {
-  const int l = lane_id();
-  f32x4* mb = const_cast<f32x4*>(sh.r.mb[wave_id()]);
+  const int l = lane4();
+  f32x4* mb = const_cast<f32x4*>(sh.r.mb[wave4()]);
   if (l < 4) mb[l] = acc;
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -1315,7 +1323,7 @@ __device__ __forceinline__ void bcast4x4(const FlushShared4T<CF>& sh, const f32x
 // M[a][r] = sum_v Q_old[v][a] Q[v][r] (Q from sh.qT): every lane gets all 16 entries
 template <bool CF>
 __device__ __forceinline__ void gram_qold_q(const FlushShared4T<CF>& sh, float M[4][4]) {
-  const int l = lane_id(), q = l >> 4, l16 = l & 15;
+  const int l = lane4(), q = l >> 4, l16 = l & 15;
   f32x4 macc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int ks = 0; ks < 4; ++ks) {
@@ -1335,7 +1343,7 @@ __device__ __forceinline__ void gram_qold_q(const FlushShared4T<CF>& sh, float M
 template <bool TR, bool CF>
 __device__ __forceinline__ void p_step4(const FlushShared4T<CF>& sh, const f16x4 (&bh)[2][8], f16x4 (&bt)[2][8], float pn,
                                         int R, f32x4& pg) {
-  const int l = lane_id(), w = wave_id(), q = l >> 4, l16 = l & 15;
+  const int l = lane4(), w = wave4(), q = l >> 4, l16 = l & 15;
   float M[4][4];
   gram_qold_q(sh, M);
   f16x4 ident;
@@ -1367,7 +1375,7 @@ __device__ void flush_head4(FlushShared4T<CF>& sh, const lq_state& st, const flo
   static_assert(!KDA || (K_ == KD && V_ == VD), "KDA heads are 128 x 128");
   const int HV = st.HV, L = st.L, R = st.R;
   const long long sh_ = (long long)slot * HV + hv;
-  const int tid = opaque_tid(), l = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), q = l >> 4, l16 = l & 15;
+  const int tid = tid4(), l = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), q = l >> 4, l16 = l & 15;
   char* base = block_base(st, slot, hv);
   int8_t* Sq = (int8_t*)base;
   float* Sk = (float*)(base + V_ * K_);

@@ -10,7 +10,7 @@
 //     the int8 tile, bf16 / fp16 MFMA for the window-key and factor dots), fed by 16-byte loads issued up front.
 //   * KDA (K = V = 128): two waves per value head, the same matrix-core dots, the per-channel gate folded into the
 //     key operands and the window's decayed keys formed by a backward scan split between the two waves.
-#include "lq_flush_core.h"
+#include "lq_flush64_core.h"
 
 namespace {
 
@@ -56,19 +56,28 @@ constexpr float KSPLIT = 64.0f;   // kn / qn scaled by 2^6 before the fp16 hi / 
 // The MFMA B-operand tables (dig, bkq, hkq) are read as 16-byte fragments of up to six rows at once: their rows are
 // padded by 16 bytes so that those rows start in different LDS banks (unpadded, 128- or 256-byte rows all start in
 // the same bank).
+// The GEMV rows take the bytes of the window's dot operands, which no wave reads past the barrier before the GEMV, and an
+// entry's weight waits where its first coefficient goes: at K = V = 128 and G = 1 two units then fit the 40 KiB of four
+// workgroups per CU (the hkq rows unpadded there).
 constexpr int DIGP = 16, OPP = 8;
 template <int K_, int V_, int G, int RM>
 struct StepShared {
+  static constexpr int HPP = G == 1 && RM == 4 && K_ == 128 ? 0 : OPP;
   bf16_t ub[G][LMAX][V_];  // the window's u_j rows per value head (direct global -> LDS loads)
   int8_t dig[G][6][K_ + DIGP];   // int8 GEMV B operand: k digits 0-2, q digits 0-2
-  bf16_t bkq[6][K_ + OPP];       // key-dot B operand: bf16 hi / mid / lo of kn, then of qn
-  f16_t hkq[4][K_ + OPP];        // factor-dot B operand: fp16 hi / lo of 64 kn, then of 64 qn
-  float2 mq[G][V_];        // GEMV rows (k, q) in digit units
-  float2 cwq[G][LMAX];     // (w_j dk_j, w_j dq_j) per value head: buffered entry j's coefficients in A4 / A5
+  union {
+    struct {
+      bf16_t bkq[6][K_ + OPP];   // key-dot B operand: bf16 hi / mid / lo of kn, then of qn
+      f16_t hkq[4][K_ + HPP];    // factor-dot B operand: fp16 hi / lo of 64 kn, then of 64 qn
+    };
+    float2 mq[G][V_];      // GEMV rows (k, q) in digit units
+  };
+  float2 cwq[G][LMAX];     // (w_j dk_j, w_j dq_j) per value head: buffered entry j's coefficients in A4 / A5; the gated
+                           // weight w_j in .x until the key dots are done
   float2 duq[G][RM];       // (dU_r, dQ_r) per value head, factor r
-  float w[G][LMAX];        // gated entry weights w_j per value head
   float sc[G][8];          // per value head: alpha, beta, kappa, kmax, qmax
 };
+static_assert(2 * sizeof(StepShared<128, 128, 1, 4>) <= 40960, "two units in the LDS of four workgroups per CU");
 
 // ------------------------------------------------------------------------------------------------------------------
 // GDN step  (kernels.py:129-144 gate / beta, 236-279 norms and weights, 380-585 stream, dots and appends)
@@ -85,36 +94,74 @@ struct StepShared {
 // The per-head scalar work (norms, gate, beta, digits) runs in one wave per value head.  The window's u_j rows reach
 // LDS by direct global -> LDS loads.  <= 128 VGPRs and < 40 KiB LDS: four workgroups per CU, the whole B = 64 x H = 16
 // grid resident at once.
-// FL (fused flush, K = V = 128 and G = 2 only): after its step the workgroup flushes the heads whose window it has just
-// filled (or found full), with the four-wave flush of lq_flush_core.h over the same 256 threads -- one launch per decode
-// call instead of two.  The step's LDS and the flush's share the same bytes (both fit the 40 KiB that four workgroups
-// per CU allow).
+// FL (fused flush): after its step the workgroup flushes the heads whose window it has just filled (or found full), with
+// the four-wave flush of lq_flush_core.h (lq_flush64_core.h) over the same threads -- one launch per decode call instead
+// of two.  The step's LDS and the flush's share the same bytes.  A workgroup of 256 threads flushes its heads one after
+// the other; one of 512 (G = 4) two at a time, one per 256 threads, which pass the same barriers: when only one head of
+// a pair is due, both halves flush it (every load of a flush precedes its first store by a barrier, and both store the
+// same bytes).  At G = 1 a unit is 128 threads, so a workgroup of the fused kernel takes UW = 2 units, the key heads
+// hk, hk + 1 of one row, coupled by the barriers alone.
 // ------------------------------------------------------------------------------------------------------------------
 // waves per value head of the step: V / 64, and two at V = 64 (each wave then owns 32 rows of the tile), so that a
 // 64-row head's bytes are requested by as many waves as a 128-row head's
 template <int V_>
 constexpr int step_wph() { return V_ == 64 ? 2 : V_ / 64; }
 
+// UW: units (key heads) per workgroup
+template <int G, bool FL>
+constexpr int step_units() { return FL && G == 1 ? 2 : 1; }
+
 template <int K_, int V_, int G, bool FL, int RM>
 struct StepLds {
-  StepShared<K_, V_, G, RM> st;
+  StepShared<K_, V_, G, RM> st[1];
 };
+template <int K_>
+struct FlushLds { using type = lqf::FlushShared4T<true>; };
+template <>
+struct FlushLds<64> { using type = lqf::FlushShared64; };
 template <int K_, int V_, int G, int RM>
 struct StepLds<K_, V_, G, true, RM> {
   union {
-    StepShared<K_, V_, G, RM> st;
-    lqf::FlushShared4T<true> fl;
+    StepShared<K_, V_, G, RM> st[step_units<G, true>()];
+    typename FlushLds<K_>::type fl[G == 4 ? 2 : 1];
   };
 };
+
+// Flushes the due ones of the NH value heads hv0 .. of one row (bit i of due: head hv0 + i), all of one slot: uniform
+// over the workgroup, which has NH = 2 heads on 256 threads or 4 on 512.
+template <int K_, int V_, int G, int NH, class LDS>
+__device__ __forceinline__ void flush_due(LDS& lds, const lq_state& st, const float* Q0, int slot, int hv0,
+                                          unsigned due, float qm) {
+  const int sub = NH == 4 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;   // this thread's half of 512
+  if constexpr (K_ == 64 && V_ == 64 && G % 2 == 0) {  // pairs of heads of one key head, the mask naming the due ones
+    int p = sub;
+    unsigned m = (due >> (2 * p)) & 3u;
+    if (NH == 4 && m == 0) m = (due >> (2 * (p ^= 1))) & 3u;
+    lqf::flush_head64<64, 2>(lds.fl[sub], st, Q0, slot, hv0 + 2 * p, m, qm);
+  } else {
+#pragma unroll 1
+    for (int p = 0; p < 2; ++p) {
+      int i = NH == 4 ? 2 * p + sub : p;
+      if (NH == 4) {
+        if (((due >> (2 * p)) & 3u) == 0) continue;
+        if (!((due >> i) & 1u)) i ^= 1;
+      } else if (!((due >> i) & 1u)) {
+        continue;
+      }
+      if constexpr (K_ == 64) lqf::flush_head64<V_, 1>(lds.fl[sub], st, Q0, slot, hv0 + i, 1u, qm);
+      else lqf::flush_head4<K_, V_, true>(lds.fl[sub], st, Q0, slot, hv0 + i, qm);
+    }
+  }
+}
 
 // RM: factors held per head.  4 (R <= 4): the G R <= 16 factor rows of the workgroup's heads are one MFMA tile, taken
 // by the last wave.  16 (the rank ablation R <= 16, K = V = 128; kernels.py:63, 457-469): up to G tiles, tile g taken
 // by the second wave of head g.
-template <int K_, int V_, int G, bool CONV, bool FL, int RM = 4, bool DF = false>
-__global__ __launch_bounds__(64 * step_wph<V_>() * G) __attribute__((amdgpu_waves_per_eu(4)))
-void gdn_step_kernel(lq_state st, lq_step_io io, lq_conv cv, int* dlist, const float* Q0) {
+template <int K_, int V_, int G, bool CONV, bool FL, int RM, bool DF>
+__device__ __forceinline__ void gdn_step(const lq_state& st, const lq_step_io& io, const lq_conv& cv, int* dlist,
+                                         const float* Q0) {
   static_assert(!DF || FL, "deferred flush (lq_gdn_decode_deferred): the fused decode kernel");
-  static_assert(!FL || (K_ == 128 && V_ == 128 && G == 2), "fused flush: the four-wave layout, 128 x 128 heads");
+  static_assert(!DF || (K_ == 128 && V_ == 128 && G == 2), "deferred flush: 128 x 128 heads, two per key head");
   static_assert(RM == 4 || (RM == 16 && K_ == 128 && V_ == 128 && !FL), "ranks above 4: 128 x 128 heads, no fused flush");
   constexpr int KD = K_, VD = V_;
   constexpr int WPH = step_wph<V_>();   // waves per value head
@@ -122,13 +169,16 @@ void gdn_step_kernel(lq_state st, lq_step_io io, lq_conv cv, int* dlist, const f
   constexpr int NE = KD / 64;   // channels per lane in the scalar work
   constexpr int KS32 = KD / 32, KS64 = KD / 64;   // k-steps of the 16x16x32 (bf16 / fp16) and 16x16x64 (int8) MFMAs
   constexpr bool NT = KD == 128;                  // non-temporal bulk loads (see ld_once)
+  constexpr int UW = step_units<G, FL>(), NH = UW * G;      // units, and value heads, of the workgroup
   __shared__ StepLds<K_, V_, G, FL, RM> lds;
-  StepShared<K_, V_, G, RM>& sh = lds.st;
   const int H = st.H, HV = st.HV, L = st.L, R = st.R;
-  const int n = blockIdx.x / H;
-  const int hk = blockIdx.x - n * H;
-  const int tid = threadIdx.x;
-  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave in the workgroup
+  const int n = blockIdx.x / (H / UW);
+  const int hk0 = (blockIdx.x - n * (H / UW)) * UW;         // the workgroup's first key head
+  const int un = UW == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * WPH * G));   // this wave's unit
+  const int hk = hk0 + un;
+  StepShared<K_, V_, G, RM>& sh = lds.st[un];
+  const int tid = UW == 1 ? threadIdx.x : threadIdx.x % (64 * WPH * G);   // thread in the unit
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave in the unit
   const int g = wv / WPH;       // value head of this wave within the key head
   const int wi = wv % WPH;      // its tile part: rows RW wi ..
   const int lane = tid & 63;
@@ -153,7 +203,7 @@ void gdn_step_kernel(lq_state st, lq_step_io io, lq_conv cv, int* dlist, const f
         const float qm = code_range(st);
 #pragma unroll
         for (int g2 = 0; g2 < G; ++g2)
-          if ((pend >> g2) & 1u) lqf::flush_head4<128, 128, true>(lds.fl, st, Q0, slot0, hk * G + g2, qm);
+          if ((pend >> g2) & 1u) lqf::flush_head4<128, 128, true>(lds.fl[0], st, Q0, slot0, hk * G + g2, qm);
       }
     }
   }
@@ -216,11 +266,14 @@ void gdn_step_kernel(lq_state st, lq_step_io io, lq_conv cv, int* dlist, const f
 #pragma unroll
   for (int r = 0; r < RM; ++r) qt[r] = h2f(UQp[min(r, R - 1) * (KD + VD) + KD + lt]);
   const float P = st.Pbuf[sh_];
-  // Window fills of the G value heads: uniform loads, served by the scalar data cache.  A vector load here would queue
+  // Window fills of the value heads: uniform loads, served by the scalar data cache.  A vector load here would queue
   // behind the bulk loads the CU's other workgroups have issued, and every later load of this workgroup waits for it.
-  int hg[G];
+  int hw[NH];                   // the workgroup's heads
 #pragma unroll
-  for (int g2 = 0; g2 < G; ++g2) hg[g2] = st.hcnt[(long long)slot * HV + hk * G + g2];
+  for (int i = 0; i < NH; ++i) hw[i] = st.hcnt[(long long)slot * HV + hk0 * G + i];
+  int hg[G];                    // the unit's
+#pragma unroll
+  for (int g2 = 0; g2 < G; ++g2) hg[g2] = UW == 1 || un == 0 ? hw[g2] : hw[NH - G + g2];
   __builtin_amdgcn_sched_barrier(0);
   // ---- per value head scalar work, one wave (wi = 0), before the window fills arrive: gate, beta, norms, digits,
   //      key-dot operands.  Its global writes (key append, gated weights) wait until the end, so that nothing joins
@@ -329,7 +382,7 @@ void gdn_step_kernel(lq_state st, lq_step_io io, lq_conv cv, int* dlist, const f
   bool flush_after = false;
   if constexpr (FL) {
 #pragma unroll
-    for (int g2 = 0; g2 < G; ++g2) flush_after = flush_after || hg[g2] >= L - 1;
+    for (int i = 0; i < NH; ++i) flush_after = flush_after || hw[i] >= L - 1;
   }
   if (!CONV && G <= 2 && !flush_after) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   int h = hg[0], hmax = hg[0];
@@ -344,7 +397,7 @@ void gdn_step_kernel(lq_state st, lq_step_io io, lq_conv cv, int* dlist, const f
 #pragma unroll
     for (int e = 0; e < NE; ++e) {
       const int c = lane + 64 * e;
-      if (c < h) sh.w[g][c] = wjv[e];
+      if (c < h) sh.cwq[g][c].x = wjv[e];
     }
   }
   // The big loads, in the order the work after them needs them: the window (values u_j into LDS, then the buffered
@@ -396,7 +449,7 @@ void gdn_step_kernel(lq_state st, lq_step_io io, lq_conv cv, int* dlist, const f
     for (int e = 0; e < NE; ++e) {
       wjv[e] = wx[e] * alpha;
       const int c = lane + 64 * e;
-      if (live && c < h) sh.w[g][c] = wjv[e];
+      if (live && c < h) sh.cwq[g][c].x = wjv[e];
     }
     if (lane == 0) { sh.sc[g][0] = alpha; sh.sc[g][1] = beta; }
   }
@@ -439,7 +492,12 @@ void gdn_step_kernel(lq_state st, lq_step_io io, lq_conv cv, int* dlist, const f
           const int j = j0 + 4 * q4 + i;
           if ((n16 == 0 || n16 == 4) && j < hmax) {
 #pragma unroll
-            for (int g2 = 0; g2 < G; ++g2) ((float*)&sh.cwq[g2][j])[n16 >> 2] = sh.w[g2][j] * s;
+            for (int g2 = 0; g2 < G; ++g2) {          // both lanes read w_j in one instruction, then write
+              float* cw = (float*)&sh.cwq[g2][j];
+              const float w = cw[0];
+              __builtin_amdgcn_wave_barrier();
+              cw[n16 >> 2] = w * s;
+            }
           }
         }
       }
@@ -564,25 +622,33 @@ void gdn_step_kernel(lq_state st, lq_step_io io, lq_conv cv, int* dlist, const f
   if constexpr (FL) {
     // the flush of this workgroup's heads whose window is now full (hcnt was L - 1 before the step, or already L):
     // the fills are uniform loads, so every wave takes the same branch and reaches the same barriers
-    bool due[G], any = false;
+    unsigned due = 0;
 #pragma unroll
-    for (int g2 = 0; g2 < G; ++g2) {
-      due[g2] = hg[g2] >= L - 1;
-      any = any || due[g2];
-    }
-    if (any) {
+    for (int i = 0; i < NH; ++i) due |= (hw[i] >= L - 1 ? 1u : 0u) << i;
+    if (due) {
       __syncthreads();          // the step is done with the shared bytes, and its appends are visible to the workgroup
       const float qm = code_range(st);
-      bool first = true;        // DF: the first due head now, the others at the start of the next call
-#pragma unroll
-      for (int g2 = 0; g2 < G; ++g2)
-        if (due[g2]) {
-          if (!DF || first) lqf::flush_head4<128, 128, true>(lds.fl, st, Q0, slot, hk * G + g2, qm);
-          else if (tid == 0) note_due(st.ctl, dlist, n * HV + hk * G + g2);   // a standalone flush finds it
-          first = false;
-        }
+      if constexpr (DF) {       // the first due head now, the other at the start of the next call
+        lqf::flush_head4<128, 128, true>(lds.fl[0], st, Q0, slot, hk * G + (due & 1u ? 0 : 1), qm);
+        if (due == 3u && tid == 0) note_due(st.ctl, dlist, n * HV + hk * G + 1);   // a standalone flush finds it
+      } else {
+        flush_due<K_, V_, G, NH>(lds, st, Q0, slot, hk0 * G, due, qm);
+      }
     }
   }
+}
+
+template <int K_, int V_, int G, bool CONV, bool FL, int RM = 4, bool DF = false>
+__global__ __launch_bounds__(64 * step_wph<V_>() * G) __attribute__((amdgpu_waves_per_eu(4)))
+void gdn_step_kernel(lq_state st, lq_step_io io, lq_conv cv, int* dlist, const float* Q0) {
+  gdn_step<K_, V_, G, CONV, FL, RM, DF>(st, io, cv, dlist, Q0);
+}
+// the one-launch decode at GQA 1: W = 2 value heads, of two key heads, per workgroup
+template <int K_, int V_, int W, bool CONV>
+__global__ __launch_bounds__(64 * step_wph<V_>() * W) __attribute__((amdgpu_waves_per_eu(4)))
+void gdn_step_kernel(lq_state st, lq_step_io io, lq_conv cv, const float* Q0) {
+  static_assert(W == step_units<1, true>(), "value heads of a workgroup");
+  gdn_step<K_, V_, 1, CONV, true, 4, false>(st, io, cv, nullptr, Q0);
 }
 
 // ------------------------------------------------------------------------------------------------------------------
@@ -1030,6 +1096,38 @@ static int launch_gdn_dims(const lq_state* st, const lq_step_io* io, const lq_co
   return st->V == 128 ? launch_gdn<64, 128, CONV>(st, io, cv, dlist, s) : launch_gdn<64, 64, CONV>(st, io, cv, dlist, s);
 }
 
+// the decode call in one launch: each workgroup flushes the heads whose window it fills
+template <int K_, int V_, bool CONV>
+static int launch_decode(const lq_state* st, const lq_step_io* io, const lq_conv& cv, const float* Q0, hipStream_t s) {
+  const int G = st->HV / st->H;
+  const dim3 grid((unsigned)(io->N * (G == 1 ? st->H / 2 : st->H)));
+  switch (G) {
+    case 1: gdn_step_kernel<K_, V_, 2, CONV><<<grid, 128 * step_wph<V_>(), 0, s>>>(*st, *io, cv, Q0); break;
+    case 2: gdn_step_kernel<K_, V_, 2, CONV, true><<<grid, 128 * step_wph<V_>(), 0, s>>>(*st, *io, cv, nullptr, Q0); break;
+    case 4: gdn_step_kernel<K_, V_, 4, CONV, true><<<grid, 256 * step_wph<V_>(), 0, s>>>(*st, *io, cv, nullptr, Q0); break;
+    default: return LQ_ERR_ARG;
+  }
+  return hipGetLastError() == hipSuccess ? LQ_OK : LQ_ERR_HIP;
+}
+template <bool CONV>
+static int launch_decode_dims(const lq_state* st, const lq_step_io* io, const lq_conv& cv, const float* Q0,
+                              hipStream_t s) {
+  if (st->K == 128) return launch_decode<128, 128, CONV>(st, io, cv, Q0, s);
+  return st->V == 128 ? launch_decode<64, 128, CONV>(st, io, cv, Q0, s) : launch_decode<64, 64, CONV>(st, io, cv, Q0, s);
+}
+// Which calls take one launch.  The second launch, the flush, costs a call ~2 us also when nothing is due.  Window 16,
+// us per call, two launches -> one: 128 x 128 at GQA 4, B = 24, 16 key heads 16.5 -> 14.8, B = 200 78.2 -> 75.4; at GQA 1,
+// B = 64, 32 heads 21.0 -> 16.4, B = 200 45.8 -> 41.7; (64, 128) at GQA 2, B = 64 13.0 -> 10.5; (64, 64) at GQA 1,
+// B = 64 10.9 -> 8.5.  GQA 1 pairs two key heads of a row in a workgroup, so an odd H takes two launches.  So do large
+// (64, 64) batches at GQA 4, whose flush needs twice the step's LDS and registers (two workgroups per CU against the
+// step's four): 16.6 -> 14.3 us at 4 workgroups per CU, 20.9 -> 20.0 at 6, 25.2 -> 25.6 at 8, 35.7 -> 39.0 at 12.
+static bool one_launch(const lq_state* st, int N) {
+  const int G = st->HV / st->H;
+  if (st->R > 4 || (G == 1 && st->H % 2 != 0)) return false;
+  if (G == 4 && st->V == 64) return (long long)N * st->H <= 6ll * lq_num_cus();
+  return G == 1 || G == 2 || G == 4;
+}
+
 // the plain GDN / KDA step of every row, arguments already checked
 int lq_launch_step(const lq_state* st, const lq_step_io* io, int kda, float glb, int* dlist, hipStream_t s) {
   if (io->N == 0) return LQ_OK;
@@ -1075,18 +1173,15 @@ static int gdn_decode(const lq_state* st, const lq_step_io* io, const lq_conv* c
   const float qmax = st->qmax > 0.f ? st->qmax : LQ_QMAX;
   if ((rc = lq_check_flush(st, Q0, io->idx, io->N, 0, qmax))) return rc;
   if (io->N == 0) return LQ_OK;
-  if (st->K == 128 && st->V == 128 && st->HV == 2 * st->H && st->R <= 4) {   // one launch: the step flushes its own due heads
+  if (deferred && st->K == 128 && st->V == 128 && st->HV == 2 * st->H && st->R <= 4) {
     const dim3 grid((unsigned)(io->N * st->H));
     const lq_conv none = {};
-    if (deferred) {
-      if (cv) gdn_step_kernel<128, 128, 2, true, true, 4, true><<<grid, 256, 0, s>>>(*st, *io, *cv, nullptr, Q0);
-      else gdn_step_kernel<128, 128, 2, false, true, 4, true><<<grid, 256, 0, s>>>(*st, *io, none, nullptr, Q0);
-    } else {
-      if (cv) gdn_step_kernel<128, 128, 2, true, true><<<grid, 256, 0, s>>>(*st, *io, *cv, nullptr, Q0);
-      else gdn_step_kernel<128, 128, 2, false, true><<<grid, 256, 0, s>>>(*st, *io, none, nullptr, Q0);
-    }
+    if (cv) gdn_step_kernel<128, 128, 2, true, true, 4, true><<<grid, 256, 0, s>>>(*st, *io, *cv, nullptr, Q0);
+    else gdn_step_kernel<128, 128, 2, false, true, 4, true><<<grid, 256, 0, s>>>(*st, *io, none, nullptr, Q0);
     return hipGetLastError() == hipSuccess ? LQ_OK : LQ_ERR_HIP;
   }
+  if (one_launch(st, io->N))
+    return cv ? launch_decode_dims<true>(st, io, *cv, Q0, s) : launch_decode_dims<false>(st, io, lq_conv{}, Q0, s);
   rc = cv ? launch_gdn_dims<true>(st, io, *cv, nullptr, s) : lq_launch_step(st, io, 0, 0.f, nullptr, s);
   if (rc) return rc;
   return lq_launch_flush(st, Q0, io->idx, io->N, 0, qmax, nullptr, s);

@@ -167,7 +167,7 @@ class LeapQuantState:
         if self.kda:                 # the step, then the flush of the heads it fills
             _lib.check(L.lq_kda_decode(ctypes.byref(st), ctypes.byref(io), ctypes.c_float(self.glb), KN._p(self.Q0),
                                        stream), "lq_kda_decode")
-        else:                        # step + flush of the heads it fills (one launch for 128 x 128 heads, GQA 2)
+        else:                        # step + flush of the heads it fills (one launch at ranks up to 4)
             fn = L.lq_gdn_decode_deferred if self.defer_flush else L.lq_gdn_decode
             _lib.check(fn(ctypes.byref(st), ctypes.byref(io), None, KN._p(self.Q0), stream), "lq_gdn_decode")
 
