@@ -97,10 +97,11 @@ static_assert(2 * sizeof(StepShared<128, 128, 1, 4>) <= 40960, "two units in the
 // FL (fused flush): after its step the workgroup flushes the heads whose window it has just filled (or found full), with
 // the four-wave flush of lq_flush_core.h (lq_flush64_core.h) over the same threads -- one launch per decode call instead
 // of two.  The step's LDS and the flush's share the same bytes.  A workgroup of 256 threads flushes its heads one after
-// the other; one of 512 (G = 4) two at a time, one per 256 threads, which pass the same barriers: when only one head of
-// a pair is due, both halves flush it (every load of a flush precedes its first store by a barrier, and both store the
-// same bytes).  At G = 1 a unit is 128 threads, so a workgroup of the fused kernel takes UW = 2 units, the key heads
-// hk, hk + 1 of one row, coupled by the barriers alone.
+// the other; a larger one several side by side, one per group of 256 threads, which pass the same barriers: a group whose
+// head is not due joins a due one (every load of a flush precedes its first store by a barrier, and both store the same
+// bytes).  At G = 1 a unit is 128 threads, so a workgroup of the fused kernel takes UW = 2 units, the key heads hk, hk + 1
+// of one row, coupled by the barriers alone.  Small launches add waves that only flush, 256 threads per value head, so
+// that a workgroup's heads are flushed at the same time (the kernels with helper waves below).
 // ------------------------------------------------------------------------------------------------------------------
 // waves per value head of the step: V / 64, and two at V = 64 (each wave then owns 32 rows of the tile), so that a
 // 64-row head's bytes are requested by as many waves as a 128-row head's
@@ -126,28 +127,33 @@ struct StepLds<K_, V_, G, true, RM> {
     typename FlushLds<K_>::type fl[G == 4 ? 2 : 1];
   };
 };
+// with helper waves: one unit, and a flush per value head
+template <int K_, int V_, int G>
+struct WideLds {
+  union {
+    StepShared<K_, V_, G, 4> st[1];
+    typename FlushLds<K_>::type fl[G];
+  };
+};
 
-// Flushes the due ones of the NH value heads hv0 .. of one row (bit i of due: head hv0 + i), all of one slot: uniform
-// over the workgroup, which has NH = 2 heads on 256 threads or 4 on 512.
-template <int K_, int V_, int G, int NH, class LDS>
+// Flushes the due ones of the NH value heads hv0 .. of one row (bit i of due: head hv0 + i), all of one slot, on NG
+// groups of 256 threads; `due` (not zero) is uniform over the workgroup.
+template <int K_, int V_, int G, int NH, int NG, class LDS>
 __device__ __forceinline__ void flush_due(LDS& lds, const lq_state& st, const float* Q0, int slot, int hv0,
                                           unsigned due, float qm) {
-  const int sub = NH == 4 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;   // this thread's half of 512
+  const int sub = NG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;   // this thread's group
   if constexpr (K_ == 64 && V_ == 64 && G % 2 == 0) {  // pairs of heads of one key head, the mask naming the due ones
+    static_assert(NH == 2 * NG, "one pair per group");
     int p = sub;
     unsigned m = (due >> (2 * p)) & 3u;
-    if (NH == 4 && m == 0) m = (due >> (2 * (p ^= 1))) & 3u;
+    if (NG == 2 && m == 0) m = (due >> (2 * (p ^= 1))) & 3u;
     lqf::flush_head64<64, 2>(lds.fl[sub], st, Q0, slot, hv0 + 2 * p, m, qm);
   } else {
 #pragma unroll 1
-    for (int p = 0; p < 2; ++p) {
-      int i = NH == 4 ? 2 * p + sub : p;
-      if (NH == 4) {
-        if (((due >> (2 * p)) & 3u) == 0) continue;
-        if (!((due >> i) & 1u)) i ^= 1;
-      } else if (!((due >> i) & 1u)) {
-        continue;
-      }
+    for (int p = 0; p < NH / NG; ++p) {                // heads NG p .. NG p + NG - 1 at a time
+      const unsigned m = (due >> (NG * p)) & ((1u << NG) - 1u);
+      if (m == 0) continue;
+      const int i = NG * p + (NG > 1 && ((m >> sub) & 1u) ? sub : __ffs(m) - 1);
       if constexpr (K_ == 64) lqf::flush_head64<V_, 1>(lds.fl[sub], st, Q0, slot, hv0 + i, 1u, qm);
       else lqf::flush_head4<K_, V_, true>(lds.fl[sub], st, Q0, slot, hv0 + i, qm);
     }
@@ -157,9 +163,11 @@ __device__ __forceinline__ void flush_due(LDS& lds, const lq_state& st, const fl
 // RM: factors held per head.  4 (R <= 4): the G R <= 16 factor rows of the workgroup's heads are one MFMA tile, taken
 // by the last wave.  16 (the rank ablation R <= 16, K = V = 128; kernels.py:63, 457-469): up to G tiles, tile g taken
 // by the second wave of head g.
-template <int K_, int V_, int G, bool CONV, bool FL, int RM, bool DF>
-__device__ __forceinline__ void gdn_step(const lq_state& st, const lq_step_io& io, const lq_conv& cv, int* dlist,
-                                         const float* Q0) {
+// Steps the UW units of a workgroup, and returns the mask of its value heads whose window is now full (bit i: value head
+// hk0 G + i of the row), 0 for a padding row; `slot_` is the row's slot.
+template <int K_, int V_, int G, bool CONV, bool FL, int UW, int RM, bool DF, class LDS>
+__device__ __forceinline__ unsigned gdn_step(LDS& lds, const lq_state& st, const lq_step_io& io, const lq_conv& cv,
+                                             int* dlist, const float* Q0, int& slot_) {
   static_assert(!DF || FL, "deferred flush (lq_gdn_decode_deferred): the fused decode kernel");
   static_assert(!DF || (K_ == 128 && V_ == 128 && G == 2), "deferred flush: 128 x 128 heads, two per key head");
   static_assert(RM == 4 || (RM == 16 && K_ == 128 && V_ == 128 && !FL), "ranks above 4: 128 x 128 heads, no fused flush");
@@ -169,8 +177,7 @@ __device__ __forceinline__ void gdn_step(const lq_state& st, const lq_step_io& i
   constexpr int NE = KD / 64;   // channels per lane in the scalar work
   constexpr int KS32 = KD / 32, KS64 = KD / 64;   // k-steps of the 16x16x32 (bf16 / fp16) and 16x16x64 (int8) MFMAs
   constexpr bool NT = KD == 128;                  // non-temporal bulk loads (see ld_once)
-  constexpr int UW = step_units<G, FL>(), NH = UW * G;      // units, and value heads, of the workgroup
-  __shared__ StepLds<K_, V_, G, FL, RM> lds;
+  constexpr int NH = UW * G;                                // value heads of the workgroup
   const int H = st.H, HV = st.HV, L = st.L, R = st.R;
   const int n = blockIdx.x / (H / UW);
   const int hk0 = (blockIdx.x - n * (H / UW)) * UW;         // the workgroup's first key head
@@ -229,7 +236,7 @@ __device__ __forceinline__ void gdn_step(const lq_state& st, const lq_step_io& i
   // padding row (kernels.py:374-378); a slot outside the cache (or, fused conv, outside the conv state) counts as one
   if (slot <= 0 || slot >= st.NS || (CONV && slot >= cv.NS)) {
     if (rowl) out[lt] = 0;
-    return;
+    return 0u;
   }
   // Every load below is unconditional (clamped addresses) and none sits in a divergent block: a load whose result is
   // merged at the end of an exec-masked block makes the compiler wait for ALL loads in flight, the tile included.
@@ -619,36 +626,73 @@ __device__ __forceinline__ void gdn_step(const lq_state& st, const lq_step_io& i
     }
   }
   }  // live
-  if constexpr (FL) {
-    // the flush of this workgroup's heads whose window is now full (hcnt was L - 1 before the step, or already L):
-    // the fills are uniform loads, so every wave takes the same branch and reaches the same barriers
-    unsigned due = 0;
+  // the heads whose window is now full: hcnt was L - 1 before the step, or already L
+  unsigned due = 0;
 #pragma unroll
-    for (int i = 0; i < NH; ++i) due |= (hw[i] >= L - 1 ? 1u : 0u) << i;
-    if (due) {
-      __syncthreads();          // the step is done with the shared bytes, and its appends are visible to the workgroup
-      const float qm = code_range(st);
-      if constexpr (DF) {       // the first due head now, the other at the start of the next call
-        lqf::flush_head4<128, 128, true>(lds.fl[0], st, Q0, slot, hk * G + (due & 1u ? 0 : 1), qm);
-        if (due == 3u && tid == 0) note_due(st.ctl, dlist, n * HV + hk * G + 1);   // a standalone flush finds it
-      } else {
-        flush_due<K_, V_, G, NH>(lds, st, Q0, slot, hk0 * G, due, qm);
-      }
-    }
-  }
+  for (int i = 0; i < NH; ++i) due |= (hw[i] >= L - 1 ? 1u : 0u) << i;
+  slot_ = slot;
+  return due;
 }
 
 template <int K_, int V_, int G, bool CONV, bool FL, int RM = 4, bool DF = false>
 __global__ __launch_bounds__(64 * step_wph<V_>() * G) __attribute__((amdgpu_waves_per_eu(4)))
 void gdn_step_kernel(lq_state st, lq_step_io io, lq_conv cv, int* dlist, const float* Q0) {
-  gdn_step<K_, V_, G, CONV, FL, RM, DF>(st, io, cv, dlist, Q0);
+  __shared__ StepLds<K_, V_, G, FL, RM> lds;
+  int slot;
+  const unsigned due = gdn_step<K_, V_, G, CONV, FL, 1, RM, DF>(lds, st, io, cv, dlist, Q0, slot);
+  // the fills are uniform loads, so every wave takes the same branches and reaches the same barriers
+  if constexpr (FL) {
+    if (due) {
+      __syncthreads();          // the step is done with the shared bytes, and its appends are visible to the workgroup
+      const float qm = code_range(st);
+      const int n = blockIdx.x / st.H, hv0 = (blockIdx.x - n * st.H) * G;
+      if constexpr (DF) {       // the first due head now, the other at the start of the next call
+        lqf::flush_head4<128, 128, true>(lds.fl[0], st, Q0, slot, hv0 + (due & 1u ? 0 : 1), qm);
+        if (due == 3u && threadIdx.x == 0) note_due(st.ctl, dlist, n * st.HV + hv0 + 1);   // a standalone flush finds it
+      } else {
+        flush_due<K_, V_, G, G, G == 4 ? 2 : 1>(lds, st, Q0, slot, hv0, due, qm);
+      }
+    }
+  }
 }
 // the one-launch decode at GQA 1: W = 2 value heads, of two key heads, per workgroup
 template <int K_, int V_, int W, bool CONV>
 __global__ __launch_bounds__(64 * step_wph<V_>() * W) __attribute__((amdgpu_waves_per_eu(4)))
 void gdn_step_kernel(lq_state st, lq_step_io io, lq_conv cv, const float* Q0) {
   static_assert(W == step_units<1, true>(), "value heads of a workgroup");
-  gdn_step<K_, V_, 1, CONV, true, 4, false>(st, io, cv, nullptr, Q0);
+  __shared__ StepLds<K_, V_, 1, true, 4> lds;
+  int slot;
+  const unsigned due = gdn_step<K_, V_, 1, CONV, true, W, 4, false>(lds, st, io, cv, nullptr, Q0, slot);
+  if (due) {
+    __syncthreads();
+    const int n = blockIdx.x / (st.H / W), hv0 = (blockIdx.x - n * (st.H / W)) * W;
+    flush_due<K_, V_, 1, W, 1>(lds, st, Q0, slot, hv0, due, code_range(st));
+  }
+}
+// the one-launch decode with helper waves: one key head per workgroup, G value heads, 256 G = 128 W threads.  The waves
+// past the step's pass its barriers, and then each group of 256 threads flushes a head.
+template <int K_, int V_, int W, bool CONV, int G>
+__global__ __launch_bounds__(128 * W) __attribute__((amdgpu_waves_per_eu(4)))
+void gdn_step_kernel(lq_state st, lq_step_io io, lq_conv cv, const float* Q0) {
+  static_assert(W == 2 * G && step_wph<V_>() == 2, "two step waves and two helpers per value head");
+  __shared__ WideLds<K_, V_, G> lds;
+  const int n = blockIdx.x / st.H, hv0 = (blockIdx.x - n * st.H) * G;
+  int slot;
+  unsigned due = 0;
+  if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) < 2 * G) {
+    due = gdn_step<K_, V_, G, CONV, true, 1, 4, false>(lds, st, io, cv, nullptr, Q0, slot);
+  } else {
+    slot = io.idx[n];
+    if (slot <= 0 || slot >= st.NS || (CONV && slot >= cv.NS)) return;   // a padding row: the step's waves return too
+#pragma unroll
+    for (int i = 0; i < G; ++i) due |= (st.hcnt[(long long)slot * st.HV + hv0 + i] >= st.L - 1 ? 1u : 0u) << i;
+    __syncthreads();            // the step's two barriers
+    __syncthreads();
+  }
+  if (due) {
+    __syncthreads();
+    flush_due<K_, V_, G, G, G>(lds, st, Q0, slot, hv0, due, code_range(st));
+  }
 }
 
 // ------------------------------------------------------------------------------------------------------------------
@@ -729,21 +773,47 @@ __device__ __forceinline__ void kda_scan_rows(KdaShared& sh, const uint32_t (&kr
 struct KdaChunk {
   int cb, jb, cnt;          // chunk start; this wave's first entry and entry count
 };
+template <bool FL>
 __device__ __forceinline__ KdaChunk kda_chunk(int h, int k, int wi) {
-  const int ce = h - KCH * k, cb = max(ce - KCH, 0), c = ce - cb;
+  const int ce = FL ? max(h - KCH * k, 0) : h - KCH * k, cb = max(ce - KCH, 0), c = ce - cb;
   const int c0 = min(c, 4 * ((c + 7) >> 3));
   return KdaChunk{cb, wi ? cb + c0 : cb, wi ? c - c0 : c0};
 }
 
-__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(4)))
-void kda_step_kernel(lq_state st, lq_step_io io, float glb, int* dlist) {
-  __shared__ KdaShared sh;
+// Steps the UW value heads of a workgroup, each a unit of two waves.  FL (the one-launch decode): the waves then flush the
+// heads the workgroup has filled (or found full), in the bytes that held the step's data.  UW = 2: the units hv, hv + 1 of
+// a row, coupled by the barriers alone.  Returns the mask of the heads whose window is now full, 0 for a padding row;
+// `slot_` is the row's slot.
+template <int UW>
+struct KdaLds {
+  union {
+    KdaShared st[UW];
+    lqf::FlushShared4 fl;
+  };
+};
+static_assert(sizeof(KdaLds<2>) <= 40960, "four workgroups per CU");
+
+// chunks that the heads of a workgroup take (their fills hw), which is how many of the step's barriers its waves pass
+template <int UW>
+__device__ __forceinline__ int kda_chunks(const int (&hw)[UW], int L) {
+  int nck = 0;
+#pragma unroll
+  for (int i = 0; i < UW; ++i) nck = max(nck, hw[i] < L ? (hw[i] + KCH - 1) / KCH : 0);
+  return nck;
+}
+
+template <int UW, bool FL>
+__device__ __forceinline__ void kda_step(KdaShared* units, const lq_state& st, const lq_step_io& io, float glb,
+                                             int* dlist, int& slot_, unsigned& due_) {
   const int H = st.H, HV = st.HV, L = st.L, R = st.R;
   const int G = HV / H;
-  const int n = blockIdx.x / HV;
-  const int hv = blockIdx.x - n * HV;
+  const int n = blockIdx.x / (HV / UW);
+  const int un = UW == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 7);   // this wave's unit
+  const int hv0 = (blockIdx.x - n * (HV / UW)) * UW, hv = hv0 + un;
   const int hk = hv / G;
-  const int lt = threadIdx.x;
+  __shared__ KdaShared own[UW];  // the lone step's (taken by reference from the kernel, it cost 24 bytes per lane of spills)
+  KdaShared& sh = FL ? units[un] : own[un];
+  const int lt = UW == 1 ? threadIdx.x : threadIdx.x & 127;
   const int wi = __builtin_amdgcn_readfirstlane(lt >> 6);
   const int lane = lt & 63;
   const int n16 = lane & 15, q4 = lane >> 4;
@@ -759,7 +829,10 @@ void kda_step_kernel(lq_state st, lq_step_io io, float glb, int* dlist) {
   const bf16_t* mrow = (const bf16_t*)io.mixed + (long long)n * MIX;
   // Window fill: a uniform load, served by the scalar data cache (a vector load here would queue behind the bulk loads
   // the CU's other workgroups have issued, and every later load of this workgroup would wait for it).
-  const int hfill = st.hcnt[sh_];
+  int hw[UW];                   // of the workgroup's heads
+#pragma unroll
+  for (int i = 0; i < UW; ++i) hw[i] = st.hcnt[(long long)slot * HV + hv0 + i];
+  const int hfill = UW == 1 || un == 0 ? hw[0] : hw[UW - 1];
   __builtin_amdgcn_sched_barrier(0);
   // per-channel operands: wave 0 (scalar work) channels c = lane, lane + 64; wave 1 (its own gate) c = 2 lane + e
   bf16_t kxr[2], qxr[2], axr[2];
@@ -781,18 +854,20 @@ void kda_step_kernel(lq_state st, lq_step_io io, float glb, int* dlist) {
   const float vin = bf2f(mrow[2ll * H * KD + hv * VD + lt]);
   const float sv = Svp[lt];
   __builtin_amdgcn_sched_barrier(0);
-  const int h = hfill;
-  if (h >= L) {                 // a full window is never stepped: zero output, and the head is flagged again so that
-    if (lt == 0) note_due(st.ctl, dlist, n * HV + hv);   // the flush after this step takes it
+  const bool live = hfill < L;  // a full window is never stepped
+  if (!FL && !live) {           // zero output, and the head is flagged again so that the flush after this step takes it
+    if (lt == 0) note_due(st.ctl, dlist, n * HV + hv);
     out[lt] = 0;
     return;
   }
+  const int h = !FL || live ? hfill : 0;   // FL: a full head passes the barriers and writes a zero output only
   // the four factor rows (2 KiB, inside the checkpoint block whatever R) to LDS, one KiB per wave
   lds_load16((const char*)UQp + 1024 * wi + 16 * lane, (char*)&sh.uq[2 * wi][0]);
   // The window's live entries j < h, chunk by chunk (kda_chunk).  Each wave's decays go straight to its own LDS rows
   // (1 KiB = 4 rows per wave instruction, rows past the buffer's last re-reading it); its values u_j and keys K_j go
   // to registers, a channel pair (2 lane, 2 lane + 1) per lane and row.  The first chunk, then the int8 tile.
-  const int nck = (h + KCH - 1) / KCH;
+  // FL: the units pass the same barriers (one without a chunk k takes no entries of it)
+  const int nck = FL ? kda_chunks<UW>(hw, L) : (h + KCH - 1) / KCH;
   uint32_t ur[16], kr[16];
   const char* gg = (const char*)((const f16_t*)st.Gbuf + sh_ * L * KD);
   const uint32_t* ug = (const uint32_t*)((const bf16_t*)st.Ubuf + sh_ * L * VD) + lane;
@@ -815,7 +890,7 @@ void kda_step_kernel(lq_state st, lq_step_io io, float glb, int* dlist) {
         for (int i = 0; i < 4; ++i) kr[4 * g4 + i] = ld_once(kg + (c.jb + min(4 * g4 + i, c.cnt - 1)) * (KD / 2));
       }
   };
-  KdaChunk ck = kda_chunk(h, 0, wi);                  // h = 0: no entries
+  KdaChunk ck = kda_chunk<FL>(h, 0, wi);                  // h = 0: no entries
   load_chunk(ck);
   __builtin_amdgcn_sched_barrier(0);
   i32x4 afr[4][2];
@@ -981,7 +1056,7 @@ void kda_step_kernel(lq_state st, lq_step_io io, float glb, int* dlist) {
   //      continues the product wave 0 reached, wave 0 the one wave 1 reaches ----
   for (int k = 1; k < nck; ++k) {
     __syncthreads();            // the previous chunk's decayed keys and cwq are read; wave 0's product is in dhand
-    ck = kda_chunk(h, k, wi);
+    ck = kda_chunk<FL>(h, k, wi);
     load_chunk(ck);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this chunk's decay rows in LDS (keys and values with them)
     if (wi == 1) {
@@ -1038,13 +1113,16 @@ void kda_step_kernel(lq_state st, lq_step_io io, float glb, int* dlist) {
   const float yq = (mqr.y * (sh.sc[3] * (1.0f / DIGIT_SCALE))) * sv;
   const float u = beta * (vin - (mq + a6 + a4));        // kernels.py:1065
   const float y = yq + a7 + a5 + kappa * u;             // kernels.py:1066
+  if (!live) {
+    out[lt] = 0;
+  } else {
   out[lt] = f2bf(y);
   ((bf16_t*)st.Ubuf)[(sh_ * L + h) * VD + lt] = f2bf(u);
   if (hv % G == 0) ((bf16_t*)st.Kbuf)[(((long long)slot * H + hk) * L + h) * KD + lt] = sh.bkq[0][lt];   // bf16(kn)
   if (lt == 0) {
     st.Wbuf[sh_ * L + h] = 1.0f;
     st.hcnt[sh_] = h + 1;
-    if (h + 1 == L) note_due(st.ctl, dlist, n * HV + hv);   // this head is due: the flush that follows takes it
+    if (!FL && h + 1 == L) note_due(st.ctl, dlist, n * HV + hv);   // due: the flush that follows takes it
   }
   if (wi == 0) {                // gate state (kernels.py:895-896)
 #pragma unroll
@@ -1053,6 +1131,51 @@ void kda_step_kernel(lq_state st, lq_step_io io, float glb, int* dlist) {
       st.Pbuf[sh_ * KD + c] = gnv[e];
       ((f16_t*)st.Gbuf)[(sh_ * L + h) * KD + c] = f2h(env[e]);
     }
+  }
+  }  // live
+  if constexpr (FL) {
+#pragma unroll
+    for (int i = 0; i < UW; ++i) due_ |= (hw[i] >= L - 1 ? 1u : 0u) << i;
+    slot_ = slot;
+  }
+}
+
+__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(4)))
+void kda_step_kernel(lq_state st, lq_step_io io, float glb, int* dlist) {
+  int slot;
+  unsigned due;
+  kda_step<1, false>(nullptr, st, io, glb, dlist, slot, due);
+}
+// the four-wave flush of KDA heads behind their own step: W = 2 heads per workgroup, or (W = 1) one head with two waves
+// that pass the step's barriers and only flush
+template <int W>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+void flush4_kernel(lq_state st, lq_step_io io, float glb, const float* Q0) {
+  __shared__ KdaLds<W> lds;
+  const int n = blockIdx.x / (st.HV / W), hv0 = (blockIdx.x - n * (st.HV / W)) * W;
+  int slot;
+  unsigned due = 0;
+  if (W == 2 || __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) < 2) {
+    kda_step<W, true>(lds.st, st, io, glb, nullptr, slot, due);
+  } else {
+    slot = io.idx[n];
+    if (slot <= 0 || slot >= st.NS) return;           // a padding row: the step's waves return too
+    const int hw[1] = {st.hcnt[(long long)slot * st.HV + hv0]};
+    due = hw[0] >= st.L - 1 ? 1u : 0u;
+    __syncthreads();            // the step's barriers
+    for (int k = 1; k < kda_chunks<1>(hw, st.L); ++k) {
+      __syncthreads();
+      __syncthreads();
+    }
+    __syncthreads();
+  }
+  // the fills are uniform: every wave takes the same branches
+  if (due) {
+    __syncthreads();            // the step is done with the shared bytes, and its appends are visible to the workgroup
+    const float qm = code_range(st);
+#pragma unroll 1
+    for (int i = 0; i < W; ++i)
+      if ((due >> i) & 1u) lqf::flush_head4<KD, VD, true, true>(lds.fl, st, Q0, slot, hv0 + i, qm);
   }
 }
 
@@ -1096,15 +1219,47 @@ static int launch_gdn_dims(const lq_state* st, const lq_step_io* io, const lq_co
   return st->V == 128 ? launch_gdn<64, 128, CONV>(st, io, cv, dlist, s) : launch_gdn<64, 64, CONV>(st, io, cv, dlist, s);
 }
 
+// Small launches, up to four heads per CU, take the kernels with helper waves: their workgroups flush their heads side by
+// side, and all stay resident.  A flush call of one row (us, in turn -> side by side): two GQA 1 heads 21.6 -> 14.6, two of
+// a key head 21.6 -> 16.8, four 29.2 -> 25.4, two KDA heads 24.6 -> 15.2.  Window 16, us per call without -> with: GQA 1,
+// 16 heads, B = 16 7.5 -> 6.5, B = 64 (4 heads per CU) 9.7 -> 9.6; GQA 2, B = 16 (2) 7.4 -> 7.3, B = 64 (8) 15.3 -> 17.4;
+// GQA 4, B = 16 (4) 9.4 -> 9.2, B = 32 (8) 15.7 -> 17.7; KDA, 32 heads, B = 1 8.2 -> 6.9, B = 32 (4) 13.0 -> 11.9,
+// B = 48 (6) 16.7 -> 18.6.
+static bool helper_waves(const lq_state* st, int N) { return (long long)N * st->HV <= 4ll * lq_num_cus(); }
+
 // the decode call in one launch: each workgroup flushes the heads whose window it fills
+template <int K_, int V_, bool CONV, int G>
+static void launch_wide(const lq_state* st, const lq_step_io* io, const lq_conv& cv, const float* Q0, hipStream_t s) {
+  gdn_step_kernel<K_, V_, 2 * G, CONV, G><<<dim3((unsigned)(io->N * st->H)), 256 * G, 0, s>>>(*st, *io, cv, Q0);
+}
 template <int K_, int V_, bool CONV>
 static int launch_decode(const lq_state* st, const lq_step_io* io, const lq_conv& cv, const float* Q0, hipStream_t s) {
   const int G = st->HV / st->H;
   const dim3 grid((unsigned)(io->N * (G == 1 ? st->H / 2 : st->H)));
+  const bool wide = helper_waves(st, io->N);
   switch (G) {
-    case 1: gdn_step_kernel<K_, V_, 2, CONV><<<grid, 128 * step_wph<V_>(), 0, s>>>(*st, *io, cv, Q0); break;
-    case 2: gdn_step_kernel<K_, V_, 2, CONV, true><<<grid, 128 * step_wph<V_>(), 0, s>>>(*st, *io, cv, nullptr, Q0); break;
-    case 4: gdn_step_kernel<K_, V_, 4, CONV, true><<<grid, 256 * step_wph<V_>(), 0, s>>>(*st, *io, cv, nullptr, Q0); break;
+    case 1:
+      if (wide) launch_wide<K_, V_, CONV, 1>(st, io, cv, Q0, s);
+      else gdn_step_kernel<K_, V_, 2, CONV><<<grid, 128 * step_wph<V_>(), 0, s>>>(*st, *io, cv, Q0);
+      break;
+    case 2:
+      if constexpr (V_ == 128) {
+        if (wide) {
+          launch_wide<K_, V_, CONV, 2>(st, io, cv, Q0, s);
+          break;
+        }
+      }
+      gdn_step_kernel<K_, V_, 2, CONV, true><<<grid, 128 * step_wph<V_>(), 0, s>>>(*st, *io, cv, nullptr, Q0);
+      break;
+    case 4:
+      if constexpr (V_ == 128) {
+        if (wide) {
+          launch_wide<K_, V_, CONV, 4>(st, io, cv, Q0, s);
+          break;
+        }
+      }
+      gdn_step_kernel<K_, V_, 4, CONV, true><<<grid, 256 * step_wph<V_>(), 0, s>>>(*st, *io, cv, nullptr, Q0);
+      break;
     default: return LQ_ERR_ARG;
   }
   return hipGetLastError() == hipSuccess ? LQ_OK : LQ_ERR_HIP;
@@ -1212,6 +1367,19 @@ extern "C" int lq_kda_decode(const lq_state* st, const lq_step_io* io, float glb
   if ((rc = lq_check_flush(st, Q0, io->idx, io->N, 1, qmax))) return rc;
   if (io->N == 0) return LQ_OK;
   hipStream_t s = (hipStream_t)stream;
+  const long long heads = (long long)io->N * st->HV;
+  if (helper_waves(st, io->N)) {
+    flush4_kernel<1><<<dim3((unsigned)heads), 256, 0, s>>>(*st, *io, glb, Q0);
+    return hipGetLastError() == hipSuccess ? LQ_OK : LQ_ERR_HIP;
+  }
+  // One launch, two heads per workgroup, up to one round of workgroups (eight heads per CU), and for windows of one chunk
+  // below two: us per call, two launches -> one, 32 heads, W = 16: B = 48 18.6 -> 16.7, B = 64 21.7 -> 20.0, B = 96 27.9
+  // -> 27.3, B = 120 32.7 -> 31.7; W = 64, whose units also meet at each chunk's barriers: B = 48 21.9 -> 21.4, B = 64
+  // 25.6 -> 25.7, B = 96 33.9 -> 35.1.  An odd HV takes two.
+  if (st->HV % 2 == 0 && (heads <= 8ll * lq_num_cus() || (st->L <= KCH && heads < 16ll * lq_num_cus()))) {
+    flush4_kernel<2><<<dim3((unsigned)(heads / 2)), 256, 0, s>>>(*st, *io, glb, Q0);
+    return hipGetLastError() == hipSuccess ? LQ_OK : LQ_ERR_HIP;
+  }
   if ((rc = lq_launch_step(st, io, 1, glb, nullptr, s))) return rc;
   return lq_launch_flush(st, Q0, io->idx, io->N, 1, qmax, nullptr, s);
 }

@@ -164,7 +164,7 @@ class LeapQuantState:
         io = KN._step_io(mixed, a, b, A_log, dt_bias, idx, out, self.kstep_scale)
         stream = ctypes.c_void_p(torch.cuda.current_stream(mixed.device).cuda_stream)
         L = self._lib
-        if self.kda:                 # the step, then the flush of the heads it fills
+        if self.kda:                 # step + flush of the heads it fills (one launch for small batches)
             _lib.check(L.lq_kda_decode(ctypes.byref(st), ctypes.byref(io), ctypes.c_float(self.glb), KN._p(self.Q0),
                                        stream), "lq_kda_decode")
         else:                        # step + flush of the heads it fills (one launch at ranks up to 4)

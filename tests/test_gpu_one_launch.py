@@ -1,8 +1,8 @@
-"""GPU: the one-launch GDN decode (lq_gdn_decode: the step's workgroups flush the heads whose window they fill) against
-the step followed by the standalone flush on a copy of the state, byte for byte: every head-dim pair and GQA factor,
-window lengths on both sides of a staged half (32 entries), rows whose heads are due together and rows where they stand
-at different fills (one head of a pair due, a head found full, none due), padding rows."""
-import numpy as np
+"""GPU: the one-launch decodes (lq_gdn_decode, lq_kda_decode: the step's workgroups flush the heads whose window they
+fill) against the step followed by the standalone flush on a copy of the state, byte for byte: every head-dim pair and
+GQA factor, window lengths on both sides of a staged half (32 entries), rows whose heads are due together and rows where
+they stand at different fills (one head of a pair due, a head found full, none due), padding rows; launches of up to four
+heads per CU, whose workgroups have helper waves, and larger ones."""
 import pytest
 import torch
 
@@ -11,9 +11,9 @@ from tests import lqgpu as G
 pytestmark = pytest.mark.gpu
 
 
-def _state(g, NS, HV, H, K, V, L, R, qmax):
+def _state(g, NS, HV, H, K, V, L, R, qmax, kda=False, glb=0.0):
     ssm = torch.zeros(NS, HV, V, K, device=G.DEV).normal_(0.0, 0.02, generator=g)
-    lq = G.LeapQuantState(ssm, H, L=L, R=R, qmax=qmax)
+    lq = G.LeapQuantState(ssm, H, kda=kda, gate_lower_bound=glb, L=L, R=R, qmax=qmax)
     lq.quantize(ssm, torch.arange(1, NS, device=G.DEV))
     # fills: slot 1 all heads L - 1, slot 2 all full but one, slot 3 none due, the others any mix per head
     fill = torch.randint(max(0, L - 3), L + 1, (NS, HV), generator=g, device=G.DEV, dtype=torch.int32)
@@ -24,42 +24,66 @@ def _state(g, NS, HV, H, K, V, L, R, qmax):
     lq.hcnt.copy_(fill)
     j = torch.arange(L, device=G.DEV)
     lq.Wbuf.copy_(torch.rand(NS, HV, L, device=G.DEV, generator=g) * (j < fill[..., None]))
-    lq.Pbuf.copy_(torch.rand(lq.Pbuf.shape, device=G.DEV, generator=g))
+    lq.Pbuf.copy_(torch.rand(lq.Pbuf.shape, device=G.DEV, generator=g) * (-1.0 if kda else 1.0))
+    if kda:                                             # decays below 1, 1 past the fill
+        e = 0.8 + 0.2 * torch.rand(lq.Gbuf.shape, device=G.DEV, generator=g)
+        lq.Gbuf.copy_(torch.where((j < fill[..., None])[..., None], e, torch.ones_like(e)))
     lq.Kbuf.copy_(torch.randn(lq.Kbuf.shape, device=G.DEV, generator=g) * 0.09)
     lq.Ubuf.copy_(torch.randn(lq.Ubuf.shape, device=G.DEV, generator=g) * 0.5)
     return ssm, lq
 
 
-@pytest.mark.parametrize("K,V", [(128, 128), (64, 128), (64, 64)])
-@pytest.mark.parametrize("GQA", [1, 2, 4])
-@pytest.mark.parametrize("L,R,qmax", [(16, 4, 127.0), (33, 3, 31.0), (64, 4, 127.0), (1, 1, 127.0)])
-def test_one_launch_equals_step_then_flush(K, V, GQA, L, R, qmax):
-    g = torch.Generator(device=G.DEV)
-    g.manual_seed(K + V + GQA + L)
-    NS, H = 9, 4
-    HV = H * GQA
-    ssm, lq = _state(g, NS, HV, H, K, V, L, R, qmax)
+def _check(g, lq, ssm, H, N, rest):
+    """Two decode calls (the second steps the windows that the first has reset) of N rows, padding rows among them,
+    against step + flush on a copy of the state."""
+    NS, HV, K, V, L = lq.NS, lq.HV, lq.K, lq.V, lq.L
     ssm2 = ssm.clone()
-    lq2 = G.LeapQuantState(ssm2, H, L=L, R=R, qmax=qmax)
-    for k in ("hcnt", "Wbuf", "Pbuf", "Kbuf", "Ubuf"):
+    lq2 = G.LeapQuantState(ssm2, H, L=L, **rest)
+    bufs = ("hcnt", "Wbuf", "Pbuf", "Kbuf", "Ubuf") + (("Gbuf",) if lq.kda else ())
+    for k in bufs:
         getattr(lq2, k).copy_(getattr(lq, k))
-    lq2.ctl[0] = 1                                      # heads found full are due too (the scan's flag is theirs)
-    idx = torch.tensor([3, 1, 0, 8, 2, -1, 5, 4, 7, NS + 3], device=G.DEV, dtype=torch.int32)
-    N = len(idx)
+    idx = (torch.randperm(NS - 1, device=G.DEV, generator=g)[:N] + 1).int()
+    idx[:5] = torch.tensor([3, 0, 1, -1, NS + 3], device=G.DEV)
+    idx[5:] = idx[5:][torch.randperm(N - 5, device=G.DEV, generator=g)]
+    idx[5:] = torch.where((idx[5:] == 3) | (idx[5:] == 1), torch.zeros_like(idx[5:]), idx[5:])
     bf = lambda *s: torch.randn(*s, device=G.DEV, generator=g).bfloat16()
-    for _ in range(2):                                  # the second call steps the windows the first has reset
-        mixed, a, b = bf(N, 2 * H * K + HV * V), bf(N, HV), bf(N, HV)
-        A_log, dt_bias = torch.zeros(HV, device=G.DEV), torch.zeros(HV, device=G.DEV)
+    KA = K if lq.kda else 1
+    A_log, dt_bias = torch.zeros(HV, device=G.DEV), torch.zeros(HV * KA, device=G.DEV)
+    for _ in range(2):
+        mixed, a, b = bf(N, 2 * H * K + HV * V), bf(N, HV, KA), bf(N, HV)
         o1 = torch.empty(N, HV, V, device=G.DEV, dtype=torch.bfloat16)
         o2 = torch.empty_like(o1)
         lq.decode(ssm, mixed, a, b, A_log, dt_bias, idx, o1)
         v = lq2.views(ssm2)
-        lq2.kstep(v["q32"], v["Sk"], v["Sv"], v["skv"], lq2.Kbuf, lq2.Ubuf, lq2.Wbuf, lq2.Pbuf, lq2.hcnt, mixed, a, b,
-                  A_log, dt_bias, v["uq"], idx, o2)
+        lq2.kstep(v["q32"], v["Sk"], v["Sv"], v["skv"], lq2.Kbuf, lq2.Ubuf, lq2.Wbuf, lq2.Pbuf,
+                  *((lq2.Gbuf,) if lq.kda else ()), lq2.hcnt, mixed, a, b, A_log, dt_bias, v["uq"], idx, o2)
         lq2.flush(ssm2, idx)
         torch.cuda.synchronize()
         assert torch.equal(o1, o2)
         assert torch.equal(ssm.view(torch.int32), ssm2.view(torch.int32))
-        for k in ("hcnt", "Wbuf", "Pbuf", "Kbuf", "Ubuf"):
+        for k in bufs:
             assert torch.equal(getattr(lq, k), getattr(lq2, k)), k
         assert int((lq.hcnt[idx[(idx > 0) & (idx < NS)].long()] >= L).sum()) == 0
+
+
+@pytest.mark.parametrize("K,V", [(128, 128), (64, 128), (64, 64)])
+@pytest.mark.parametrize("GQA", [1, 2, 4])
+@pytest.mark.parametrize("L,R,qmax", [(16, 4, 127.0), (33, 3, 31.0), (64, 4, 127.0), (1, 1, 127.0)])
+@pytest.mark.parametrize("heads", [100, 1100])
+def test_gdn_one_launch_equals_step_then_flush(K, V, GQA, L, R, qmax, heads):
+    g = torch.Generator(device=G.DEV)
+    g.manual_seed(K + V + GQA + L + heads)
+    H = 3 if (GQA, heads) == (1, 100) else 4            # an odd number of key heads at GQA 1
+    N = max(9, heads // (H * GQA) + 1)
+    ssm, lq = _state(g, N + 4, H * GQA, H, K, V, L, R, qmax)
+    _check(g, lq, ssm, H, N, dict(R=R, qmax=qmax))
+
+
+@pytest.mark.parametrize("L,R,glb", [(16, 4, 0.0), (33, 2, -5.0), (64, 4, 0.0), (1, 1, 0.0)])
+@pytest.mark.parametrize("HV,H,heads", [(3, 3, 100), (8, 4, 1100), (5, 5, 1100), (16, 16, 4200)])
+def test_kda_one_launch_equals_step_then_flush(HV, H, heads, L, R, glb):
+    g = torch.Generator(device=G.DEV)
+    g.manual_seed(HV + L + heads)
+    N = heads // HV + 1
+    ssm, lq = _state(g, N + 4, HV, H, 128, 128, L, R, 127.0, kda=True, glb=glb)
+    _check(g, lq, ssm, H, N, dict(R=R, kda=True, gate_lower_bound=glb))
