@@ -104,6 +104,7 @@ class LeapQuantState:
             self.kdeq = _make_dequant(NS, HV, K, V, L, SS, buf_dtype=KN.BF16, R=R, qmax=qmax)
             self.kquant = _make_quantize(NS, HV, K, V, L, SS, R=R, ITERS=1, qmax=qmax)
         self._lib = _lib.lib()
+        self._scale = self.kstep_scale
         self._vkey = None
         self._skey = None
         self._scan_src = None
@@ -120,6 +121,13 @@ class LeapQuantState:
             self._param_f32[key] = t.detach().float().contiguous()
         return self._param_f32[key]
 
+    def _param(self, t, shape):
+        """A gate parameter as contiguous fp32 values of `shape`.  Only the address goes to the kernels, so a tensor of as
+        many contiguous values is taken as it is (a reshape costs the host ~2 us, three of them 6 of a decode call's 12)."""
+        t = self._as_f32(t)
+        n = shape[0] * shape[1] if len(shape) == 2 else shape[0]
+        return t if t.numel() == n and t.is_contiguous() else t.reshape(shape).contiguous()
+
     def views(self, ssm):
         k = _ident(ssm)
         if self._vkey != k:
@@ -127,8 +135,9 @@ class LeapQuantState:
         return self._v
 
     def _struct(self, ssm):
-        """lq_state of this layer for the cache tensor ssm (cached per tensor identity)."""
-        k = _ident(ssm)
+        """lq_state of this layer for the cache tensor ssm: it holds the tensor's address and this state's own sizes, so
+        it is rebuilt when the address changes."""
+        k = ssm.data_ptr()
         if self._skey != k:
             if ssm.data_ptr() % 16 or self.SS % 4:
                 raise ValueError("the fp32 state cache must be 16-byte aligned with a slot stride divisible by 4")
@@ -142,14 +151,12 @@ class LeapQuantState:
         """One decode token per row, then the end-of-window flush of the heads whose window became full (one C call:
         lq_gdn_decode, or lq_kda_decode).
         a: GDN (N, HV) | KDA (N, HV, K) raw gate;  dt_bias: GDN (HV,) | KDA (HV*K,)."""
-        A_log = self._as_f32(A_log)
-        dt_bias = self._as_f32(dt_bias)
         KA = self.K if self.kda else 1
         N = idx.shape[0]
         self._check_gate(a, N, KA)
-        a = a.reshape(N, self.HV, KA).contiguous()
-        dt_bias = dt_bias.reshape(self.HV, KA).contiguous()
-        A_log = A_log.reshape(self.HV).contiguous()
+        a = a.contiguous()
+        dt_bias = self._param(dt_bias, (self.HV, KA))
+        A_log = self._param(A_log, (self.HV,))
         idx = idx if idx.dtype == torch.int32 else idx.to(torch.int32)
         idx = idx.contiguous()
         if (mixed.dtype != torch.bfloat16 or not mixed.is_contiguous()
@@ -161,15 +168,16 @@ class LeapQuantState:
             raise ValueError("b: bf16 [N, HV] expected")
         b = b.contiguous()
         st = self._struct(ssm)
-        io = KN._step_io(mixed, a, b, A_log, dt_bias, idx, out, self.kstep_scale)
-        stream = ctypes.c_void_p(torch.cuda.current_stream(mixed.device).cuda_stream)
+        dev = KN._dev
+        io = _lib.LqStepIO(dev(mixed), dev(a), dev(b), dev(A_log), dev(dt_bias), dev(idx), dev(out), N, self._scale)
+        stream = KN._raw_stream(mixed)
         L = self._lib
         if self.kda:                 # step + flush of the heads it fills (one launch for small batches)
-            _lib.check(L.lq_kda_decode(ctypes.byref(st), ctypes.byref(io), ctypes.c_float(self.glb), KN._p(self.Q0),
-                                       stream), "lq_kda_decode")
+            _lib.check(L.lq_kda_decode(ctypes.byref(st), ctypes.byref(io), self.glb, dev(self.Q0), stream),
+                       "lq_kda_decode")
         else:                        # step + flush of the heads it fills (one launch at ranks up to 4)
             fn = L.lq_gdn_decode_deferred if self.defer_flush else L.lq_gdn_decode
-            _lib.check(fn(ctypes.byref(st), ctypes.byref(io), None, KN._p(self.Q0), stream), "lq_gdn_decode")
+            _lib.check(fn(ctypes.byref(st), ctypes.byref(io), None, dev(self.Q0), stream), "lq_gdn_decode")
 
     def decode_conv(self, ssm, x, conv_state, conv_weight, conv_bias, silu, a, b, A_log, dt_bias, idx, out):
         """GDN decode with the conv1d update fused into the step (lq_gdn_step_conv): x is the raw projection
@@ -187,13 +195,11 @@ class LeapQuantState:
         if conv_bias is not None and (conv_bias.dtype != torch.bfloat16 or conv_bias.numel() != C
                                       or not conv_bias.is_contiguous()):
             raise ValueError("conv_bias: bf16 [C] expected")
-        A_log = self._as_f32(A_log)
-        dt_bias = self._as_f32(dt_bias)
         N = idx.shape[0]
         self._check_gate(a, N, 1)
-        a = a.reshape(N, self.HV).contiguous()
-        dt_bias = dt_bias.reshape(self.HV).contiguous()
-        A_log = A_log.reshape(self.HV).contiguous()
+        a = a.contiguous()
+        dt_bias = self._param(dt_bias, (self.HV,))
+        A_log = self._param(A_log, (self.HV,))
         idx = idx if idx.dtype == torch.int32 else idx.to(torch.int32)
         idx = idx.contiguous()
         if x.dtype != torch.bfloat16 or not x.is_contiguous() or x.shape != (N, C):
@@ -204,11 +210,12 @@ class LeapQuantState:
             raise ValueError("b: bf16 [N, HV] expected")
         b = b.contiguous()
         st = self._struct(ssm)
-        io = KN._step_io(x, a, b, A_log, dt_bias, idx, out, self.kstep_scale)
+        dev = KN._dev
+        io = _lib.LqStepIO(dev(x), dev(a), dev(b), dev(A_log), dev(dt_bias), dev(idx), dev(out), N, self._scale)
         cv = KN.conv_struct(conv_state, w, conv_bias, silu)
-        stream = ctypes.c_void_p(torch.cuda.current_stream(x.device).cuda_stream)
+        stream = KN._raw_stream(x)
         fn = self._lib.lq_gdn_decode_deferred if self.defer_flush else self._lib.lq_gdn_decode
-        _lib.check(fn(ctypes.byref(st), ctypes.byref(io), ctypes.byref(cv), KN._p(self.Q0), stream), "lq_gdn_decode")
+        _lib.check(fn(ctypes.byref(st), ctypes.byref(io), ctypes.byref(cv), dev(self.Q0), stream), "lq_gdn_decode")
 
     def _check_gate(self, a, N, KA):
         """The raw gate `a` is read as bf16, N x HV (GDN) or N x HV x K (KDA) values (kernels.py:86, 738)."""
@@ -234,46 +241,46 @@ class LeapQuantState:
         idx = idx if idx.dtype == torch.int32 else idx.to(torch.int32)
         idx = idx.contiguous()
         st = self._struct_scan(ssm)
-        stream = ctypes.c_void_p(torch.cuda.current_stream(idx.device).cuda_stream)
         _lib.check(self._lib.lq_flush(ctypes.byref(st), KN._p(self.Q0), KN._p(idx), idx.shape[0], 1 if self.kda else 0,
-                                      ctypes.c_float(self.qmax), stream), "lq_flush")
+                                      ctypes.c_float(self.qmax), KN._stream(idx)), "lq_flush")
 
     @property
     def kstep_scale(self):
         return 128 ** -0.5 if self.kda else self.K ** -0.5
 
-    def _kda_round_trip(self, ssm, idx, fn, *extra):
+    def _check_round_trip(self, ssm, idx):
+        KN._check_view(ssm, self.NS, self.HV, self.V, self.K, self.SS)
+        if idx.dim() != 1:
+            raise ValueError("idx: 1-D expected, got shape %s" % (tuple(idx.shape),))
+
+    def _round_trip(self, ssm, idx, fn, *extra):
         idx = idx if idx.dtype == torch.int32 else idx.to(torch.int32)
         idx = idx.contiguous()
         st = self._struct(ssm)
-        stream = ctypes.c_void_p(torch.cuda.current_stream(idx.device).cuda_stream)
         _lib.check(getattr(self._lib, fn)(ctypes.byref(st), *extra, KN._p(idx), idx.shape[0],
-                                          ctypes.c_float(self.qmax), stream), fn)
+                                          ctypes.c_float(self.qmax), KN._stream(idx)), fn)
 
     def dequantize(self, ssm, idx):
         """Materialise the fp32 state of the slots idx in place (before the engine's own prefill kernel runs)."""
         if idx.numel() == 0:
             return
         if self.kda:                 # S = (Q U^T + deq) diag(exp(P)) + decayed window (state.py:118-128), HIP
-            self._kda_round_trip(ssm, idx, "lq_kda_dequant")
+            self._round_trip(ssm, idx, "lq_kda_dequant")
             return
-        idx = idx.to(torch.int32).contiguous()
+        self._check_round_trip(ssm, idx)
         if self.defer_flush:         # a head left full by a deferred decode is flushed before its state is read
             self.flush(ssm, idx)
-        v = self.views(ssm)
-        self.kdeq(ssm, v["Sq"], v["Sk"], v["Sv"], self.Kbuf, self.Ubuf, self.Wbuf, self.Pbuf, self.Gbuf, self.hcnt,
-                  v["uq"], idx)
+        self._round_trip(ssm, idx, "lq_dequant")
 
     def quantize(self, ssm, idx):
         """Write the 8-bit checkpoint of the fp32 states in the slots idx and reset their windows (after a prefill)."""
         if idx.numel() == 0:
             return
         if self.kda:                 # rank-R fit (3 rounds) + residual codes, window reset (state.py:130-142), HIP
-            self._kda_round_trip(ssm, idx, "lq_kda_checkpoint", KN._p(self.Q0))
+            self._round_trip(ssm, idx, "lq_kda_checkpoint", KN._p(self.Q0))
             return
-        v = self.views(ssm)
-        self.kquant(ssm, v["Sq"], v["Sk"], v["Sv"], v["uq"], self.Wbuf, self.Pbuf, self.hcnt, self.Q0,
-                    idx.to(torch.int32).contiguous())
+        self._check_round_trip(ssm, idx)
+        self._round_trip(ssm, idx, "lq_quantize", KN._p(self.Q0))
 
 
 _STATES = {}        # cache identity -> the LeapQuantState built for it
