@@ -61,7 +61,7 @@ constexpr float KSPLIT = 64.0f;   // kn / qn scaled by 2^6 before the fp16 hi / 
 // workgroups per CU (the hkq rows unpadded there).
 constexpr int DIGP = 16, OPP = 8;
 template <int K_, int V_, int G, int RM>
-struct StepShared {
+struct alignas(16) StepShared {   // so that the 16-byte fragment reads are one instruction, not two 8-byte ones
   static constexpr int HPP = G == 1 && RM == 4 && K_ == 128 ? 0 : OPP;
   bf16_t ub[G][LMAX][V_];  // the window's u_j rows per value head (direct global -> LDS loads)
   int8_t dig[G][6][K_ + DIGP];   // int8 GEMV B operand: k digits 0-2, q digits 0-2
@@ -208,7 +208,7 @@ __device__ __forceinline__ unsigned gdn_step(LDS& lds, const lq_state& st, const
       for (int g2 = 0; g2 < G; ++g2) pend |= (st.hcnt[(long long)slot0 * HV + hk * G + g2] >= L ? 1u : 0u) << g2;
       if (pend) {
         const float qm = code_range(st);
-#pragma unroll
+#pragma unroll 1
         for (int g2 = 0; g2 < G; ++g2)
           if ((pend >> g2) & 1u) lqf::flush_head4<128, 128, true>(lds.fl[0], st, Q0, slot0, hk * G + g2, qm);
       }
@@ -715,7 +715,7 @@ void gdn_step_kernel(lq_state st, lq_step_io io, lq_conv cv, const float* Q0) {
 // ------------------------------------------------------------------------------------------------------------------
 constexpr int KCH = 32;             // window entries per chunk
 
-struct KdaShared {
+struct alignas(16) KdaShared {      // 16-byte fragment reads, as StepShared (config 2: 44.9 -> 42.7 us per call)
   f16_t gk[KCH][KD];        // a chunk's step decays e_j (row j - cb); the scan overwrites them with K~_j (bf16)
   float2 part[2][VD];       // per wave: (A4, A5) sums of row v over the wave's entries of every chunk
   float2 mq[VD];            // GEMV rows (k, q) in digit units
