@@ -109,32 +109,10 @@ __device__ __forceinline__ float xor32_max(float x) {
 __device__ __forceinline__ float sum64(float x) { return xor32_sum(xor16_sum(sum16(x))); }
 __device__ __forceinline__ float max64(float x) { return xor32_max(xor16_max(max16(x))); }
 
-// the same exchanges on fp64 values (both 32-bit halves moved by the same lane pattern)
-template <int CTRL>
-__device__ __forceinline__ double dppd(double x) {
-  const unsigned long long u = __builtin_bit_cast(unsigned long long, x);
-  const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)u, CTRL, 0xf, 0xf, false);
-  const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(u >> 32), CTRL, 0xf, 0xf, false);
-  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
-}
+// an fp64 value of its 32-bit halves
 __device__ __forceinline__ double join_d(unsigned lo, unsigned hi) {
   return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
 }
-__device__ __forceinline__ double sum64d(double x) {
-  x += dppd<DPP_XOR1>(x);
-  x += dppd<DPP_XOR2>(x);
-  x += dppd<DPP_HALF_MIRROR>(x);
-  x += dppd<DPP_MIRROR>(x);
-  unsigned long long u = __builtin_bit_cast(unsigned long long, x);
-  auto l16 = __builtin_amdgcn_permlane16_swap((unsigned)u, (unsigned)u, false, false);
-  auto h16 = __builtin_amdgcn_permlane16_swap((unsigned)(u >> 32), (unsigned)(u >> 32), false, false);
-  x = join_d(l16[0], h16[0]) + join_d(l16[1], h16[1]);
-  u = __builtin_bit_cast(unsigned long long, x);
-  auto l32 = __builtin_amdgcn_permlane32_swap((unsigned)u, (unsigned)u, false, false);
-  auto h32 = __builtin_amdgcn_permlane32_swap((unsigned)(u >> 32), (unsigned)(u >> 32), false, false);
-  return join_d(l32[0], h32[0]) + join_d(l32[1], h32[1]);
-}
-
 // ---- gates (scalar, per (row, head) or per channel); evaluated in fp64 and rounded once ----------------------------
 __device__ __forceinline__ double softplus20(double x) {
   return x <= LQ_SOFTPLUS_THRESHOLD ? log1p(exp(x)) : x;

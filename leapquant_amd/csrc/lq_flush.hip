@@ -4,11 +4,12 @@
 // 2246-2331 (lowrank).  Layout of the checkpoint and window buffer: include/lq.h.  The per-head flush and the tile
 // helpers are in lq_flush_core.h.
 //
-// One workgroup of 512 threads (8 waves) per (slot, value head) (the flush is persistent: a workgroup takes its due
-// heads one after another; quantize / dequant / lowrank take one head each); the GDN flush of 128 x 128 heads runs the
-// four-wave layout instead (256 threads, four heads per CU).  Due heads are found on the device (hcnt == L), so the
-// fixed grid is graph-capture safe.
+// One workgroup of 256 threads (four waves, four heads per CU) per (slot, value head), for the flush and the quantize; the
+// flush is persistent (a workgroup takes its due heads one after another).  The dequant of other heads than 128 x 128 at
+// R <= 4 and the low-rank factoriser take 512 threads.  Due heads are found on the device (hcnt == L), so the fixed grid
+// is graph-capture safe.
 #include "lq_flush64_core.h"
+#include "lq_flush8_core.h"
 
 #include <type_traits>
 
@@ -160,16 +161,6 @@ __device__ void flush_listed(unsigned long long& due, const lq_state& st, const 
 // no path's registers weigh on another's (one kernel holding all three spilled up to 64 bytes per lane more).
 enum { FS_STATIC = 0, FS_DYNAMIC = 1, FS_LISTED = 2 };
 
-template <int K_ = KD, int V_ = VD, int RA = 4, int MODE = FS_STATIC>
-__global__ __launch_bounds__(FT) __attribute__((amdgpu_waves_per_eu(4)))
-void flush_kernel(lq_state st, const float* __restrict__ Q0, const int* __restrict__ idx, int N, float qmax,
-                  int* dlist) {
-  __shared__ FlushShared<RA> sh;
-  auto head = [&](int slot, int hv, unsigned, int* sched) { flush_head<K_, V_, RA>(sh, st, Q0, slot, hv, qmax, sched); };
-  if constexpr (MODE == FS_LISTED) flush_listed(sh.due, st, idx, N, dlist, head);
-  else flush_scan<1, MODE == FS_DYNAMIC>(sh.due, st, idx, N, head);
-}
-
 template <int K_ = KD, int V_ = VD, int MODE = FS_STATIC, bool KDA = false>
 __global__ __launch_bounds__(FT4) __attribute__((amdgpu_waves_per_eu(4)))
 void flush4_kernel(lq_state st, const float* __restrict__ Q0, const int* __restrict__ idx, int N, float qmax,
@@ -178,6 +169,18 @@ void flush4_kernel(lq_state st, const float* __restrict__ Q0, const int* __restr
   auto head = [&](int slot, int hv, unsigned, int* sched) {
     flush_head4<K_, V_, true, KDA>(sh, st, Q0, slot, hv, qmax, sched);
   };
+  if constexpr (MODE == FS_LISTED) flush_listed(sh.due, st, idx, N, dlist, head);
+  else flush_scan<1, MODE == FS_DYNAMIC>(sh.due, st, idx, N, head);
+}
+
+// ranks 5 to 8 (GDN 128 x 128 heads)
+template <int RA, int MODE>
+__global__ __launch_bounds__(FT4) __attribute__((amdgpu_waves_per_eu(4)))
+void flush4_kernel(lq_state st, const float* __restrict__ Q0, const int* __restrict__ idx, int N, int* dlist,
+                   float qmax) {
+  static_assert(RA == R8, "eight factor columns");
+  __shared__ FlushShared8 sh;
+  auto head = [&](int slot, int hv, unsigned, int* sched) { flush_head8(sh, st, Q0, slot, hv, qmax, sched); };
   if constexpr (MODE == FS_LISTED) flush_listed(sh.due, st, idx, N, dlist, head);
   else flush_scan<1, MODE == FS_DYNAMIC>(sh.due, st, idx, N, head);
 }
@@ -200,8 +203,7 @@ void flush64_kernel(lq_state st, const float* __restrict__ Q0, const int* __rest
 // low-rank factoriser's iters = 3, kernels.py:2318-2326), then the residual codes.  KDA resets its window as
 // state.py:138-142 does (Pbuf = 0 per channel, Gbuf = 1).
 // ------------------------------------------------------------------------------------------------------------------
-// Four waves per head (256 threads), so that four heads fit on a CU at <= 128 VGPRs (the flush's eight-wave layout
-// fits two): wave w holds key channels 32 w .. 32 w + 31 as two groups of 16, lane l rows 16 nt + (l & 15) and, in group
+// Four waves per head (256 threads), so that four heads fit on a CU at <= 128 VGPRs (an eight-wave layout fits two): wave w holds key channels 32 w .. 32 w + 31 as two groups of 16, lane l rows 16 nt + (l & 15) and, in group
 // cg, channels 32 w + 16 cg + 4 (l >> 4) + i, i < 4 -- 64 fp32 of the state per lane.
 constexpr int QW = 4;                 // waves per head
 constexpr int QT = 64 * QW;           // threads per workgroup
@@ -339,7 +341,7 @@ void quantize_kernel(lq_state st, const float* __restrict__ Q0, const int* __res
   const int tid = threadIdx.x, l = lane_id(), w = wave_id(), q = l >> 4;
   char* base = block_base(st, slot, hv);
   const float* S = (const float*)base;
-  QTile t;                                            // a K_ x V_ < 128 x 128 head zero-padded (see flush_head)
+  QTile t;                                            // a K_ x V_ < 128 x 128 head zero-padded
 #pragma unroll
   for (int cg = 0; cg < 2; ++cg) {
     const int c = 32 * w + 16 * cg + 4 * q;
@@ -1012,15 +1014,14 @@ int lq_launch_flush(const lq_state* st, const float* Q0, const int* idx, int N, 
                     hipStream_t s) {
   if (N == 0) return LQ_OK;
   const int total = N * st->HV;
-  const dim3 g((unsigned)(total < 2 * lq_num_cus() ? total : 2 * lq_num_cus()));   // persistent: two workgroups per CU at most
-  const dim3 g4((unsigned)(total < 4 * lq_num_cus() ? total : 4 * lq_num_cus()));  // four-wave flush: four per CU
+  const dim3 g4((unsigned)(total < 4 * lq_num_cus() ? total : 4 * lq_num_cus()));  // persistent: four workgroups per CU at most
   if (kda) {
     with_mode(st, dlist, total, g4.x, [&](auto m) {
       flush4_kernel<KD, VD, decltype(m)::value, true><<<g4, FT4, 0, s>>>(*st, Q0, idx, N, qmax, dlist);
     });
   } else if (st->K == KD && st->R > 4) {
-    with_mode(st, dlist, total, g.x, [&](auto m) {
-      flush_kernel<KD, VD, 8, decltype(m)::value><<<g, FT, 0, s>>>(*st, Q0, idx, N, qmax, dlist);
+    with_mode(st, dlist, total, g4.x, [&](auto m) {
+      flush4_kernel<8, decltype(m)::value><<<g4, FT4, 0, s>>>(*st, Q0, idx, N, dlist, qmax);
     });
   } else if (st->K == KD) {
     with_mode(st, dlist, total, g4.x, [&](auto m) {

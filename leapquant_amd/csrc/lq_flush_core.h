@@ -1,10 +1,10 @@
-// Per-head flush core shared by liblq's kernels: the end-of-window flush of one (slot, head) on the matrix cores, in
-// an eight-wave (flush_head) and a four-wave (flush_head4) layout, with the helpers the standalone quantize, dequant
-// and low-rank kernels also use.  Semantics: /root/reference/leapquant/kernels.py:1077-2033 (flush).
+// Per-head flush core shared by liblq's kernels: the end-of-window flush of one (slot, head) on the matrix cores
+// (flush_head4, four waves), with the helpers the standalone quantize, dequant and low-rank kernels also use.  Semantics: /root/reference/leapquant/kernels.py:1077-2033 (flush).
 //
-// The head's 128 x 128 matrix lives in registers in the accumulator layout of v_mfma_f32_16x16x32_bf16: wave w owns
-// key channels c in [16w, 16w + 16), lane l holds
-//     acc[nt][i] = M[c][v],   c = 16 w + 4 (l >> 4) + i,   v = 16 nt + (l & 15).
+// The head's 128 x 128 matrix lives in registers in the accumulator layout of v_mfma_f32_16x16x32_bf16: in the eight-wave
+// layout (Tile: dequant_kernel, lowrank_kernel) wave w owns key channels c in [16w, 16w + 16) and lane l holds
+//     acc[nt][i] = M[c][v],   c = 16 w + 4 (l >> 4) + i,   v = 16 nt + (l & 15);
+// the four-wave layout (Tile4) is described at flush_head4.
 // The window rebuild (a rank-L GEMM, ~29 flop/byte at L = 64) runs on MFMA with bf16 hi/lo operands exactly where the
 // reference splits.  The flush's rebuilt matrix B is fp16-exact, so every 128-long contraction of the subspace step
 // (P = B^T Q, Q = B P, the R x R Gram corrections, the rank-R residual updates) is an fp16 MFMA with fp32 accumulation
@@ -125,33 +125,6 @@ __device__ __forceinline__ f16x4 pinned(f16x4 x) {
 
 struct Tile {
   f32x4 a[8];
-};
-
-// RA = factor columns held (4: R <= 4; 8: the R = 8 GDN flush, kernels.py:1091, 1123), as NB = RA / 4 blocks of four
-template <int RA = 4>
-struct FlushShared {
-  static constexpr int NB = RA / 4;
-  union {
-    bf16_t op[3][KD][OPS];     // rebuild operands [c or v][j]
-    struct {                   // after the rebuild
-      f32x4 qpart[NW][NB][VD]; // per-wave partial Q rows
-      float rmx[4 * NW][VD];   // per-(wave, lane group) row maxima of the scaled residual
-      float rq[VD];            // qmax / row scale
-      f16_t ppT[RA][KD];       // P16^T
-      f16x4 qo16[NB][VD];      // old Q rows [v][a], fp16 (residual B operand)
-      f16x4 qn16[NB][VD];      // Q16 rows [v][r] (residual B operand)
-    } r;
-  };
-  float skl[KD];               // column factor of the dequant (Sk, KDA: Sk pc)
-  float svr[VD];               // row factor of the dequant (Sv pn / qmax, KDA: Sv / qmax)
-  float w[LPMAX];
-  f32x4 uoc[NB][KD];           // old U rows [c][a] (KDA: fp16(U pc)), a >= R zero
-  f32x4 qov[NB][VD];           // old Q rows [v][a], a >= R zero
-  f16_t uoT[RA][KD];           // the same, fp16 transposed (MFMA operands)
-  f16_t qoT[RA][VD];
-  f16_t qT[RA][VD];            // Q^T operand of the P steps: fp16-rounded Q0, then Q16
-  f32x4 qv[NB][VD];            // Q rows: fp32 before CholeskyQR, then Q16
-  unsigned long long due;      // persistent flush: due mask of the current candidate chunk
 };
 
 // Thread index as seen by the per-head code.  Re-read through an empty asm at the start of every head so that the
@@ -356,68 +329,12 @@ __device__ __forceinline__ void mgs_n(float (&p0)[N], float (&p1)[N], int R) {
   }
 }
 
-// CholeskyQR pass of the wider-rank flush (R = 8, kernels.py:1744-1772) on N columns: the same factorisation, but a
-// pivot that has lost all but 1e-6 of its Gram diagonal drops its column (1 / L_jj = 0) instead of being floored;
-// columns past R are zero and stay zero.  Gram, factor and substitution run in fp64: a column that depends on the
-// earlier ones leaves a pivot of ~1e-14 G_jj in fp64, but fp32 sums of 128 rows leave ~1e-6 G_jj of rounding -- the
-// drop threshold itself -- so in fp32 whether such a column is dropped would be up to the rounding.
 // lane l's fp64 value, uniform over the wave
 __device__ __forceinline__ double rl_d(double x, int l) {
   const unsigned long long u = __builtin_bit_cast(unsigned long long, x);
   return join_d((unsigned)__builtin_amdgcn_readlane((int)(unsigned)u, l),
                 (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(u >> 32), l));
 }
-template <int N>
-__device__ __forceinline__ void cholqr_pass_drop(float (&p0)[N], float (&p1)[N]) {
-  static_assert(N * (N + 1) / 2 <= 64, "one triangle entry per lane");
-  const int lane = lane_id();
-  double a = 0.0;                                     // lane t: entry t of the packed lower triangle (Gram, then factor)
-#pragma unroll
-  for (int r = 0; r < N; ++r)
-#pragma unroll
-    for (int c = 0; c <= r; ++c) {
-      const double g = sum64d(fma((double)p0[r], (double)p0[c], (double)p1[r] * (double)p1[c]));
-      a = lane == r * (r + 1) / 2 + c ? g : a;
-    }
-#pragma unroll
-  for (int j = 0; j < N; ++j) {
-    const int rj = j * (j + 1) / 2;
-#pragma unroll
-    for (int k = 0; k < j; ++k) {
-      const int rk = k * (k + 1) / 2;
-      double ac = rl_d(a, rj + k);
-#pragma unroll
-      for (int m = 0; m < k; ++m) ac -= rl_d(a, rj + m) * rl_d(a, rk + m);
-      ac *= rl_d(a, rk + k);                          // L_jk (the diagonal entries hold 1 / L_kk)
-      a = lane == rj + k ? ac : a;
-    }
-    const double gjj = rl_d(a, rj + j);
-    double ac = gjj;
-#pragma unroll
-    for (int m = 0; m < j; ++m) {
-      const double ljm = rl_d(a, rj + m);
-      ac -= ljm * ljm;
-    }
-    ac = ac > 1e-6 * gjj + 1e-30 ? 1.0 / sqrt(fmax(ac, 1e-30)) : 0.0;
-    a = lane == rj + j ? ac : a;
-  }
-#pragma unroll
-  for (int s = 0; s < 2; ++s) {
-    float (&p)[N] = s ? p1 : p0;
-    double x[N];
-#pragma unroll
-    for (int j = 0; j < N; ++j) {
-      const int rj = j * (j + 1) / 2;
-      double ac = (double)p[j];
-#pragma unroll
-      for (int m = 0; m < j; ++m) ac -= x[m] * rl_d(a, rj + m);
-      x[j] = ac * rl_d(a, rj + j);
-    }
-#pragma unroll
-    for (int j = 0; j < N; ++j) p[j] = (float)x[j];
-  }
-}
-
 // the 8 code words of the lane's tile entries (issued early; consumed by tile_add_words).  A head of K_ x V_ < 128 x
 // 128 sits zero-padded in the tile: entries past its rows / columns read as 0 (clamped addresses, no divergent load).
 template <int K_ = KD, int V_ = VD>
@@ -432,24 +349,6 @@ __device__ __forceinline__ void load_code_words(uint32_t wds[8], const int8_t* S
     wds[nt] = (cok && (V_ == VD || v < V_)) ? x : 0u;
   }
 }
-// t += the dequantised checkpoint codes  x svr[v] x skl[c], each term rounded to fp32 before the add.  The flush adds
-// them after the window's MFMA products, which it accumulates from zero: the window terms are up to ~20x larger than
-// their sum (they cancel), and an accumulator seeded with the checkpoint term rounds them at a coarser step.
-__device__ __forceinline__ void tile_add_words(Tile& t, const uint32_t wds[8], const float* svr, const float* skl) {
-#pragma clang fp contract(off)
-  const int l = lane_id(), w = wave_id(), q = l >> 4;
-  const int c0 = 16 * w + 4 * q;
-  float kc[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) kc[i] = skl[c0 + i];
-#pragma unroll
-  for (int nt = 0; nt < 8; ++nt) {
-    const float rv = svr[16 * nt + (l & 15)];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) t.a[nt][i] = t.a[nt][i] + ((float)(int)(int8_t)(wds[nt] >> (8 * i)) * rv) * kc[i];
-  }
-}
-
 // acc[c][v] += sum_j A[c][j] B[v][j] over nks 32-entry steps (bf16 operands from LDS, fp32 accumulate)
 __device__ __forceinline__ void rebuild_mfma(Tile& t, const bf16_t (*A)[OPS], const bf16_t (*B)[OPS], int nks) {
   const int l = lane_id(), w = wave_id(), q = l >> 4;
@@ -523,74 +422,6 @@ __device__ __forceinline__ f32x4 sum_parts(const f32x4 (*part)[VD], int v) {
   return s;
 }
 
-// M[a][r] = sum_k X[k][a] Y[k][r] over 128 k for a, r < RA, from the fp16 transposed operands X^T, Y^T ([RA][128]): the
-// MFMA leaves M[a][r] in lane 16 (a >> 2) + r, element a & 3; every lane gets all RA x RA entries
-template <int RA>
-__device__ __forceinline__ void gram_t(const f16_t (*XT)[128], const f16_t (*YT)[128], float (&M)[RA][RA]) {
-  const int l = lane_id(), q = l >> 4, l16 = l & 15;
-  const bool rla = l16 < RA;
-  const f16x8 z8 = {};
-  f32x4 macc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int ks = 0; ks < 4; ++ks) {
-    const f16x8 ao = rla ? *(const f16x8*)&XT[l16][32 * ks + 8 * q] : z8;
-    const f16x8 by = rla ? *(const f16x8*)&YT[l16][32 * ks + 8 * q] : z8;
-    macc = mma32(ao, by, macc);
-  }
-#pragma unroll
-  for (int a = 0; a < RA; ++a)
-#pragma unroll
-    for (int r = 0; r < RA; ++r) M[a][r] = rl(macc[a & 3], 16 * (a >> 2) + r);
-}
-
-// ------------------------------------------------------------------------------------------------------------------
-// flush (kernels.py:1077-2033): one due (slot, head)
-// ------------------------------------------------------------------------------------------------------------------
-// P = B^T Q + pn U_old (Q_old^T Q) for this wave's 16 key channels, fp16-rounded (kernels.py:1580-1700).  Q^T comes
-// from sh.qT; bt[nt] is the transposed packing of B (lane l: B[16 w + (l & 15)][16 nt + 4 (l >> 4) + i]).  Lanes
-// l < 16 RA / 4 return P[16 w + (l & 15)][4 (l >> 4) + i] (zero for columns >= R); the other lanes return zeros.
-template <int RA>
-__device__ __forceinline__ f32x4 p_step(const FlushShared<RA>& sh, const f16x4 bt[8], float pn, int R) {
-  constexpr int NB = RA / 4;
-  const int l = lane_id(), w = wave_id(), q = l >> 4, l16 = l & 15;
-  const bool rla = l16 < RA;
-  const f16x4 z4 = {};
-  float M[RA][RA];                                    // Q_old^T Q
-  gram_t<RA>(sh.qoT, sh.qT, M);
-  // P^T[r][c] = sum_v Q^T[r][v] B[c][v]  (k = v from the transposed packing)
-  f32x4 pacc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int nt = 0; nt < 8; ++nt) {
-    const f16x4 aq = rla ? *(const f16x4*)&sh.qT[l16][16 * nt + 4 * q] : z4;
-    pacc = mma16(aq, bt[nt], pacc);
-  }
-  float uo[RA];
-#pragma unroll
-  for (int b = 0; b < NB; ++b) {
-    const f32x4 x = sh.uoc[b][16 * w + l16];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) uo[4 * b + i] = x[i];
-  }
-  f32x4 p;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    float corr = 0.f;
-#pragma unroll
-    for (int a = 0; a < RA; ++a) {
-      float m = M[a][i];                              // column r = 4 q + i of this lane
-#pragma unroll
-      for (int b = 1; b < NB; ++b) m = q == b ? M[a][4 * b + i] : m;
-      corr = a == 0 ? uo[0] * m : corr + uo[a] * m;
-    }
-    p[i] = (q < NB && 4 * q + i < R) ? hround(pacc[i] + pn * corr) : 0.f;
-  }
-  return p;
-}
-
-// A GDN head of K_ x V_ < 128 x 128 (kernels.py:1089: (64, 128), (64, 64)) runs zero-padded in the 128 x 128 tile:
-// its loads read zeros past its rows / columns, every product and Gram sum then only adds exact zeros, the column
-// means divide by V_, and the stores write its own rows / columns only.  RA = 8 (GDN 128 x 128, R = 8): the factor
-// products carry eight columns (lanes l < 32 of each MFMA) and CholeskyQR drops dependent columns (kernels.py:1744-1772).
 // Dynamic head schedule of the persistent flush (lq_state.sched, LQ_SCHED_INTS ints): eight counters 256 bytes apart;
 // workgroup b uses counter b % 8 (the dispatcher deals workgroups round-robin over the eight XCDs), so that the
 // grid's takes spread over eight addresses instead of queueing on one (one counter measured 41.5 -> 51 us on a flush
@@ -636,333 +467,11 @@ __device__ __forceinline__ int take_result(int take) {
   return take;
 }
 
-template <int K_ = KD, int V_ = VD, int RA = 4>
-__device__ void flush_head(FlushShared<RA>& sh, const lq_state& st, const float* __restrict__ Q0, int slot, int hv,
-                           float qmax, int* sched = nullptr) {
-  static_assert(RA == 4 || (RA == 8 && K_ == KD && V_ == VD), "R = 8: 128 x 128 heads");
-  constexpr int NB = RA / 4;
-  const int HV = st.HV, L = st.L, R = st.R;
-  const long long sh_ = (long long)slot * HV + hv;
-  const int tid = opaque_tid(), l = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), q = l >> 4, l16 = l & 15;
-  const int qb = q < NB ? q : NB - 1;                 // this lane's factor block in the MFMA operands (lanes < 16 NB)
-  char* base = block_base(st, slot, hv);
-  int8_t* Sq = (int8_t*)base;
-  float* Sk = (float*)(base + V_ * K_);
-  float* Sv = Sk + K_;
-  f16_t* UQ = (f16_t*)(Sv + V_);
-  const int LP = (L + 31) & ~31;
-
-  // ---- stage 1: every load of the head up front (scalars, scales, factors, window rows, code words) ----
-  const float pn = fmaxf(st.Pbuf[sh_], LQ_PNMIN);     // kernels.py:1471
-  const float rpn = 1.0f / pn;                        // kernels.py:1477
-  const int cv = tid & 127;                           // column (tid < 128) or row (128 <= tid < 256) of the stage-1 loads
-  const bool colt = tid < KD;
-  const int nc = colt ? K_ : V_;                      // this thread's column / row count
-  const bool cok = (K_ == KD && V_ == VD) || cv < nc;
-  const int cvc = (K_ == KD && V_ == VD) ? cv : min(cv, nc - 1);
-  const int vq = V_ == VD ? cv : min(cv, V_ - 1);
-  const float scv = cok ? (colt ? Sk[cvc] : Sv[cvc]) : 0.f;
-  float uqv[RA], q0v[RA];
-#pragma unroll
-  for (int a = 0; a < RA; ++a) {
-    const float x = h2f(UQ[min(a, R - 1) * (K_ + V_) + (colt ? 0 : K_) + cvc]);
-    uqv[a] = cok ? x : 0.f;
-    const float y = Q0[vq * R + min(a, R - 1)];
-    q0v[a] = (V_ == VD || cv < V_) ? y : 0.f;
-  }
-  const float wv = st.Wbuf[sh_ * L + min(tid, L - 1)];
-  WinRegs win;
-  load_window<K_, V_>(win, st, slot, hv, L, LP);
-  uint32_t wds[8];
-  load_code_words<K_, V_>(wds, Sq);
-
-  if (tid < KD) {
-    const int c = cv;
-    sh.skl[c] = scv;
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      f32x4 u;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int a = 4 * b + i;
-        u[i] = a < R ? uqv[a] : 0.f;
-        sh.uoT[a][c] = f2h(u[i]);
-      }
-      sh.uoc[b][c] = u;
-    }
-  } else if (tid < KD + VD) {
-    const int v = cv;
-    sh.svr[v] = scv * (pn / qmax);                                                    // kernels.py:1483
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      f32x4 o;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int a = 4 * b + i;
-        o[i] = a < R ? uqv[a] : 0.f;
-        sh.qoT[a][v] = f2h(o[i]);
-        sh.qT[a][v] = f2h(a < R ? hround(q0v[a]) : 0.f);                              // kernels.py:1573-1577
-      }
-      sh.qov[b][v] = o;
-    }
-  }
-  if (tid < LPMAX) sh.w[tid] = tid < L ? wv : 0.f;
-  __syncthreads();
-  store_window(sh, win, L, LP);
-  __syncthreads();
-
-  // ---- stage 2: B = deq(S0) pn + window, fp16 (kernels.py:1483-1571) ----
-  f16x4 bh[8], bt[8];                                 // B packed: k = c (tile layout) and k = v (transposed)
-  {
-    Tile t;
-#pragma unroll
-    for (int nt = 0; nt < 8; ++nt) t.a[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    rebuild_mfma(t, sh.op[0], sh.op[1], LP / 32);
-    rebuild_mfma(t, sh.op[0], sh.op[2], LP / 32);
-    tile_add_words(t, wds, sh.svr, sh.skl);
-    f16x4 ident;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) ident[i] = (4 * q + i == l16) ? (_Float16)1.0f : (_Float16)0.0f;
-#pragma unroll
-    for (int nt = 0; nt < 8; ++nt) {
-      bh[nt] = to_h4(t.a[nt]);                        // the fp16 rounding of B
-      bt[nt] = to_h4(mma16(bh[nt], ident, f32x4{0.f, 0.f, 0.f, 0.f}));   // exact: B^T block through the identity
-    }
-  }
-
-  // ---- stage 3: subspace iteration (ITERS = 1) with the algebraic rank-R corrections (kernels.py:1580-1842) ----
-  const f32x4 p16 = p_step<RA>(sh, bt, pn, R);        // P16 rows of this wave (lanes < 16 NB)
-  __syncthreads();                                    // every wave is past the rebuild: the op region is free
-  if (tid < VD) {
-#pragma unroll
-    for (int b = 0; b < NB; ++b) sh.r.qo16[b][tid] = to_h4(sh.qov[b][tid]);
-  }
-  // Q = B P16 + pn Q_old (U_old^T P16): per-wave partials of B P16 over the wave's 16 channels, summed below
-  if (q < NB) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) sh.r.ppT[4 * q + i][16 * w + l16] = f2h(p16[i]);
-  }
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  {
-    const f16x4 z4 = {};
-    const f16x4 ap = l16 < RA ? *(const f16x4*)&sh.r.ppT[l16][16 * w + 4 * q] : z4;   // A[r][c] = P16^T
-#pragma unroll
-    for (int nt = 0; nt < 8; ++nt) {
-      const f32x4 d = mma16(ap, bh[nt], f32x4{0.f, 0.f, 0.f, 0.f});                 // Q^T[4 q + i][16 nt + l]
-      if (q < NB) sh.r.qpart[w][qb][16 * nt + l16] = d;
-    }
-  }
-  __syncthreads();
-  if (tid < VD) {                                     // waves 0 and 1: one row v per thread
-    // M2[a][r] = sum_c U_old[c][a] P16[c][r] over all 128 channels (every column of P16 is in ppT now)
-    float M2[RA][RA];
-    gram_t<RA>(sh.uoT, sh.r.ppT, M2);
-    const int v = tid;
-    float qo[RA];
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      const f32x4 x = sh.qov[b][v];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) qo[4 * b + i] = x[i];
-    }
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      f32x4 s = sh.r.qpart[0][b][v];
-#pragma unroll
-      for (int w2 = 1; w2 < NW; ++w2) s += sh.r.qpart[w2][b][v];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float corr = qo[0] * M2[0][4 * b + i];
-#pragma unroll
-        for (int a = 1; a < RA; ++a) corr += qo[a] * M2[a][4 * b + i];
-        s[i] += pn * corr;
-      }
-      sh.qv[b][v] = s;
-    }
-  }
-  __syncthreads();
-  // CholeskyQR2 (wave 0), fp16 Q.  The serial phases of one wave run at raised wave priority: the CU's other workgroup
-  // competes for the same SIMDs while this one's other waves wait at the barrier (config 3: flush 339 -> 331 us,
-  // quantize 222 -> 214 us with the same in its MGS phases)
-  if (w == 0) {
-    __builtin_amdgcn_s_setprio(3);
-    if constexpr (RA == 4) {
-      f32x4 p0 = sh.qv[0][l], p1 = sh.qv[0][l + 64];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) { if (r >= R) { p0[r] = 0.f; p1[r] = 0.f; } }
-      cholqr_pass(p0, p1);
-      cholqr_pass(p0, p1);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        p0[r] = r < R ? hround(p0[r]) : 0.f;
-        p1[r] = r < R ? hround(p1[r]) : 0.f;
-        sh.qT[r][l] = f2h(p0[r]);
-        sh.qT[r][l + 64] = f2h(p1[r]);
-      }
-      sh.qv[0][l] = p0;
-      sh.qv[0][l + 64] = p1;
-      sh.r.qn16[0][l] = to_h4(p0);
-      sh.r.qn16[0][l + 64] = to_h4(p1);
-    } else {
-      float p0[RA], p1[RA];
-#pragma unroll
-      for (int b = 0; b < NB; ++b) {
-        const f32x4 x0 = sh.qv[b][l], x1 = sh.qv[b][l + 64];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          p0[4 * b + i] = 4 * b + i < R ? x0[i] : 0.f;
-          p1[4 * b + i] = 4 * b + i < R ? x1[i] : 0.f;
-        }
-      }
-      cholqr_pass_drop<RA>(p0, p1);
-      cholqr_pass_drop<RA>(p0, p1);
-#pragma unroll
-      for (int b = 0; b < NB; ++b) {
-        f32x4 y0, y1;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int r = 4 * b + i;
-          y0[i] = r < R ? hround(p0[r]) : 0.f;
-          y1[i] = r < R ? hround(p1[r]) : 0.f;
-          sh.qT[r][l] = f2h(y0[i]);
-          sh.qT[r][l + 64] = f2h(y1[i]);
-        }
-        sh.qv[b][l] = y0;
-        sh.qv[b][l + 64] = y1;
-        sh.r.qn16[b][l] = to_h4(y0);
-        sh.r.qn16[b][l + 64] = to_h4(y1);
-      }
-    }
-    __builtin_amdgcn_s_setprio(0);
-  }
-  __syncthreads();
-  const f32x4 u16 = p_step<RA>(sh, bt, pn, R);        // U16 = P step with Q16 (lanes < 16 NB: rows 16 w + l)
-
-  // ---- stage 4: residual E = fp16(pn (B / pn + Q_old U_old^T) - Q U^T) (kernels.py:1888-1928) ----
-  // E kept packed in B's registers (B is dead after the Q partials), consumed through v_fma_mix_f32 as in flush_head4
-  {
-    const f16x4 z4 = {};
-    const f16x4 auo = q < NB ? to_h4(sh.uoc[qb][16 * w + l16]) : z4;                // A[c][a] = U_old
-    const f16x4 aun = q < NB ? to_h4(-u16) : z4;                                     // A[c][r] = -U16
-#pragma unroll
-    for (int nt = 0; nt < 8; ++nt) {
-      const int v = 16 * nt + l16;
-      // B[a][v] = Q_old^T, B[r][v] = Q16^T; rows past the lane's factor block meet the zero columns of A
-      const f16x4 bqo = sh.r.qo16[qb][v];
-      const f16x4 bqn = sh.r.qn16[qb][v];
-      const f16x4 b = bh[nt];
-      f32x4 e = {h4mul<0>(b, rpn), h4mul<1>(b, rpn), h4mul<2>(b, rpn), h4mul<3>(b, rpn)};
-      e = mma16(auo, bqo, e);
-      e *= pn;
-      e = mma16(aun, bqn, e);
-      bh[nt] = to_h4(e);                                                            // E, fp16
-    }
-  }
-
-  // ---- stage 5: column smoothing scales (kernels.py:1929-1958) ----
-  float rsk[4];
-  {
-    float cs[4], x0 = 0.f, x1 = 0.f, x2 = 0.f, x3 = 0.f;
-#pragma unroll
-    for (int nt = 0; nt < 8; ++nt) {
-      x0 = h4abs_add<0>(bh[nt], x0);
-      x1 = h4abs_add<1>(bh[nt], x1);
-      x2 = h4abs_add<2>(bh[nt], x2);
-      x3 = h4abs_add<3>(bh[nt], x3);
-    }
-    cs[0] = sum16(x0);
-    cs[1] = sum16(x1);
-    cs[2] = sum16(x2);
-    cs[3] = sum16(x3);
-    // the square root and division once per column: lane l takes column 4 q + (l & 3) of its row group
-    const int ic = l & 3;
-    const float msum = (ic == 0 ? cs[0] : ic == 1 ? cs[1] : ic == 2 ? cs[2] : cs[3]) * (1.0f / V_);
-    const float sq = sqrtf(msum);
-    const float rs = fminf(1.0f / sq, 1.0f / LQ_EPS);
-    if (l16 < 4 && (K_ == KD || 16 * w + 4 * q + l16 < K_)) Sk[16 * w + 4 * q + l16] = fmaxf(sq, LQ_EPS);
-    rsk[0] = dpp<0x00>(rs);                           // quad_perm [i, i, i, i]: column i of the lane's quad
-    rsk[1] = dpp<0x55>(rs);
-    rsk[2] = dpp<0xaa>(rs);
-    rsk[3] = dpp<0xff>(rs);
-  }
-  int next = 0;                                       // dynamic schedule: this workgroup's next candidate
-  if (sched && tid == 0) next = sched_take(sched);
-  // ---- stage 6: row scales and codes (kernels.py:1974-2009) ----
-  Tile t;                                             // E rsk, fp32
-#pragma unroll
-  for (int nt = 0; nt < 8; ++nt) {
-    float m = 0.f;
-    const f16x4 e = bh[nt];
-    t.a[nt] = f32x4{h4mul<0>(e, rsk[0]), h4mul<1>(e, rsk[1]), h4mul<2>(e, rsk[2]), h4mul<3>(e, rsk[3])};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) m = fmaxf(m, fabsf(t.a[nt][i]));
-    sh.r.rmx[4 * w + q][16 * nt + l16] = m;
-  }
-  __syncthreads();
-  if (tid < VD) {
-    float m = sh.r.rmx[0][tid];
-#pragma unroll
-    for (int k = 1; k < 4 * NW; ++k) m = fmaxf(m, sh.r.rmx[k][tid]);
-    const float rmax = fmaxf(m, LQ_EPS);
-    if (V_ == VD || tid < V_) Sv[tid] = rmax;
-    sh.r.rq[tid] = qmax * (1.0f / rmax);
-  }
-  __syncthreads();
-  uint32_t cw[8];                                     // code words of rows 16 nt + l16, channels 16 w + 4 q ..
-#pragma unroll
-  for (int nt = 0; nt < 8; ++nt) {
-    const int v = 16 * nt + l16;
-    const float rq = sh.r.rq[v];
-    uint32_t b[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) b[i] = __float_as_uint(__builtin_fmaf(t.a[nt][i], rq, 12582912.0f));   // RNE via 1.5 2^23
-    const uint32_t lo = __builtin_amdgcn_perm(b[1], b[0], 0x0c0c0400u), hi = __builtin_amdgcn_perm(b[3], b[2], 0x0c0c0400u);
-    cw[nt] = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
-  }
-  if constexpr (K_ == KD && V_ == VD) {
-    // a 4 x 4 transpose over the lane groups (register j of group q -> register q of group j) gives lane (q, l16) the
-    // four words of row 16 (4 m + q) + l16, channels 16 w .. 16 w + 15: two 16-byte stores instead of eight 4-byte ones
-#pragma unroll
-    for (int m = 0; m < 2; ++m) {
-      uint32_t a0 = cw[4 * m], a1 = cw[4 * m + 1], a2 = cw[4 * m + 2], a3 = cw[4 * m + 3];
-      swap32(a0, a2);
-      swap32(a1, a3);
-      swap16(a0, a1);
-      swap16(a2, a3);
-      *(uint4*)(Sq + (16 * (4 * m + q) + l16) * KD + 16 * w) = make_uint4(a0, a1, a2, a3);
-    }
-  } else {
-#pragma unroll
-    for (int nt = 0; nt < 8; ++nt) {
-      const int v = 16 * nt + l16;
-      if ((K_ == KD || 16 * w + 4 * q < K_) && (V_ == VD || v < V_)) *(uint32_t*)(Sq + v * K_ + 16 * w + 4 * q) = cw[nt];
-    }
-  }
-  // ---- stage 7: factors, window reset (kernels.py:1836-1842, 2014-2025) ----
-  if (q < NB && (K_ == KD || 16 * w + l16 < K_)) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (4 * q + i < R) UQ[(4 * q + i) * (K_ + V_) + 16 * w + l16] = f2h(u16[i]);
-  }
-  if (tid < V_) {
-    for (int r = 0; r < R; ++r) UQ[r * (K_ + V_) + K_ + tid] = f2h(sh.qv[r >> 2][tid][r & 3]);
-  }
-  if (tid < L) st.Wbuf[sh_ * L + tid] = 0.f;
-  if (tid == 0) {
-    st.Pbuf[sh_] = 1.f;
-    st.hcnt[sh_] = 0;
-    if (sched) sh.due = (unsigned long long)sched_candidate(take_result(next));
-  }
-  __syncthreads();                                    // LDS reuse by the next head of this workgroup
-}
-
 // ------------------------------------------------------------------------------------------------------------------
 // Four-wave flush (GDN with R <= 4, and KDA): one due head per workgroup of 256 threads, <= 40 KiB LDS and <= 128
-// VGPRs, so that four heads share a CU (the eight-wave flush above fits two).  The flush is latency-bound -- each head
-// is a chain of dependent, barrier-separated phases -- so heads in flight per CU set its rate.  Same arithmetic, in the
-// same order, as flush_head; only the distribution over the lanes differs: wave w owns key channels [32 w, 32 w + 32)
-// as two groups g of 16, and lane l holds
+// VGPRs, so that four heads share a CU (a layout of eight waves per head fits two, and took 1.4 times as long).  Each head is
+// a chain of dependent, barrier-separated phases, of which four per CU keep the VALU issue busy.  Wave w owns key channels
+// [32 w, 32 w + 32) as two groups g of 16, and lane l holds
 //     a[g][nt][i] = M[c][v],   c = 32 w + 16 g + 4 (l >> 4) + i,   v = 16 nt + (l & 15).
 // The window is staged and multiplied in halves of 32 entries.  KDA (kernels.py:1443-1471, 1519): pn = 1, the
 // per-channel decay exp(Pbuf[c]) folds into the column factor Sk and the old U rows, and the window's keys enter as
@@ -995,6 +504,7 @@ struct Tile4 {
 
 template <bool CF>
 struct FlushShared4T {
+  static constexpr bool conflict_free = CF;
   static constexpr int FP = CF ? FTP : 0, RP = CF ? RMP : 0;
   union {
     bf16_t op[3][KD][OPS4];    // rebuild operands of one window half [c or v][j]
@@ -1054,10 +564,11 @@ __device__ __forceinline__ void load_half(WinHalf& r, const lq_state& st, int sl
 // the even group's) write c8 + (e + 4) mod 8: rows 8 + 4 or 8 - 4 apart are 80 or 240 dwords apart, 16 banks off, so
 // the two groups of a half-wave write disjoint banks (rows exactly 8 apart, 160 dwords, share all 16).  Without CF no
 // rotation (the same bytes either way).
-template <bool KDA = false, bool CF>
-__device__ __forceinline__ void store_half(FlushShared4T<CF>& sh, const WinHalf& r, int h, int hf) {
+template <bool KDA = false, class SH>
+__device__ __forceinline__ void store_half(SH& sh, const WinHalf& r, int h, int hf) {
   // the split is of the fp32-rounded product: no fusing of w u into the lo subtraction (kernels.py:1509-1511)
 #pragma clang fp contract(off)
+  constexpr bool CF = SH::conflict_free;
   const int t = tid4(), jl = 2 * (t % 16), c8 = (t / 16) * 8;
   const bool rot = CF && ((t / 16) & 1);
   const int j0 = HALF * hf + jl;
@@ -1283,7 +794,9 @@ __device__ __forceinline__ void load_code_words4(uint32_t wds[2][8], const int8_
     }
   }
 }
-// t += codes x svr[v] x skl[c], each term rounded to fp32 before the add (after the window products; see flush_head)
+// t += codes x svr[v] x skl[c], each term rounded to fp32 before the add after the window products:
+// those are up to ~20x larger than their sum (they cancel), and an accumulator seeded with the checkpoint term rounds
+// them at a coarser step
 __device__ __forceinline__ void tile_add_words4(Tile4& t, const uint32_t wds[2][8], const float* svr,
                                                 const float* skl) {
 #pragma clang fp contract(off)
@@ -1366,6 +879,108 @@ __device__ __forceinline__ void p_step4(const FlushShared4T<CF>& sh, const f16x4
     const float pa = g1 ? pacc[1][r] : pacc[0][r];
     const float corr = uo[0] * M[0][r] + uo[1] * M[1][r] + uo[2] * M[2][r] + uo[3] * M[3][r];
     pg[r] = r < R ? hround(pa + pn * corr) : 0.f;
+  }
+}
+
+// The smoothed residual's scales and codes, from E (fp16, the tile layout) to the checkpoint block at `base`; takes the
+// workgroup's next candidate of the dynamic schedule on the way (see sched_take).
+template <int K_, int V_, class SH>
+__device__ __forceinline__ void store_codes4(SH& sh, const f16x4 (&bh)[2][8], char* base, float qmax, int* sched,
+                                             int& next) {
+  const int tid = tid4(), l = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), q = l >> 4, l16 = l & 15;
+  int8_t* Sq = (int8_t*)base;
+  float* Sk = (float*)(base + V_ * K_);
+  float* Sv = Sk + K_;
+  // ---- stage 5: column smoothing scales (kernels.py:1929-1958) ----
+  float rsk[2][4];
+#pragma unroll
+  for (int g = 0; g < 2; ++g) {
+    float cs[4], x0 = 0.f, x1 = 0.f, x2 = 0.f, x3 = 0.f;
+#pragma unroll
+    for (int nt = 0; nt < 8; ++nt) {
+      x0 = h4abs_add<0>(bh[g][nt], x0);
+      x1 = h4abs_add<1>(bh[g][nt], x1);
+      x2 = h4abs_add<2>(bh[g][nt], x2);
+      x3 = h4abs_add<3>(bh[g][nt], x3);
+    }
+    cs[0] = sum16(x0);
+    cs[1] = sum16(x1);
+    cs[2] = sum16(x2);
+    cs[3] = sum16(x3);
+    // the square root and division once per column: lane l takes column 4 q + (l & 3) of its row group
+    const int ic = l & 3;
+    const float msum = (ic == 0 ? cs[0] : ic == 1 ? cs[1] : ic == 2 ? cs[2] : cs[3]) * (1.0f / V_);
+    const float sq = sqrtf(msum);
+    const float rs = fminf(1.0f / sq, 1.0f / LQ_EPS);
+    const int cc = 32 * w + 16 * g + 4 * q + l16;
+    if (l16 < 4 && (K_ == KD || cc < K_)) Sk[cc] = fmaxf(sq, LQ_EPS);
+    rsk[g][0] = dpp<0x00>(rs);                        // quad_perm [i, i, i, i]: column i of the lane's quad
+    rsk[g][1] = dpp<0x55>(rs);
+    rsk[g][2] = dpp<0xaa>(rs);
+    rsk[g][3] = dpp<0xff>(rs);
+  }
+  if (sched && tid == 0) next = sched_take(sched);
+  // ---- stage 6: row scales and codes (kernels.py:1974-2009) ----
+  Tile4 t;                                            // E rsk, fp32
+#pragma unroll
+  for (int nt = 0; nt < 8; ++nt) {
+    float m = 0.f;
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      const f16x4 e = bh[g][nt];
+      t.a[g][nt] = f32x4{h4mul<0>(e, rsk[g][0]), h4mul<1>(e, rsk[g][1]), h4mul<2>(e, rsk[g][2]),
+                         h4mul<3>(e, rsk[g][3])};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) m = fmaxf(m, fabsf(t.a[g][nt][i]));
+    }
+    sh.r.rmx[4 * w + q][16 * nt + l16] = m;
+  }
+  __syncthreads();
+  if (tid < VD) {
+    float m = sh.r.rmx[0][tid];
+#pragma unroll
+    for (int k = 1; k < 4 * NW4; ++k) m = fmaxf(m, sh.r.rmx[k][tid]);
+    const float rmax = fmaxf(m, LQ_EPS);
+    if (V_ == VD || tid < V_) Sv[tid] = rmax;
+    sh.r.rq[tid] = qmax * (1.0f / rmax);
+  }
+  __syncthreads();
+  uint32_t cw[2][8];                                  // code words, laid out as load_code_words4 delivers them
+#pragma unroll
+  for (int nt = 0; nt < 8; ++nt) {
+    const int v = 16 * nt + l16;
+    const float rq = sh.r.rq[v];
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      uint32_t b[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) b[i] = __float_as_uint(__builtin_fmaf(t.a[g][nt][i], rq, 12582912.0f));   // RNE via 1.5 2^23
+      const uint32_t lo = __builtin_amdgcn_perm(b[1], b[0], 0x0c0c0400u), hi = __builtin_amdgcn_perm(b[3], b[2], 0x0c0c0400u);
+      cw[g][nt] = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+    }
+  }
+  if constexpr (K_ == KD && V_ == VD) {
+    // the inverse of load_code_words4's transpose, then four 16-byte stores per lane (each wave instruction 32 rows x
+    // 32 bytes) instead of sixteen 4-byte ones
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      uint32_t a0 = cw[0][2 * k], a1 = cw[1][2 * k], a2 = cw[0][2 * k + 1], a3 = cw[1][2 * k + 1];
+      swap16(a0, a1);
+      swap16(a2, a3);
+      swap32(a0, a2);
+      swap32(a1, a3);
+      *(uint4*)(Sq + (16 * (2 * k + (q >> 1)) + l16) * KD + 32 * w + 16 * (q & 1)) = make_uint4(a0, a1, a2, a3);
+    }
+  } else {
+#pragma unroll
+    for (int nt = 0; nt < 8; ++nt) {
+      const int v = 16 * nt + l16;
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        const int c = 32 * w + 16 * g + 4 * q;
+        if ((K_ == KD || c < K_) && (V_ == VD || v < V_)) *(uint32_t*)(Sq + v * K_ + c) = cw[g][nt];
+      }
+    }
   }
 }
 
@@ -1593,98 +1208,8 @@ __device__ void flush_head4(FlushShared4T<CF>& sh, const lq_state& st, const flo
     }
   }
 
-  // ---- stage 5: column smoothing scales (kernels.py:1929-1958) ----
-  float rsk[2][4];
-#pragma unroll
-  for (int g = 0; g < 2; ++g) {
-    float cs[4], x0 = 0.f, x1 = 0.f, x2 = 0.f, x3 = 0.f;
-#pragma unroll
-    for (int nt = 0; nt < 8; ++nt) {
-      x0 = h4abs_add<0>(bh[g][nt], x0);
-      x1 = h4abs_add<1>(bh[g][nt], x1);
-      x2 = h4abs_add<2>(bh[g][nt], x2);
-      x3 = h4abs_add<3>(bh[g][nt], x3);
-    }
-    cs[0] = sum16(x0);
-    cs[1] = sum16(x1);
-    cs[2] = sum16(x2);
-    cs[3] = sum16(x3);
-    // the square root and division once per column: lane l takes column 4 q + (l & 3) of its row group
-    const int ic = l & 3;
-    const float msum = (ic == 0 ? cs[0] : ic == 1 ? cs[1] : ic == 2 ? cs[2] : cs[3]) * (1.0f / V_);
-    const float sq = sqrtf(msum);
-    const float rs = fminf(1.0f / sq, 1.0f / LQ_EPS);
-    const int cc = 32 * w + 16 * g + 4 * q + l16;
-    if (l16 < 4 && (K_ == KD || cc < K_)) Sk[cc] = fmaxf(sq, LQ_EPS);
-    rsk[g][0] = dpp<0x00>(rs);                        // quad_perm [i, i, i, i]: column i of the lane's quad
-    rsk[g][1] = dpp<0x55>(rs);
-    rsk[g][2] = dpp<0xaa>(rs);
-    rsk[g][3] = dpp<0xff>(rs);
-  }
   int next = 0;                                       // dynamic schedule: this workgroup's next candidate
-  if (sched && tid == 0) next = sched_take(sched);
-  // ---- stage 6: row scales and codes (kernels.py:1974-2009) ----
-  Tile4 t;                                            // E rsk, fp32
-#pragma unroll
-  for (int nt = 0; nt < 8; ++nt) {
-    float m = 0.f;
-#pragma unroll
-    for (int g = 0; g < 2; ++g) {
-      const f16x4 e = bh[g][nt];
-      t.a[g][nt] = f32x4{h4mul<0>(e, rsk[g][0]), h4mul<1>(e, rsk[g][1]), h4mul<2>(e, rsk[g][2]),
-                         h4mul<3>(e, rsk[g][3])};
-#pragma unroll
-      for (int i = 0; i < 4; ++i) m = fmaxf(m, fabsf(t.a[g][nt][i]));
-    }
-    sh.r.rmx[4 * w + q][16 * nt + l16] = m;
-  }
-  __syncthreads();
-  if (tid < VD) {
-    float m = sh.r.rmx[0][tid];
-#pragma unroll
-    for (int k = 1; k < 4 * NW4; ++k) m = fmaxf(m, sh.r.rmx[k][tid]);
-    const float rmax = fmaxf(m, LQ_EPS);
-    if (V_ == VD || tid < V_) Sv[tid] = rmax;
-    sh.r.rq[tid] = qmax * (1.0f / rmax);
-  }
-  __syncthreads();
-  uint32_t cw[2][8];                                  // code words, laid out as load_code_words4 delivers them
-#pragma unroll
-  for (int nt = 0; nt < 8; ++nt) {
-    const int v = 16 * nt + l16;
-    const float rq = sh.r.rq[v];
-#pragma unroll
-    for (int g = 0; g < 2; ++g) {
-      uint32_t b[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) b[i] = __float_as_uint(__builtin_fmaf(t.a[g][nt][i], rq, 12582912.0f));   // RNE via 1.5 2^23
-      const uint32_t lo = __builtin_amdgcn_perm(b[1], b[0], 0x0c0c0400u), hi = __builtin_amdgcn_perm(b[3], b[2], 0x0c0c0400u);
-      cw[g][nt] = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
-    }
-  }
-  if constexpr (K_ == KD && V_ == VD) {
-    // the inverse of load_code_words4's transpose, then four 16-byte stores per lane (each wave instruction 32 rows x
-    // 32 bytes) instead of sixteen 4-byte ones
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      uint32_t a0 = cw[0][2 * k], a1 = cw[1][2 * k], a2 = cw[0][2 * k + 1], a3 = cw[1][2 * k + 1];
-      swap16(a0, a1);
-      swap16(a2, a3);
-      swap32(a0, a2);
-      swap32(a1, a3);
-      *(uint4*)(Sq + (16 * (2 * k + (q >> 1)) + l16) * KD + 32 * w + 16 * (q & 1)) = make_uint4(a0, a1, a2, a3);
-    }
-  } else {
-#pragma unroll
-    for (int nt = 0; nt < 8; ++nt) {
-      const int v = 16 * nt + l16;
-#pragma unroll
-      for (int g = 0; g < 2; ++g) {
-        const int c = 32 * w + 16 * g + 4 * q;
-        if ((K_ == KD || c < K_) && (V_ == VD || v < V_)) *(uint32_t*)(Sq + v * K_ + c) = cw[g][nt];
-      }
-    }
-  }
+  store_codes4<K_, V_>(sh, bh, base, qmax, sched, next);
   // ---- stage 7: factors, window reset (kernels.py:1836-1842, 2014-2025) ----
   if constexpr (K_ == KD && V_ == VD) {
     // the factor rows [U_r | Q_r] from their fp16 tables (U16^T above, Q16^T from the CholeskyQR): thread t writes

@@ -11,6 +11,7 @@
 //   * KDA (K = V = 128): two waves per value head, the same matrix-core dots, the per-channel gate folded into the
 //     key operands and the window's decayed keys formed by a backward scan split between the two waves.
 #include "lq_flush64_core.h"
+#include "lq_flush8_core.h"
 
 namespace {
 
@@ -116,15 +117,17 @@ template <int K_, int V_, int G, bool FL, int RM>
 struct StepLds {
   StepShared<K_, V_, G, RM> st[1];
 };
-template <int K_>
+template <int K_, int RM>
 struct FlushLds { using type = lqf::FlushShared4T<true>; };
 template <>
-struct FlushLds<64> { using type = lqf::FlushShared64; };
+struct FlushLds<64, 4> { using type = lqf::FlushShared64; };
+template <>
+struct FlushLds<128, 16> { using type = lqf::FlushShared8; };   // ranks 5 to 8
 template <int K_, int V_, int G, int RM>
 struct StepLds<K_, V_, G, true, RM> {
   union {
     StepShared<K_, V_, G, RM> st[step_units<G, true>()];
-    typename FlushLds<K_>::type fl[G == 4 ? 2 : 1];
+    typename FlushLds<K_, RM>::type fl[G == 4 ? 2 : 1];
   };
 };
 // with helper waves: one unit, and a flush per value head
@@ -132,13 +135,13 @@ template <int K_, int V_, int G>
 struct WideLds {
   union {
     StepShared<K_, V_, G, 4> st[1];
-    typename FlushLds<K_>::type fl[G];
+    typename FlushLds<K_, 4>::type fl[G];
   };
 };
 
 // Flushes the due ones of the NH value heads hv0 .. of one row (bit i of due: head hv0 + i), all of one slot, on NG
 // groups of 256 threads; `due` (not zero) is uniform over the workgroup.
-template <int K_, int V_, int G, int NH, int NG, class LDS>
+template <int K_, int V_, int G, int NH, int NG, int RM = 4, class LDS>
 __device__ __forceinline__ void flush_due(LDS& lds, const lq_state& st, const float* Q0, int slot, int hv0,
                                           unsigned due, float qm) {
   const int sub = NG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;   // this thread's group
@@ -155,6 +158,7 @@ __device__ __forceinline__ void flush_due(LDS& lds, const lq_state& st, const fl
       if (m == 0) continue;
       const int i = NG * p + (NG > 1 && ((m >> sub) & 1u) ? sub : __ffs(m) - 1);
       if constexpr (K_ == 64) lqf::flush_head64<V_, 1>(lds.fl[sub], st, Q0, slot, hv0 + i, 1u, qm);
+      else if constexpr (RM > 4) lqf::flush_head8(lds.fl[sub], st, Q0, slot, hv0 + i, qm);
       else lqf::flush_head4<K_, V_, true>(lds.fl[sub], st, Q0, slot, hv0 + i, qm);
     }
   }
@@ -170,7 +174,7 @@ __device__ __forceinline__ unsigned gdn_step(LDS& lds, const lq_state& st, const
                                              int* dlist, const float* Q0, int& slot_) {
   static_assert(!DF || FL, "deferred flush (lq_gdn_decode_deferred): the fused decode kernel");
   static_assert(!DF || (K_ == 128 && V_ == 128 && G == 2), "deferred flush: 128 x 128 heads, two per key head");
-  static_assert(RM == 4 || (RM == 16 && K_ == 128 && V_ == 128 && !FL), "ranks above 4: 128 x 128 heads, no fused flush");
+  static_assert(RM == 4 || (RM == 16 && K_ == 128 && V_ == 128 && !DF), "ranks above 4: 128 x 128 heads");
   constexpr int KD = K_, VD = V_;
   constexpr int WPH = step_wph<V_>();   // waves per value head
   constexpr int RW = VD / WPH;          // tile rows per wave
@@ -650,7 +654,7 @@ void gdn_step_kernel(lq_state st, lq_step_io io, lq_conv cv, int* dlist, const f
         lqf::flush_head4<128, 128, true>(lds.fl[0], st, Q0, slot, hv0 + (due & 1u ? 0 : 1), qm);
         if (due == 3u && threadIdx.x == 0) note_due(st.ctl, dlist, n * st.HV + hv0 + 1);   // a standalone flush finds it
       } else {
-        flush_due<K_, V_, G, G, G == 4 ? 2 : 1>(lds, st, Q0, slot, hv0, due, qm);
+        flush_due<K_, V_, G, G, G == 4 ? 2 : 1, RM>(lds, st, Q0, slot, hv0, due, qm);
       }
     }
   }
@@ -1264,9 +1268,18 @@ static int launch_decode(const lq_state* st, const lq_step_io* io, const lq_conv
   }
   return hipGetLastError() == hipSuccess ? LQ_OK : LQ_ERR_HIP;
 }
+// the same at ranks 5 to 8 (the rank ablation: GQA 2 and 4)
+template <bool CONV>
+static int launch_decode8(const lq_state* st, const lq_step_io* io, const lq_conv& cv, const float* Q0, hipStream_t s) {
+  const dim3 grid((unsigned)(io->N * st->H));
+  if (st->HV == 2 * st->H) gdn_step_kernel<128, 128, 2, CONV, true, 16><<<grid, 256, 0, s>>>(*st, *io, cv, nullptr, Q0);
+  else gdn_step_kernel<128, 128, 4, CONV, true, 16><<<grid, 512, 0, s>>>(*st, *io, cv, nullptr, Q0);
+  return hipGetLastError() == hipSuccess ? LQ_OK : LQ_ERR_HIP;
+}
 template <bool CONV>
 static int launch_decode_dims(const lq_state* st, const lq_step_io* io, const lq_conv& cv, const float* Q0,
                               hipStream_t s) {
+  if (st->R > 4) return launch_decode8<CONV>(st, io, cv, Q0, s);
   if (st->K == 128) return launch_decode<128, 128, CONV>(st, io, cv, Q0, s);
   return st->V == 128 ? launch_decode<64, 128, CONV>(st, io, cv, Q0, s) : launch_decode<64, 64, CONV>(st, io, cv, Q0, s);
 }
@@ -1278,7 +1291,7 @@ static int launch_decode_dims(const lq_state* st, const lq_step_io* io, const lq
 // step's four): 16.6 -> 14.3 us at 4 workgroups per CU, 20.9 -> 20.0 at 6, 25.2 -> 25.6 at 8, 35.7 -> 39.0 at 12.
 static bool one_launch(const lq_state* st, int N) {
   const int G = st->HV / st->H;
-  if (st->R > 4 || (G == 1 && st->H % 2 != 0)) return false;
+  if (G == 1 && (st->R > 4 || st->H % 2 != 0)) return false;
   if (G == 4 && st->V == 64) return (long long)N * st->H <= 6ll * lq_num_cus();
   return G == 1 || G == 2 || G == 4;
 }

@@ -79,6 +79,15 @@ def test_gdn_one_launch_equals_step_then_flush(K, V, GQA, L, R, qmax, heads):
     _check(g, lq, ssm, H, N, dict(R=R, qmax=qmax))
 
 
+@pytest.mark.parametrize("GQA,L,R", [(1, 16, 8), (2, 16, 8), (2, 33, 8), (2, 64, 8), (4, 16, 8), (4, 64, 8)])
+def test_rank8_one_launch_equals_step_then_flush(GQA, L, R):
+    g = torch.Generator(device=G.DEV)
+    g.manual_seed(GQA + L + R)
+    H, N = 3, 30
+    ssm, lq = _state(g, N + 4, H * GQA, H, 128, 128, L, R, 127.0)
+    _check(g, lq, ssm, H, N, dict(R=R))
+
+
 @pytest.mark.parametrize("L,R,glb", [(16, 4, 0.0), (33, 2, -5.0), (64, 4, 0.0), (1, 1, 0.0)])
 @pytest.mark.parametrize("HV,H,heads", [(3, 3, 100), (8, 4, 1100), (5, 5, 1100), (16, 16, 4200)])
 def test_kda_one_launch_equals_step_then_flush(HV, H, heads, L, R, glb):
