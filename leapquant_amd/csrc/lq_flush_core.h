@@ -794,7 +794,7 @@ __device__ __forceinline__ void load_code_words4(uint32_t wds[2][8], const int8_
     }
   }
 }
-// t += codes x svr[v] x skl[c], each term rounded to fp32 before the add after the window products:
+// t += codes x svr[v] x skl[c], each term rounded to fp32 before the add; added after the window products:
 // those are up to ~20x larger than their sum (they cancel), and an accumulator seeded with the checkpoint term rounds
 // them at a coarser step
 __device__ __forceinline__ void tile_add_words4(Tile4& t, const uint32_t wds[2][8], const float* svr,
