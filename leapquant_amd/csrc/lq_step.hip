@@ -167,6 +167,23 @@ __device__ __forceinline__ void flush_due(LDS& lds, const lq_state& st, const fl
 // RM: factors held per head.  4 (R <= 4): the G R <= 16 factor rows of the workgroup's heads are one MFMA tile, taken
 // by the last wave.  16 (the rank ablation R <= 16, K = V = 128; kernels.py:63, 457-469): up to G tiles, tile g taken
 // by the second wave of head g.
+// The row, and the unit in it, of a one-launch decode's workgroup: block b of `per` blocks a row.  Of the first `rot` rows
+// (rotated_rows; their number is in io.N, which is beside the first thing that a workgroup reads), each full round of 256
+// blocks (one per CU) takes its rows rotated by three more than the round before.  `per` a power of two: shifts and masks
+// (four divisions in their place cost config 1 0.6 us a call).
+constexpr int CUS = 256;
+struct RowUnit { int n, u; };
+__device__ __forceinline__ RowUnit decode_row(int b, int per, int rot) {
+  constexpr int SKEW = 3;
+  if ((per & (per - 1)) != 0 || per > CUS) {
+    const int n = b / per;
+    return {n, b - n * per};
+  }
+  const int s = __builtin_ctz(per), c = b / CUS, last = (CUS >> s) - 1;   // per = 2^s; the block's round; rows per round - 1
+  const int n = b >> s, m = (c + 1) * CUS <= rot * per ? (n & ~last) + ((n + SKEW * c) & last) : n;
+  return {m, b & (per - 1)};
+}
+
 // Steps the UW units of a workgroup, and returns the mask of its value heads whose window is now full (bit i: value head
 // hk0 G + i of the row), 0 for a padding row; `slot_` is the row's slot.
 template <int K_, int V_, int G, bool CONV, bool FL, int UW, int RM, bool DF, class LDS>
@@ -183,8 +200,8 @@ __device__ __forceinline__ unsigned gdn_step(LDS& lds, const lq_state& st, const
   constexpr bool NT = KD == 128;                  // non-temporal bulk loads (see ld_once)
   constexpr int NH = UW * G;                                // value heads of the workgroup
   const int H = st.H, HV = st.HV, L = st.L, R = st.R;
-  const int n = blockIdx.x / (H / UW);
-  const int hk0 = (blockIdx.x - n * (H / UW)) * UW;         // the workgroup's first key head
+  const RowUnit ru = FL ? decode_row(blockIdx.x, H / UW, io.N) : RowUnit{(int)blockIdx.x / H, (int)blockIdx.x % H};
+  const int n = ru.n, hk0 = ru.u * UW;                      // the row; the workgroup's first key head
   const int un = UW == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * WPH * G));   // this wave's unit
   const int hk = hk0 + un;
   StepShared<K_, V_, G, RM>& sh = lds.st[un];
@@ -212,7 +229,7 @@ __device__ __forceinline__ unsigned gdn_step(LDS& lds, const lq_state& st, const
       for (int g2 = 0; g2 < G; ++g2) pend |= (st.hcnt[(long long)slot0 * HV + hk * G + g2] >= L ? 1u : 0u) << g2;
       if (pend) {
         const float qm = code_range(st);
-#pragma unroll 1
+#pragma unroll
         for (int g2 = 0; g2 < G; ++g2)
           if ((pend >> g2) & 1u) lqf::flush_head4<128, 128, true>(lds.fl[0], st, Q0, slot0, hk * G + g2, qm);
       }
@@ -649,7 +666,8 @@ void gdn_step_kernel(lq_state st, lq_step_io io, lq_conv cv, int* dlist, const f
     if (due) {
       __syncthreads();          // the step is done with the shared bytes, and its appends are visible to the workgroup
       const float qm = code_range(st);
-      const int n = blockIdx.x / st.H, hv0 = (blockIdx.x - n * st.H) * G;
+      const RowUnit ru = decode_row(blockIdx.x, st.H, io.N);
+      const int n = ru.n, hv0 = ru.u * G;
       if constexpr (DF) {       // the first due head now, the other at the start of the next call
         lqf::flush_head4<128, 128, true>(lds.fl[0], st, Q0, slot, hv0 + (due & 1u ? 0 : 1), qm);
         if (due == 3u && threadIdx.x == 0) note_due(st.ctl, dlist, n * st.HV + hv0 + 1);   // a standalone flush finds it
@@ -669,7 +687,7 @@ void gdn_step_kernel(lq_state st, lq_step_io io, lq_conv cv, const float* Q0) {
   const unsigned due = gdn_step<K_, V_, 1, CONV, true, W, 4, false>(lds, st, io, cv, nullptr, Q0, slot);
   if (due) {
     __syncthreads();
-    const int n = blockIdx.x / (st.H / W), hv0 = (blockIdx.x - n * (st.H / W)) * W;
+    const int hv0 = decode_row(blockIdx.x, st.H / W, io.N).u * W;
     flush_due<K_, V_, 1, W, 1>(lds, st, Q0, slot, hv0, due, code_range(st));
   }
 }
@@ -680,7 +698,8 @@ __global__ __launch_bounds__(128 * W) __attribute__((amdgpu_waves_per_eu(4)))
 void gdn_step_kernel(lq_state st, lq_step_io io, lq_conv cv, const float* Q0) {
   static_assert(W == 2 * G && step_wph<V_>() == 2, "two step waves and two helpers per value head");
   __shared__ WideLds<K_, V_, G> lds;
-  const int n = blockIdx.x / st.H, hv0 = (blockIdx.x - n * st.H) * G;
+  const RowUnit ru = decode_row(blockIdx.x, st.H, io.N);
+  const int n = ru.n, hv0 = ru.u * G;
   int slot;
   unsigned due = 0;
   if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) < 2 * G) {
@@ -1223,6 +1242,24 @@ static int launch_gdn_dims(const lq_state* st, const lq_step_io* io, const lq_co
   return st->V == 128 ? launch_gdn<64, 128, CONV>(st, io, cv, dlist, s) : launch_gdn<64, 64, CONV>(st, io, cv, dlist, s);
 }
 
+// The dispatcher deals the blocks over the 256 CUs, so a CU's first four blocks are 256 apart: of rows 256 / per apart.  Rows
+// that were admitted one per call fill their windows L calls apart.  Where the two coincide -- at 16 blocks a row and the
+// default window of 16 -- the rows of a CU all flush in the same call, one CU with four flushes beside fifteen with none; the
+// same holds for rows one call apart where a flush is deferred by one.  There the rounds of 256 blocks take their rows
+// rotated by three more each: rows at different fills, W = 16, us per call, in order -> rotated: 61 rows with conv and
+// deferred flushes 31.7 -> 26.1, without conv 28.3 -> 22.9; 100 rows of 8 key heads 25.0 -> 21.0.  Elsewhere the rows stay in
+// order (64 such rows at W = 64 24.4 us in order, 24.8 rotated).
+static lq_step_io rotated_rows(const lq_state* st, const lq_step_io* io, int per, bool deferred = false) {
+  lq_step_io r = *io;
+  r.N = 0;                                            // the kernels' N: the rows that the rotation covers
+  if (per <= CUS && (per & (per - 1)) == 0)
+    for (int k = 1; k <= 3; ++k) {
+      const int d = k * (CUS / per) % st->L;
+      if (d == 0 || (deferred && (d == 1 || d == st->L - 1))) r.N = io->N;
+    }
+  return r;
+}
+
 // Small launches, up to four heads per CU, take the kernels with helper waves: their workgroups flush their heads side by
 // side, and all stay resident.  A flush call of one row (us, in turn -> side by side): two GQA 1 heads 21.6 -> 14.6, two of
 // a key head 21.6 -> 16.8, four 29.2 -> 25.4, two KDA heads 24.6 -> 15.2.  Window 16, us per call without -> with: GQA 1,
@@ -1234,17 +1271,19 @@ static bool helper_waves(const lq_state* st, int N) { return (long long)N * st->
 // the decode call in one launch: each workgroup flushes the heads whose window it fills
 template <int K_, int V_, bool CONV, int G>
 static void launch_wide(const lq_state* st, const lq_step_io* io, const lq_conv& cv, const float* Q0, hipStream_t s) {
-  gdn_step_kernel<K_, V_, 2 * G, CONV, G><<<dim3((unsigned)(io->N * st->H)), 256 * G, 0, s>>>(*st, *io, cv, Q0);
+  gdn_step_kernel<K_, V_, 2 * G, CONV, G><<<dim3((unsigned)(io->N * st->H)), 256 * G, 0, s>>>(
+      *st, rotated_rows(st, io, st->H), cv, Q0);
 }
 template <int K_, int V_, bool CONV>
 static int launch_decode(const lq_state* st, const lq_step_io* io, const lq_conv& cv, const float* Q0, hipStream_t s) {
   const int G = st->HV / st->H;
   const dim3 grid((unsigned)(io->N * (G == 1 ? st->H / 2 : st->H)));
   const bool wide = helper_waves(st, io->N);
+  const lq_step_io rio = rotated_rows(st, io, G == 1 ? st->H / 2 : st->H);
   switch (G) {
     case 1:
       if (wide) launch_wide<K_, V_, CONV, 1>(st, io, cv, Q0, s);
-      else gdn_step_kernel<K_, V_, 2, CONV><<<grid, 128 * step_wph<V_>(), 0, s>>>(*st, *io, cv, Q0);
+      else gdn_step_kernel<K_, V_, 2, CONV><<<grid, 128 * step_wph<V_>(), 0, s>>>(*st, rio, cv, Q0);
       break;
     case 2:
       if constexpr (V_ == 128) {
@@ -1253,7 +1292,7 @@ static int launch_decode(const lq_state* st, const lq_step_io* io, const lq_conv
           break;
         }
       }
-      gdn_step_kernel<K_, V_, 2, CONV, true><<<grid, 128 * step_wph<V_>(), 0, s>>>(*st, *io, cv, nullptr, Q0);
+      gdn_step_kernel<K_, V_, 2, CONV, true><<<grid, 128 * step_wph<V_>(), 0, s>>>(*st, rio, cv, nullptr, Q0);
       break;
     case 4:
       if constexpr (V_ == 128) {
@@ -1262,7 +1301,7 @@ static int launch_decode(const lq_state* st, const lq_step_io* io, const lq_conv
           break;
         }
       }
-      gdn_step_kernel<K_, V_, 4, CONV, true><<<grid, 256 * step_wph<V_>(), 0, s>>>(*st, *io, cv, nullptr, Q0);
+      gdn_step_kernel<K_, V_, 4, CONV, true><<<grid, 256 * step_wph<V_>(), 0, s>>>(*st, rio, cv, nullptr, Q0);
       break;
     default: return LQ_ERR_ARG;
   }
@@ -1272,8 +1311,9 @@ static int launch_decode(const lq_state* st, const lq_step_io* io, const lq_conv
 template <bool CONV>
 static int launch_decode8(const lq_state* st, const lq_step_io* io, const lq_conv& cv, const float* Q0, hipStream_t s) {
   const dim3 grid((unsigned)(io->N * st->H));
-  if (st->HV == 2 * st->H) gdn_step_kernel<128, 128, 2, CONV, true, 16><<<grid, 256, 0, s>>>(*st, *io, cv, nullptr, Q0);
-  else gdn_step_kernel<128, 128, 4, CONV, true, 16><<<grid, 512, 0, s>>>(*st, *io, cv, nullptr, Q0);
+  const lq_step_io rio = rotated_rows(st, io, st->H);
+  if (st->HV == 2 * st->H) gdn_step_kernel<128, 128, 2, CONV, true, 16><<<grid, 256, 0, s>>>(*st, rio, cv, nullptr, Q0);
+  else gdn_step_kernel<128, 128, 4, CONV, true, 16><<<grid, 512, 0, s>>>(*st, rio, cv, nullptr, Q0);
   return hipGetLastError() == hipSuccess ? LQ_OK : LQ_ERR_HIP;
 }
 template <bool CONV>
@@ -1344,11 +1384,16 @@ static int gdn_decode(const lq_state* st, const lq_step_io* io, const lq_conv* c
   if (deferred && st->K == 128 && st->V == 128 && st->HV == 2 * st->H && st->R <= 4) {
     const dim3 grid((unsigned)(io->N * st->H));
     const lq_conv none = {};
-    if (cv) gdn_step_kernel<128, 128, 2, true, true, 4, true><<<grid, 256, 0, s>>>(*st, *io, *cv, nullptr, Q0);
-    else gdn_step_kernel<128, 128, 2, false, true, 4, true><<<grid, 256, 0, s>>>(*st, *io, none, nullptr, Q0);
+    const lq_step_io rio = rotated_rows(st, io, st->H, true);
+      if (cv) gdn_step_kernel<128, 128, 2, true, true, 4, true><<<grid, 256, 0, s>>>(*st, rio, *cv, nullptr, Q0);
+    else gdn_step_kernel<128, 128, 2, false, true, 4, true><<<grid, 256, 0, s>>>(*st, rio, none, nullptr, Q0);
     return hipGetLastError() == hipSuccess ? LQ_OK : LQ_ERR_HIP;
   }
-  if (one_launch(st, io->N))
+  // a key head's four heads take two flushes in turn: a batch whose rows are due on different calls (which is what the
+  // deferred entry is for) flushes them sooner in a launch of their own, over all CUs (60 rows at different fills, W = 16:
+  // 50.0 us per call, in one launch 51.4)
+  const bool own_flush = deferred && st->HV == 4 * st->H && !helper_waves(st, io->N);
+  if (!own_flush && one_launch(st, io->N))
     return cv ? launch_decode_dims<true>(st, io, *cv, Q0, s) : launch_decode_dims<false>(st, io, lq_conv{}, Q0, s);
   rc = cv ? launch_gdn_dims<true>(st, io, *cv, nullptr, s) : lq_launch_step(st, io, 0, 0.f, nullptr, s);
   if (rc) return rc;

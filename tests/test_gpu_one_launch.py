@@ -96,3 +96,31 @@ def test_kda_one_launch_equals_step_then_flush(HV, H, heads, L, R, glb):
     N = heads // HV + 1
     ssm, lq = _state(g, N + 4, HV, H, 128, 128, L, R, 127.0, kda=True, glb=glb)
     _check(g, lq, ssm, H, N, dict(R=R, kda=True, gate_lower_bound=glb))
+
+
+def test_deferred_decode_of_a_large_batch():
+    """More than a round of 256 workgroups at a window whose rows are taken rotated: the deferred decode's outputs are the
+    immediate one's, and the states agree once the deferred heads are flushed."""
+    g = torch.Generator(device=G.DEV)
+    g.manual_seed(70)
+    NS, HV, H, L, N = 75, 8, 4, 16, 70
+    ssm, lq = _state(g, NS, HV, H, 128, 128, L, 4, 127.0)
+    lq.hcnt.copy_((torch.arange(NS, device=G.DEV) % L)[:, None].expand(NS, HV))
+    ssm2 = ssm.clone()
+    lq2 = G.LeapQuantState(ssm2, H, L=L, defer_flush=True)
+    for k in ("hcnt", "Wbuf", "Pbuf", "Kbuf", "Ubuf"):
+        getattr(lq2, k).copy_(getattr(lq, k))
+    idx = (torch.randperm(NS - 1, device=G.DEV, generator=g)[:N] + 1).int()
+    bf = lambda *s: torch.randn(*s, device=G.DEV, generator=g).bfloat16()
+    A_log, dt_bias = torch.zeros(HV, device=G.DEV), torch.zeros(HV, device=G.DEV)
+    for _ in range(4):
+        mixed, a, b = bf(N, 2 * H * 128 + HV * 128), bf(N, HV), bf(N, HV)
+        o1 = torch.empty(N, HV, 128, device=G.DEV, dtype=torch.bfloat16)
+        o2 = torch.empty_like(o1)
+        lq.decode(ssm, mixed, a, b, A_log, dt_bias, idx, o1)
+        lq2.decode(ssm2, mixed, a, b, A_log, dt_bias, idx, o2)
+        torch.cuda.synchronize()
+        assert torch.equal(o1, o2)
+    lq2.flush(ssm2, idx)
+    torch.cuda.synchronize()
+    assert torch.equal(ssm.view(torch.int32), ssm2.view(torch.int32)) and torch.equal(lq.hcnt, lq2.hcnt)
