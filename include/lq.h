@@ -109,10 +109,10 @@ int lq_gdn_step_conv(const lq_state* st, const lq_step_io* io, const lq_conv* cv
  * lq_gdn_step_conv), then the end-of-window flush of the heads whose window it filled (codes in [-qmax, qmax],
  * qmax = st->qmax, 0 meaning 127) -- what lq_gdn_step (or lq_gdn_step_conv) followed by lq_flush computes, in one
  * call.  Replaces make_gdn_step(...)(...) followed by make_flush(...)(...) as LeapQuantState.decode launches them
- * (/root/reference/leapquant/state.py:99-116; kernels.py:27-692, 1077-2033).  At R <= 4 it is one launch, in which each
- * workgroup flushes the heads it has just filled (or found full) on the same threads; ranks above 4, an odd H at
- * HV = H and large (64, 64) batches at HV = 4 H run the step and the flush as two launches.  Same limits as lq_gdn_step
- * and lq_flush. */
+ * (/root/reference/leapquant/state.py:99-116; kernels.py:27-692, 1077-2033).  It is one launch, in which each workgroup
+ * flushes the heads it has just filled (or found full) on the same threads; an odd H and ranks above 4 at HV = H, and large
+ * (64, 64) batches at HV = 4 H, run the step and the flush as two launches.  The heads of a key head that are not full
+ * share one fill, as their buffered keys do.  Same limits as lq_gdn_step and lq_flush. */
 int lq_gdn_decode(const lq_state* st, const lq_step_io* io, const lq_conv* cv, const float* Q0, void* stream);
 
 /* lq_gdn_decode with the flush of a key head's second value head deferred: no counterpart in the reference (whose

@@ -186,9 +186,13 @@ __device__ __forceinline__ RowUnit decode_row(int b, int per, int rot) {
 
 // Steps the UW units of a workgroup, and returns the mask of its value heads whose window is now full (bit i: value head
 // hk0 G + i of the row), 0 for a padding row; `slot_` is the row's slot.
-template <int K_, int V_, int G, bool CONV, bool FL, int UW, int RM, bool DF, class LDS>
+// KSH: the key head's value heads are 2^KSH units of G, each a workgroup of its own (FL only).  Each unit with a head to
+// step appends the key, the same bytes to the same row (the heads of a key head that are not full share one fill), so that
+// its own flush finds it whatever the other's workgroup has written.
+template <int K_, int V_, int G, bool CONV, bool FL, int UW, int RM, bool DF, int KSH = 0, class LDS>
 __device__ __forceinline__ unsigned gdn_step(LDS& lds, const lq_state& st, const lq_step_io& io, const lq_conv& cv,
                                              int* dlist, const float* Q0, int& slot_) {
+  static_assert(KSH == 0 || (FL && !CONV && UW == 1), "split key heads: the one-launch decode without conv");
   static_assert(!DF || FL, "deferred flush (lq_gdn_decode_deferred): the fused decode kernel");
   static_assert(!DF || (K_ == 128 && V_ == 128 && G == 2), "deferred flush: 128 x 128 heads, two per key head");
   static_assert(RM == 4 || (RM == 16 && K_ == 128 && V_ == 128 && !DF), "ranks above 4: 128 x 128 heads");
@@ -200,10 +204,10 @@ __device__ __forceinline__ unsigned gdn_step(LDS& lds, const lq_state& st, const
   constexpr bool NT = KD == 128;                  // non-temporal bulk loads (see ld_once)
   constexpr int NH = UW * G;                                // value heads of the workgroup
   const int H = st.H, HV = st.HV, L = st.L, R = st.R;
-  const RowUnit ru = FL ? decode_row(blockIdx.x, H / UW, io.N) : RowUnit{(int)blockIdx.x / H, (int)blockIdx.x % H};
-  const int n = ru.n, hk0 = ru.u * UW;                      // the row; the workgroup's first key head
+  const RowUnit ru = FL ? decode_row(blockIdx.x, (H << KSH) / UW, io.N) : RowUnit{(int)blockIdx.x / H, (int)blockIdx.x % H};
+  const int n = ru.n, hk0 = ru.u * UW;                      // the row; the workgroup's first unit (KSH = 0: key head)
   const int un = UW == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * WPH * G));   // this wave's unit
-  const int hk = hk0 + un;
+  const int hk = hk0 + un, hkey = hk >> KSH;                // this wave's unit and its key head
   StepShared<K_, V_, G, RM>& sh = lds.st[un];
   const int tid = UW == 1 ? threadIdx.x : threadIdx.x % (64 * WPH * G);   // thread in the unit
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave in the unit
@@ -243,8 +247,8 @@ __device__ __forceinline__ unsigned gdn_step(LDS& lds, const lq_state& st, const
 #pragma unroll
     for (int e = 0; e < NE; ++e) {
       const int c = lane + 64 * e;
-      kxr[e] = mrow[H * KD + hk * KD + c];
-      qxr[e] = mrow[hk * KD + c];
+      kxr[e] = mrow[H * KD + hkey * KD + c];
+      qxr[e] = mrow[hkey * KD + c];
     }
   }
   const bf16_t araw = ((const bf16_t*)io.a)[(long long)n * HV + hv];
@@ -385,8 +389,9 @@ __device__ __forceinline__ unsigned gdn_step(LDS& lds, const lq_state& st, const
           sh.hkq[2 * v2][c] = fh;
           sh.hkq[2 * v2 + 1][c] = f2h(xs64 - h2f(fh));
         }
-        kapp[e] = f2bf(kn[e]);
+        if (KSH == 0) kapp[e] = f2bf(kn[e]);
       }
+      if (KSH > 0) kapp[e] = f2bf(kn[e]);
       if constexpr (!GL) wjv[e] = wx[e] * alpha;   // w_j = Wbuf[j] alpha (kernels.py:270-274), written back at the end
     }
     if (lane == 0) {
@@ -449,7 +454,7 @@ __device__ __forceinline__ unsigned gdn_step(LDS& lds, const lq_state& st, const
   constexpr int KT = (4 + NWV - 1) / NWV;                   // 16-row key tiles per wave (64 rows over the waves)
   bf16x8 kfr[KT][KS32];
   {
-    const bf16_t* Kb = (const bf16_t*)st.Kbuf + ((long long)slot * H + hk) * L * KD;
+    const bf16_t* Kb = (const bf16_t*)st.Kbuf + ((long long)slot * H + hkey) * L * KD;
 #pragma unroll
     for (int t = 0; t < KT; ++t) {
       const int j = 16 * (wv + NWV * t) + n16;
@@ -632,10 +637,16 @@ __device__ __forceinline__ unsigned gdn_step(LDS& lds, const lq_state& st, const
     if (!FL && h + 1 == L) note_due(st.ctl, dlist, n * HV + hv);   // this head is due: the flush that follows takes it
   }
   if (wi == 0) {
+    bool appends = g == 0;
+    if constexpr (KSH > 0) {    // the unit's first head that is not full
+      appends = true;
+#pragma unroll
+      for (int g2 = 0; g2 < G; ++g2) appends = appends && (g2 >= g || hg[g2] >= L);
+    }
 #pragma unroll
     for (int e = 0; e < NE; ++e) {
       const int c = lane + 64 * e;
-      if (g == 0) ((bf16_t*)st.Kbuf)[(((long long)slot * H + hk) * L + h) * KD + c] = kapp[e];   // key append
+      if (appends) ((bf16_t*)st.Kbuf)[(((long long)slot * H + hkey) * L + h) * KD + c] = kapp[e];   // key append
       if (!GL && c < h) Wp[c] = wjv[e];
     }
   }
@@ -689,6 +700,18 @@ void gdn_step_kernel(lq_state st, lq_step_io io, lq_conv cv, const float* Q0) {
     __syncthreads();
     const int hv0 = decode_row(blockIdx.x, st.H / W, io.N).u * W;
     flush_due<K_, V_, 1, W, 1>(lds, st, Q0, slot, hv0, due, code_range(st));
+  }
+}
+// the one-launch decode at GQA 4: G = 2 value heads per workgroup, 2^KSH workgroups per key head
+template <int K_, int V_, int G, int KSH>
+__global__ __launch_bounds__(64 * step_wph<V_>() * G) __attribute__((amdgpu_waves_per_eu(4)))
+void gdn_step_kernel(lq_state st, lq_step_io io, const float* Q0) {
+  __shared__ StepLds<K_, V_, G, true, 4> lds;
+  int slot;
+  const unsigned due = gdn_step<K_, V_, G, false, true, 1, 4, false, KSH>(lds, st, io, lq_conv{}, nullptr, Q0, slot);
+  if (due) {
+    __syncthreads();
+    flush_due<K_, V_, G, G, 1>(lds, st, Q0, slot, decode_row(blockIdx.x, st.H << KSH, io.N).u * G, due, code_range(st));
   }
 }
 // the one-launch decode with helper waves: one key head per workgroup, G value heads, 256 G = 128 W threads.  The waves
@@ -1301,7 +1324,8 @@ static int launch_decode(const lq_state* st, const lq_step_io* io, const lq_conv
           break;
         }
       }
-      gdn_step_kernel<K_, V_, 4, CONV, true><<<grid, 256 * step_wph<V_>(), 0, s>>>(*st, rio, cv, nullptr, Q0);
+      if constexpr (CONV) gdn_step_kernel<K_, V_, 4, true, true><<<grid, 256 * step_wph<V_>(), 0, s>>>(*st, rio, cv, nullptr, Q0);
+      else gdn_step_kernel<K_, V_, 2, 1><<<dim3(2u * grid.x), 128 * step_wph<V_>(), 0, s>>>(*st, rotated_rows(st, io, 2 * st->H), Q0);
       break;
     default: return LQ_ERR_ARG;
   }
@@ -1324,15 +1348,19 @@ static int launch_decode_dims(const lq_state* st, const lq_step_io* io, const lq
   return st->V == 128 ? launch_decode<64, 128, CONV>(st, io, cv, Q0, s) : launch_decode<64, 64, CONV>(st, io, cv, Q0, s);
 }
 // Which calls take one launch.  The second launch, the flush, costs a call ~2 us also when nothing is due.  Window 16,
-// us per call, two launches -> one: 128 x 128 at GQA 4, B = 24, 16 key heads 16.5 -> 14.8, B = 200 78.2 -> 75.4; at GQA 1,
-// B = 64, 32 heads 21.0 -> 16.4, B = 200 45.8 -> 41.7; (64, 128) at GQA 2, B = 64 13.0 -> 10.5; (64, 64) at GQA 1,
+// us per call, two launches -> one: 128 x 128 at GQA 4, B = 24, 16 key heads 16.5 -> 12.5, B = 200 78.2 -> 71.8; at GQA 1,
+// B = 64, 32 heads 21.0 -> 16.4, B = 200 45.8 -> 41.7; (64, 128) at GQA 2, B = 64 13.0 -> 10.4; (64, 64) at GQA 1,
 // B = 64 10.9 -> 8.5.  GQA 1 pairs two key heads of a row in a workgroup, so an odd H takes two launches.  So do large
-// (64, 64) batches at GQA 4, whose flush needs twice the step's LDS and registers (two workgroups per CU against the
-// step's four): 16.6 -> 14.3 us at 4 workgroups per CU, 20.9 -> 20.0 at 6, 25.2 -> 25.6 at 8, 35.7 -> 39.0 at 12.
-static bool one_launch(const lq_state* st, int N) {
+// (64, 64) batches at GQA 4, whose flush needs more LDS and registers than the step: us per call at 8 rows x H per CU 25.2 ->
+// 23.7, at 10 29.8 -> 29.0, at 12.5 35.7 -> 35.1 in two launches, 37.4 in one.  With the conv a key head's four value heads
+// stay in one workgroup (they share its conv state), 16.6 -> 14.3 at 4, 20.9 -> 20.0 at 6, 25.2 -> 25.6 at 8; and its V = 128
+// heads take two flushes in turn, so that a batch whose rows are due on different calls (which is what the deferred entry is
+// for) flushes them sooner in a launch of its own, over all CUs: 24 rows 38.8 us per call, in one launch 43.2.
+static bool one_launch(const lq_state* st, int N, bool conv, bool deferred) {
   const int G = st->HV / st->H;
   if (G == 1 && (st->R > 4 || st->H % 2 != 0)) return false;
-  if (G == 4 && st->V == 64) return (long long)N * st->H <= 6ll * lq_num_cus();
+  if (G == 4 && conv && deferred && st->V == 128 && !helper_waves(st, N)) return false;
+  if (G == 4 && st->V == 64) return (long long)N * st->H <= (conv ? 6ll : 10ll) * lq_num_cus();
   return G == 1 || G == 2 || G == 4;
 }
 
@@ -1389,11 +1417,7 @@ static int gdn_decode(const lq_state* st, const lq_step_io* io, const lq_conv* c
     else gdn_step_kernel<128, 128, 2, false, true, 4, true><<<grid, 256, 0, s>>>(*st, rio, none, nullptr, Q0);
     return hipGetLastError() == hipSuccess ? LQ_OK : LQ_ERR_HIP;
   }
-  // a key head's four heads take two flushes in turn: a batch whose rows are due on different calls (which is what the
-  // deferred entry is for) flushes them sooner in a launch of their own, over all CUs (60 rows at different fills, W = 16:
-  // 50.0 us per call, in one launch 51.4)
-  const bool own_flush = deferred && st->HV == 4 * st->H && !helper_waves(st, io->N);
-  if (!own_flush && one_launch(st, io->N))
+  if (one_launch(st, io->N, cv != nullptr, deferred))
     return cv ? launch_decode_dims<true>(st, io, *cv, Q0, s) : launch_decode_dims<false>(st, io, lq_conv{}, Q0, s);
   rc = cv ? launch_gdn_dims<true>(st, io, *cv, nullptr, s) : lq_launch_step(st, io, 0, 0.f, nullptr, s);
   if (rc) return rc;

@@ -175,7 +175,7 @@ class LeapQuantState:
         if self.kda:                 # step + flush of the heads it fills (one launch for small batches)
             _lib.check(L.lq_kda_decode(ctypes.byref(st), ctypes.byref(io), self.glb, dev(self.Q0), stream),
                        "lq_kda_decode")
-        else:                        # step + flush of the heads it fills (one launch at ranks up to 4)
+        else:                        # step + flush of the heads it fills (one launch)
             fn = L.lq_gdn_decode_deferred if self.defer_flush else L.lq_gdn_decode
             _lib.check(fn(ctypes.byref(st), ctypes.byref(io), None, dev(self.Q0), stream), "lq_gdn_decode")
 

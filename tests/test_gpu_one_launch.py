@@ -15,11 +15,17 @@ def _state(g, NS, HV, H, K, V, L, R, qmax, kda=False, glb=0.0):
     ssm = torch.zeros(NS, HV, V, K, device=G.DEV).normal_(0.0, 0.02, generator=g)
     lq = G.LeapQuantState(ssm, H, kda=kda, gate_lower_bound=glb, L=L, R=R, qmax=qmax)
     lq.quantize(ssm, torch.arange(1, NS, device=G.DEV))
-    # fills: slot 1 all heads L - 1, slot 2 all full but one, slot 3 none due, the others any mix per head
-    fill = torch.randint(max(0, L - 3), L + 1, (NS, HV), generator=g, device=G.DEV, dtype=torch.int32)
+    # fills: slot 1 all heads L - 1, slot 2 all full but one, slot 3 none due, the others any mix over the key heads, with
+    # some heads full (the heads of a key head that are not full share one fill, as their buffered keys do; at GQA 4 a key
+    # head's heads, which two workgroups step, are full together: a key appended under a full head is the next one's)
+    fill = torch.randint(max(0, L - 3), L, (NS, H, 1), generator=g, device=G.DEV).expand(NS, H, HV // H).reshape(NS, HV)
+    full = torch.rand(NS, HV, device=G.DEV, generator=g) < 0.25
+    if HV // H == 4:
+        full = full.view(NS, H, 4)[:, :, :1].expand(NS, H, 4).reshape(NS, HV)
+    fill = torch.where(full, L, fill).int()
     fill[1] = L - 1
     fill[2] = L
-    fill[2, HV - 1] = max(0, L - 2)
+    fill[2, HV - HV // H:] = max(0, L - 2)
     fill[3] = max(0, L - 2)
     lq.hcnt.copy_(fill)
     j = torch.arange(L, device=G.DEV)
