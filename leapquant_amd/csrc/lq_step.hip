@@ -12,6 +12,7 @@
 //     key operands and the window's decayed keys formed by a backward scan split between the two waves.
 #include "lq_flush64_core.h"
 #include "lq_flush8_core.h"
+#include "lq_rules.h"
 
 namespace {
 
@@ -1164,7 +1165,8 @@ __device__ __forceinline__ void kda_step(KdaShared* units, const lq_state& st, c
   } else {
   out[lt] = f2bf(y);
   ((bf16_t*)st.Ubuf)[(sh_ * L + h) * VD + lt] = f2bf(u);
-  if (hv % G == 0) ((bf16_t*)st.Kbuf)[(((long long)slot * H + hk) * L + h) * KD + lt] = sh.bkq[0][lt];   // bf16(kn)
+  // key append, bf16(kn): once per key head, whose value heads FL keeps in one workgroup (lq_kda_decode_heads)
+  if (hv % G == 0) ((bf16_t*)st.Kbuf)[(((long long)slot * H + hk) * L + h) * KD + lt] = sh.bkq[0][lt];
   if (lt == 0) {
     st.Wbuf[sh_ * L + h] = 1.0f;
     st.hcnt[sh_] = h + 1;
@@ -1289,7 +1291,7 @@ static lq_step_io rotated_rows(const lq_state* st, const lq_step_io* io, int per
 // 16 heads, B = 16 7.5 -> 6.5, B = 64 (4 heads per CU) 9.7 -> 9.6; GQA 2, B = 16 (2) 7.4 -> 7.3, B = 64 (8) 15.3 -> 17.4;
 // GQA 4, B = 16 (4) 9.4 -> 9.2, B = 32 (8) 15.7 -> 17.7; KDA, 32 heads, B = 1 8.2 -> 6.9, B = 32 (4) 13.0 -> 11.9,
 // B = 48 (6) 16.7 -> 18.6.
-static bool helper_waves(const lq_state* st, int N) { return (long long)N * st->HV <= 4ll * lq_num_cus(); }
+static bool helper_waves(const lq_state* st, int N) { return lq_helper_waves(N, st->HV, lq_num_cus()); }
 
 // the decode call in one launch: each workgroup flushes the heads whose window it fills
 template <int K_, int V_, bool CONV, int G>
@@ -1449,21 +1451,15 @@ extern "C" int lq_kda_decode(const lq_state* st, const lq_step_io* io, float glb
   if ((rc = lq_check_flush(st, Q0, io->idx, io->N, 1, qmax))) return rc;
   if (io->N == 0) return LQ_OK;
   hipStream_t s = (hipStream_t)stream;
-  const long long heads = (long long)io->N * st->HV;
-  if (helper_waves(st, io->N)) {
-    flush4_kernel<1><<<dim3((unsigned)heads), 256, 0, s>>>(*st, *io, glb, Q0);
-    return hipGetLastError() == hipSuccess ? LQ_OK : LQ_ERR_HIP;
+  const unsigned heads = (unsigned)io->N * (unsigned)st->HV;
+  switch (lq_kda_decode_heads(io->N, st->HV, st->H, st->L, lq_num_cus())) {
+    case 1: flush4_kernel<1><<<dim3(heads), 256, 0, s>>>(*st, *io, glb, Q0); break;
+    case 2: flush4_kernel<2><<<dim3(heads / 2), 256, 0, s>>>(*st, *io, glb, Q0); break;
+    default:
+      if ((rc = lq_launch_step(st, io, 1, glb, nullptr, s))) return rc;
+      return lq_launch_flush(st, Q0, io->idx, io->N, 1, qmax, nullptr, s);
   }
-  // One launch, two heads per workgroup, up to one round of workgroups (eight heads per CU), and for windows of one chunk
-  // below two: us per call, two launches -> one, 32 heads, W = 16: B = 48 18.6 -> 16.7, B = 64 21.7 -> 20.0, B = 96 27.9
-  // -> 27.3, B = 120 32.7 -> 31.7; W = 64, whose units also meet at each chunk's barriers: B = 48 21.9 -> 21.4, B = 64
-  // 25.6 -> 25.7, B = 96 33.9 -> 35.1.  An odd HV takes two.
-  if (st->HV % 2 == 0 && (heads <= 8ll * lq_num_cus() || (st->L <= KCH && heads < 16ll * lq_num_cus()))) {
-    flush4_kernel<2><<<dim3((unsigned)(heads / 2)), 256, 0, s>>>(*st, *io, glb, Q0);
-    return hipGetLastError() == hipSuccess ? LQ_OK : LQ_ERR_HIP;
-  }
-  if ((rc = lq_launch_step(st, io, 1, glb, nullptr, s))) return rc;
-  return lq_launch_flush(st, Q0, io->idx, io->N, 1, qmax, nullptr, s);
+  return hipGetLastError() == hipSuccess ? LQ_OK : LQ_ERR_HIP;
 }
 
 extern "C" int lq_abi_version(void) { return LQ_ABI_VERSION; }

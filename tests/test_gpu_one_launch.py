@@ -95,7 +95,9 @@ def test_rank8_one_launch_equals_step_then_flush(GQA, L, R):
 
 
 @pytest.mark.parametrize("L,R,glb", [(16, 4, 0.0), (33, 2, -5.0), (64, 4, 0.0), (1, 1, 0.0)])
-@pytest.mark.parametrize("HV,H,heads", [(3, 3, 100), (8, 4, 1100), (5, 5, 1100), (16, 16, 4200)])
+@pytest.mark.parametrize("HV,H,heads", [(3, 3, 100), (8, 4, 1100), (5, 5, 1100), (16, 16, 4200),
+                                        # value heads sharing a key head, on both sides of four heads per CU
+                                        (8, 4, 100), (6, 2, 100), (6, 2, 1100), (8, 2, 100), (8, 2, 1100)])
 def test_kda_one_launch_equals_step_then_flush(HV, H, heads, L, R, glb):
     g = torch.Generator(device=G.DEV)
     g.manual_seed(HV + L + heads)
