@@ -15,7 +15,12 @@
  *        Wbuf f32  [NS][HV][L]     entry weights w_j (GDN: gate products since the entry; KDA: 1)
  *        Pbuf f32  [NS][HV][KA]    GDN (KA = 1): decay of the checkpoint, init 1;  KDA (KA = K): cumulative log-gate, init 0
  *        Gbuf fp16 [NS][HV][L][K]  KDA only: per-entry step decay exp(g_j), init 1
- *        hcnt i32  [NS][HV]        valid entries in the window
+ *        hcnt i32  [NS][HV]        valid entries in the window.  The value heads of a key head share one fill, as they share
+ *                                  their buffered keys: every entry point keeps it so (a head that a deferred decode left
+ *                                  full is flushed before its slot is stepped again), and a caller that writes hcnt
+ *                                  itself keeps it too.  With other fills in one key head the results are undefined where
+ *                                  its value heads are stepped by several workgroups (KDA; GDN at HV = 4 H): one head's
+ *                                  key is appended over a row that another head is reading.
  *   A row n of a call with idx[n] <= 0 is a padding row: its outputs are zero and no state is written.  A slot
  *   idx[n] >= NS (outside the cache) is treated the same way, so no index reaches memory outside the tensors.
  */
@@ -111,8 +116,7 @@ int lq_gdn_step_conv(const lq_state* st, const lq_step_io* io, const lq_conv* cv
  * call.  Replaces make_gdn_step(...)(...) followed by make_flush(...)(...) as LeapQuantState.decode launches them
  * (/root/reference/leapquant/state.py:99-116; kernels.py:27-692, 1077-2033).  It is one launch, in which each workgroup
  * flushes the heads it has just filled (or found full) on the same threads; an odd H and ranks above 4 at HV = H, and large
- * (64, 64) batches at HV = 4 H, run the step and the flush as two launches.  The heads of a key head that are not full
- * share one fill, as their buffered keys do.  Same limits as lq_gdn_step and lq_flush. */
+ * (64, 64) batches at HV = 4 H, run the step and the flush as two launches.  Same limits as lq_gdn_step and lq_flush. */
 int lq_gdn_decode(const lq_state* st, const lq_step_io* io, const lq_conv* cv, const float* Q0, void* stream);
 
 /* lq_gdn_decode with the flush of a key head's second value head deferred: no counterpart in the reference (whose

@@ -16,12 +16,13 @@ def _state(g, NS, HV, H, K, V, L, R, qmax, kda=False, glb=0.0):
     lq = G.LeapQuantState(ssm, H, kda=kda, gate_lower_bound=glb, L=L, R=R, qmax=qmax)
     lq.quantize(ssm, torch.arange(1, NS, device=G.DEV))
     # fills: slot 1 all heads L - 1, slot 2 all full but one, slot 3 none due, the others any mix over the key heads, with
-    # some heads full (the heads of a key head that are not full share one fill, as their buffered keys do; at GQA 4 a key
-    # head's heads, which two workgroups step, are full together: a key appended under a full head is the next one's)
+    # some heads full.  The value heads of a key head share one fill, as their buffered keys do (include/lq.h); full heads
+    # beside others only where one workgroup steps the whole key head, on both sides of the comparison (GDN at GQA 1 and
+    # 2): elsewhere a head appends over a row that another one, with another fill after the first call, is reading
     fill = torch.randint(max(0, L - 3), L, (NS, H, 1), generator=g, device=G.DEV).expand(NS, H, HV // H).reshape(NS, HV)
     full = torch.rand(NS, HV, device=G.DEV, generator=g) < 0.25
-    if HV // H == 4:
-        full = full.view(NS, H, 4)[:, :, :1].expand(NS, H, 4).reshape(NS, HV)
+    if HV // H == 4 or (kda and HV > H):
+        full = full.view(NS, H, HV // H)[:, :, :1].expand(NS, H, HV // H).reshape(NS, HV)
     fill = torch.where(full, L, fill).int()
     fill[1] = L - 1
     fill[2] = L
