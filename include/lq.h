@@ -31,7 +31,7 @@
 extern "C" {
 #endif
 
-#define LQ_ABI_VERSION 5
+#define LQ_ABI_VERSION 6
 #define LQ_SCHED_INTS 512   /* ints of lq_state.sched: eight counters, 256 bytes apart */
 
 enum lq_status {
@@ -72,12 +72,14 @@ typedef struct lq_step_io {
   const void* mixed;      /* bf16 [N][2*H*K + HV*V]: q (key heads) | k (key heads) | v (value heads), after the conv */
   const void* a;          /* bf16 raw gate: GDN [N][HV]; KDA [N][HV][K] */
   const void* b;          /* bf16 [N][HV]: beta = sigmoid(b) */
-  const float* A_log;     /* [HV] */
-  const float* dt_bias;   /* GDN [HV]; KDA [HV][K] */
+  const void* A_log;      /* [HV], fp32 or bf16 (gate_bf16) */
+  const void* dt_bias;    /* GDN [HV]; KDA [HV][K], fp32 or bf16 (gate_bf16) */
   const int* idx;         /* [N] state slot of each row; <= 0: padding row */
   void* out;              /* bf16 [N][HV][V] */
   int N;
   float scale;            /* query scale (K^-1/2 by default) */
+  int gate_bf16;          /* dtype of the gate parameters: bit 0 set, A_log holds bf16; bit 1 set, dt_bias does (2-byte
+                             aligned, read by the aligned 32-bit words that hold its elements); else fp32 */
 } lq_step_io;
 
 /* Depthwise causal conv1d update (vLLM's causal_conv1d_update) fused into the GDN step: the step reads the raw
@@ -208,7 +210,8 @@ int lq_conv_update(const lq_conv* cv, const void* x, void* out, const int* idx, 
 
 /* Baseline for the measurements (no reference counterpart): the same GDN decode step on a dense state S
  * [NS][HV][V][K] stored as bf16 (state_dtype 0) or fp32 (state_dtype 1), updated in place:
- * S' = alpha S + u k^T, u = beta (v - alpha S k), o = S' q.  S and io->mixed 16-byte aligned. */
+ * S' = alpha S + u k^T, u = beta (v - alpha S k), o = S' q.  S and io->mixed 16-byte aligned, fp32 gate
+ * parameters. */
 int lq_dense_step(void* S, int state_dtype, int NS, int HV, int H, int K, int V, const lq_step_io* io, void* stream);
 
 #ifdef __cplusplus

@@ -5,7 +5,7 @@ import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "_build", "liblq.so")
-ABI_VERSION = 5
+ABI_VERSION = 6
 SCHED_INTS = 512           # include/lq.h: LQ_SCHED_INTS
 
 c_void_p, c_int, c_float, c_ll = ctypes.c_void_p, ctypes.c_int, ctypes.c_float, ctypes.c_longlong
@@ -20,7 +20,7 @@ class LqState(ctypes.Structure):
 
 class LqStepIO(ctypes.Structure):
     _fields_ = [("mixed", c_void_p), ("a", c_void_p), ("b", c_void_p), ("A_log", c_void_p), ("dt_bias", c_void_p),
-                ("idx", c_void_p), ("out", c_void_p), ("N", c_int), ("scale", c_float)]
+                ("idx", c_void_p), ("out", c_void_p), ("N", c_int), ("scale", c_float), ("gate_bf16", c_int)]
 
 
 class LqConv(ctypes.Structure):

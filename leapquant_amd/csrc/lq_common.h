@@ -250,6 +250,17 @@ __attribute__((visibility("hidden"))) int lq_launch_kda_dequant4(const lq_state*
 // decode step of every row of io (GDN or KDA), due heads signalled through dlist when it is set (else st->ctl)
 __attribute__((visibility("hidden"))) int lq_launch_step(const lq_state* st, const lq_step_io* io, int kda, float glb,
                                                          int* dlist, hipStream_t s);
+// the launches of the steps and decode calls (arguments checked by their entry points), for gate parameters in fp32
+// (lq_step.hip) and where one is in bf16 (lq_step_bf16.hip)
+#define LQ_STEP_LAUNCHES(name)                                                                                              \
+  __attribute__((visibility("hidden"))) int name##_step(const lq_state* st, const lq_step_io* io, const lq_conv* cv,       \
+                                                        int kda, float glb, int* dlist, hipStream_t s);                    \
+  __attribute__((visibility("hidden"))) int name##_gdn_decode(const lq_state* st, const lq_step_io* io, const lq_conv* cv, \
+                                                              const float* Q0, bool deferred, hipStream_t s);              \
+  __attribute__((visibility("hidden"))) int name##_kda_decode(const lq_state* st, const lq_step_io* io, float glb,         \
+                                                              const float* Q0, hipStream_t s);
+LQ_STEP_LAUNCHES(lq_f32)
+LQ_STEP_LAUNCHES(lq_bf16)
 // flush of the due heads: the listed ones when dlist is set (the list is then reset), else found by the scan
 __attribute__((visibility("hidden"))) int lq_launch_flush(const lq_state* st, const float* Q0, const int* idx, int N,
                                                           int kda, float qmax, int* dlist, hipStream_t s);

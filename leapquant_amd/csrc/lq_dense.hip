@@ -54,7 +54,8 @@ void dense_step_kernel(void* S, int NS, int HV, int H, lq_step_io io) {
       kv[2 * z] = bf_lo(kw[z]); kv[2 * z + 1] = bf_hi(kw[z]);
     }
   }
-  const float alpha = gdn_alpha(bf2f(((const bf16_t*)io.a)[(long long)n * HV + hv]), io.dt_bias[hv], io.A_log[hv]);
+  const float alpha = gdn_alpha(bf2f(((const bf16_t*)io.a)[(long long)n * HV + hv]), ((const float*)io.dt_bias)[hv],
+                                ((const float*)io.A_log)[hv]);
   const float beta = beta_of(bf2f(((const bf16_t*)io.b)[(long long)n * HV + hv]));
   float nq = 0.f, nk = 0.f, nkq = 0.f;
 #pragma unroll
@@ -153,7 +154,7 @@ __global__ __launch_bounds__(256) void conv_update_kernel(lq_conv cv, const bf16
 extern "C" int lq_dense_step(void* S, int state_dtype, int NS, int HV, int H, int K, int V, const lq_step_io* io,
                              void* stream) {
   if (!S || !io || K != KD || V != VD || H <= 0 || HV <= 0 || HV % H != 0 || NS <= 0 || io->N < 0) return LQ_ERR_ARG;
-  if (state_dtype != 0 && state_dtype != 1) return LQ_ERR_ARG;
+  if ((state_dtype != 0 && state_dtype != 1) || io->gate_bf16) return LQ_ERR_ARG;
   if (io->N == 0) return LQ_OK;
   // q, k and the state rows are read by 16-byte loads: 16-byte aligned bases (the rows are multiples of 16 bytes)
   if (((uintptr_t)S & 15) || ((uintptr_t)io->mixed & 15)) return LQ_ERR_ARG;

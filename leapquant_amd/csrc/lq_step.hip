@@ -14,6 +14,16 @@
 #include "lq_flush8_core.h"
 #include "lq_rules.h"
 
+// 0: the kernels for gate parameters in fp32, and the entry points; 1 (lq_step_bf16.hip): the kernels where one is in bf16
+#ifndef LQ_GATE_BF16
+#define LQ_GATE_BF16 0
+#endif
+#if LQ_GATE_BF16
+#define LQ_LAUNCH(name) lq_bf16_##name
+#else
+#define LQ_LAUNCH(name) lq_f32_##name
+#endif
+
 namespace {
 
 constexpr int KD = 128;   // key dim
@@ -54,6 +64,41 @@ __device__ __forceinline__ T ld_nt(const T* p) {
   else return *p;
 }
 constexpr float KSPLIT = 64.0f;   // kn / qn scaled by 2^6 before the fp16 hi / lo split (keeps the lo part normal)
+
+// lq_step_io as the kernels take it: `rows` counts the rows that the row rotation covers (rotated_rows); with gate
+// parameters in bf16, its top bits say which of the two are.
+struct StepIo {
+  const void *mixed, *a, *b, *A_log, *dt_bias;
+  const int* idx;
+  void* out;
+  int rows;
+  float scale;
+  __device__ __forceinline__ int rotated() const { return LQ_GATE_BF16 ? rows & 0x3fffffff : rows; }
+};
+StepIo step_io(const lq_step_io* io, int rotated = 0) {
+  return {io->mixed, io->a, io->b, io->A_log, io->dt_bias, io->idx, io->out,
+          (int)((unsigned)rotated | (LQ_GATE_BF16 ? (unsigned)io->gate_bf16 << 30 : 0u)), io->scale};
+}
+// Element i of a gate parameter in its own dtype, so that no converted copy of it has to be made or kept (a copy made on
+// each call is a launch: 1.7 us of a 15 us call).  The 32-bit word that holds the element is loaded where the other small
+// loads are, its value taken where it is used.  The bf16 form costs a fp32 call 0.5 to 1%, hence the second set of
+// kernels (LQ_GATE_BF16): of a bf16 tensor that starts or ends inside a word, the word's other half is not used.
+struct GateWord {
+  uint32_t w;
+  unsigned half;            // 0: an fp32 word; 1, 2: its lower, upper half
+  __device__ __forceinline__ float value() const {
+    if (!LQ_GATE_BF16) return __uint_as_float(w);
+    return __uint_as_float(half == 0 ? w : half == 1 ? w << 16 : w & 0xffff0000u);
+  }
+};
+enum { GATE_A_LOG = 1, GATE_DT_BIAS = 2 };   // lq_step_io.gate_bf16
+__device__ __forceinline__ GateWord gate_word(const StepIo& io, int which, int i) {
+  const void* p = which == GATE_A_LOG ? io.A_log : io.dt_bias;
+  if (!LQ_GATE_BF16) return {__float_as_uint(((const float*)p)[i]), 0u};
+  const bool bf16 = ((unsigned)io.rows >> 30) & which;
+  const char* at = (const char*)p + (long long)i * (bf16 ? 2 : 4);
+  return {*(const uint32_t*)__builtin_align_down(at, 4), bf16 ? 1 + (((unsigned)(uintptr_t)at >> 1) & 1u) : 0u};
+}
 
 // The MFMA B-operand tables (dig, bkq, hkq) are read as 16-byte fragments of up to six rows at once: their rows are
 // padded by 16 bytes so that those rows start in different LDS banks (unpadded, 128- or 256-byte rows all start in
@@ -169,7 +214,7 @@ __device__ __forceinline__ void flush_due(LDS& lds, const lq_state& st, const fl
 // by the last wave.  16 (the rank ablation R <= 16, K = V = 128; kernels.py:63, 457-469): up to G tiles, tile g taken
 // by the second wave of head g.
 // The row, and the unit in it, of a one-launch decode's workgroup: block b of `per` blocks a row.  Of the first `rot` rows
-// (rotated_rows; their number is in io.N, which is beside the first thing that a workgroup reads), each full round of 256
+// (rotated_rows; their number is in StepIo, beside the first thing that a workgroup reads), each full round of 256
 // blocks (one per CU) takes its rows rotated by three more than the round before.  `per` a power of two: shifts and masks
 // (four divisions in their place cost config 1 0.6 us a call).
 constexpr int CUS = 256;
@@ -191,7 +236,7 @@ __device__ __forceinline__ RowUnit decode_row(int b, int per, int rot) {
 // step appends the key, the same bytes to the same row (the heads of a key head that are not full share one fill), so that
 // its own flush finds it whatever the other's workgroup has written.
 template <int K_, int V_, int G, bool CONV, bool FL, int UW, int RM, bool DF, int KSH = 0, class LDS>
-__device__ __forceinline__ unsigned gdn_step(LDS& lds, const lq_state& st, const lq_step_io& io, const lq_conv& cv,
+__device__ __forceinline__ unsigned gdn_step(LDS& lds, const lq_state& st, const StepIo& io, const lq_conv& cv,
                                              int* dlist, const float* Q0, int& slot_) {
   static_assert(KSH == 0 || (FL && !CONV && UW == 1), "split key heads: the one-launch decode without conv");
   static_assert(!DF || FL, "deferred flush (lq_gdn_decode_deferred): the fused decode kernel");
@@ -205,7 +250,7 @@ __device__ __forceinline__ unsigned gdn_step(LDS& lds, const lq_state& st, const
   constexpr bool NT = KD == 128;                  // non-temporal bulk loads (see ld_once)
   constexpr int NH = UW * G;                                // value heads of the workgroup
   const int H = st.H, HV = st.HV, L = st.L, R = st.R;
-  const RowUnit ru = FL ? decode_row(blockIdx.x, (H << KSH) / UW, io.N) : RowUnit{(int)blockIdx.x / H, (int)blockIdx.x % H};
+  const RowUnit ru = FL ? decode_row(blockIdx.x, (H << KSH) / UW, io.rotated()) : RowUnit{(int)blockIdx.x / H, (int)blockIdx.x % H};
   const int n = ru.n, hk0 = ru.u * UW;                      // the row; the workgroup's first unit (KSH = 0: key head)
   const int un = UW == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * WPH * G));   // this wave's unit
   const int hk = hk0 + un, hkey = hk >> KSH;                // this wave's unit and its key head
@@ -254,7 +299,7 @@ __device__ __forceinline__ unsigned gdn_step(LDS& lds, const lq_state& st, const
   }
   const bf16_t araw = ((const bf16_t*)io.a)[(long long)n * HV + hv];
   const bf16_t braw = ((const bf16_t*)io.b)[(long long)n * HV + hv];
-  const float dtb = io.dt_bias[hv], alog = io.A_log[hv];
+  const GateWord dtw = gate_word(io, GATE_DT_BIAS, hv), alw = gate_word(io, GATE_A_LOG, hv);
   float vin = 0.f;
   if (!CONV) vin = bf2f(mrow[2ll * H * KD + hv * VD + lt]);
 
@@ -321,7 +366,7 @@ __device__ __forceinline__ unsigned gdn_step(LDS& lds, const lq_state& st, const
   if (wi == 0) {
     float alpha = 0.f, beta = 0.f;
     if constexpr (!GL) {
-      alpha = gdn_alpha_f(bf2f(araw), dtb, alog);
+      alpha = gdn_alpha_f(bf2f(araw), dtw.value(), alw.value());
       beta = beta_f(bf2f(braw));
     }
     if (CONV) {                 // the key / query taps: loaded by the scalar-work waves only (the other waves skip them)
@@ -477,7 +522,7 @@ __device__ __forceinline__ unsigned gdn_step(LDS& lds, const lq_state& st, const
   constexpr int AFTER_WINDOW = KS32 * KT + (RW / 16) * KS64;
   __builtin_amdgcn_sched_barrier(0);
   if (GL && wi == WPH - 1) {
-    const float alpha = gdn_alpha_f(bf2f(araw), dtb, alog);
+    const float alpha = gdn_alpha_f(bf2f(araw), dtw.value(), alw.value());
     const float beta = beta_f(bf2f(braw));
 #pragma unroll
     for (int e = 0; e < NE; ++e) {
@@ -669,7 +714,7 @@ __device__ __forceinline__ unsigned gdn_step(LDS& lds, const lq_state& st, const
 
 template <int K_, int V_, int G, bool CONV, bool FL, int RM = 4, bool DF = false>
 __global__ __launch_bounds__(64 * step_wph<V_>() * G) __attribute__((amdgpu_waves_per_eu(4)))
-void gdn_step_kernel(lq_state st, lq_step_io io, lq_conv cv, int* dlist, const float* Q0) {
+void gdn_step_kernel(lq_state st, StepIo io, lq_conv cv, int* dlist, const float* Q0) {
   __shared__ StepLds<K_, V_, G, FL, RM> lds;
   int slot;
   const unsigned due = gdn_step<K_, V_, G, CONV, FL, 1, RM, DF>(lds, st, io, cv, dlist, Q0, slot);
@@ -678,7 +723,7 @@ void gdn_step_kernel(lq_state st, lq_step_io io, lq_conv cv, int* dlist, const f
     if (due) {
       __syncthreads();          // the step is done with the shared bytes, and its appends are visible to the workgroup
       const float qm = code_range(st);
-      const RowUnit ru = decode_row(blockIdx.x, st.H, io.N);
+      const RowUnit ru = decode_row(blockIdx.x, st.H, io.rotated());
       const int n = ru.n, hv0 = ru.u * G;
       if constexpr (DF) {       // the first due head now, the other at the start of the next call
         lqf::flush_head4<128, 128, true>(lds.fl[0], st, Q0, slot, hv0 + (due & 1u ? 0 : 1), qm);
@@ -692,37 +737,37 @@ void gdn_step_kernel(lq_state st, lq_step_io io, lq_conv cv, int* dlist, const f
 // the one-launch decode at GQA 1: W = 2 value heads, of two key heads, per workgroup
 template <int K_, int V_, int W, bool CONV>
 __global__ __launch_bounds__(64 * step_wph<V_>() * W) __attribute__((amdgpu_waves_per_eu(4)))
-void gdn_step_kernel(lq_state st, lq_step_io io, lq_conv cv, const float* Q0) {
+void gdn_step_kernel(lq_state st, StepIo io, lq_conv cv, const float* Q0) {
   static_assert(W == step_units<1, true>(), "value heads of a workgroup");
   __shared__ StepLds<K_, V_, 1, true, 4> lds;
   int slot;
   const unsigned due = gdn_step<K_, V_, 1, CONV, true, W, 4, false>(lds, st, io, cv, nullptr, Q0, slot);
   if (due) {
     __syncthreads();
-    const int hv0 = decode_row(blockIdx.x, st.H / W, io.N).u * W;
+    const int hv0 = decode_row(blockIdx.x, st.H / W, io.rotated()).u * W;
     flush_due<K_, V_, 1, W, 1>(lds, st, Q0, slot, hv0, due, code_range(st));
   }
 }
 // the one-launch decode at GQA 4: G = 2 value heads per workgroup, 2^KSH workgroups per key head
 template <int K_, int V_, int G, int KSH>
 __global__ __launch_bounds__(64 * step_wph<V_>() * G) __attribute__((amdgpu_waves_per_eu(4)))
-void gdn_step_kernel(lq_state st, lq_step_io io, const float* Q0) {
+void gdn_step_kernel(lq_state st, StepIo io, const float* Q0) {
   __shared__ StepLds<K_, V_, G, true, 4> lds;
   int slot;
   const unsigned due = gdn_step<K_, V_, G, false, true, 1, 4, false, KSH>(lds, st, io, lq_conv{}, nullptr, Q0, slot);
   if (due) {
     __syncthreads();
-    flush_due<K_, V_, G, G, 1>(lds, st, Q0, slot, decode_row(blockIdx.x, st.H << KSH, io.N).u * G, due, code_range(st));
+    flush_due<K_, V_, G, G, 1>(lds, st, Q0, slot, decode_row(blockIdx.x, st.H << KSH, io.rotated()).u * G, due, code_range(st));
   }
 }
 // the one-launch decode with helper waves: one key head per workgroup, G value heads, 256 G = 128 W threads.  The waves
 // past the step's pass its barriers, and then each group of 256 threads flushes a head.
 template <int K_, int V_, int W, bool CONV, int G>
 __global__ __launch_bounds__(128 * W) __attribute__((amdgpu_waves_per_eu(4)))
-void gdn_step_kernel(lq_state st, lq_step_io io, lq_conv cv, const float* Q0) {
+void gdn_step_kernel(lq_state st, StepIo io, lq_conv cv, const float* Q0) {
   static_assert(W == 2 * G && step_wph<V_>() == 2, "two step waves and two helpers per value head");
   __shared__ WideLds<K_, V_, G> lds;
-  const RowUnit ru = decode_row(blockIdx.x, st.H, io.N);
+  const RowUnit ru = decode_row(blockIdx.x, st.H, io.rotated());
   const int n = ru.n, hv0 = ru.u * G;
   int slot;
   unsigned due = 0;
@@ -850,7 +895,7 @@ __device__ __forceinline__ int kda_chunks(const int (&hw)[UW], int L) {
 }
 
 template <int UW, bool FL>
-__device__ __forceinline__ void kda_step(KdaShared* units, const lq_state& st, const lq_step_io& io, float glb,
+__device__ __forceinline__ void kda_step(KdaShared* units, const lq_state& st, const StepIo& io, float glb,
                                              int* dlist, int& slot_, unsigned& due_) {
   const int H = st.H, HV = st.HV, L = st.L, R = st.R;
   const int G = HV / H;
@@ -883,7 +928,8 @@ __device__ __forceinline__ void kda_step(KdaShared* units, const lq_state& st, c
   __builtin_amdgcn_sched_barrier(0);
   // per-channel operands: wave 0 (scalar work) channels c = lane, lane + 64; wave 1 (its own gate) c = 2 lane + e
   bf16_t kxr[2], qxr[2], axr[2];
-  float skx[2], dtx[2], pbx[2], wx[2];
+  GateWord dtw[2];
+  float skx[2], pbx[2], wx[2];
 #pragma unroll
   for (int e = 0; e < 2; ++e) {
     const int c = lane + 64 * e;
@@ -892,12 +938,12 @@ __device__ __forceinline__ void kda_step(KdaShared* units, const lq_state& st, c
     qxr[e] = mrow[hk * KD + c];
     axr[e] = ((const bf16_t*)io.a)[((long long)n * HV + hv) * KD + cg];
     skx[e] = Skp[c];
-    dtx[e] = io.dt_bias[hv * KD + cg];
+    dtw[e] = gate_word(io, GATE_DT_BIAS, hv * KD + cg);
     pbx[e] = st.Pbuf[sh_ * KD + c];
     wx[e] = st.Wbuf[sh_ * L + min(c, L - 1)];
   }
   const bf16_t braw = ((const bf16_t*)io.b)[(long long)n * HV + hv];
-  const float alog = io.A_log[hv];
+  const GateWord alw = gate_word(io, GATE_A_LOG, hv);
   const float vin = bf2f(mrow[2ll * H * KD + hv * VD + lt]);
   const float sv = Svp[lt];
   __builtin_amdgcn_sched_barrier(0);
@@ -950,7 +996,7 @@ __device__ __forceinline__ void kda_step(KdaShared* units, const lq_state& st, c
   }
   constexpr int AFTER_WINDOW = 8;   // vector memory operations issued after the first chunk's loads: the tile
   __builtin_amdgcn_sched_barrier(0);
-  const float ea = expf(alog);
+  const float ea = expf(alw.value()), dtx[2] = {dtw[0].value(), dtw[1].value()};
 
   // ---- wave 0: per-channel gate, norms, digits, dot operands.  wave 1: its own entries' decayed keys (chunk 0) ----
   float gnv[2] = {0.f, 0.f}, env[2] = {0.f, 0.f};
@@ -1189,7 +1235,7 @@ __device__ __forceinline__ void kda_step(KdaShared* units, const lq_state& st, c
 }
 
 __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(4)))
-void kda_step_kernel(lq_state st, lq_step_io io, float glb, int* dlist) {
+void kda_step_kernel(lq_state st, StepIo io, float glb, int* dlist) {
   int slot;
   unsigned due;
   kda_step<1, false>(nullptr, st, io, glb, dlist, slot, due);
@@ -1198,7 +1244,7 @@ void kda_step_kernel(lq_state st, lq_step_io io, float glb, int* dlist) {
 // that pass the step's barriers and only flush
 template <int W>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
-void flush4_kernel(lq_state st, lq_step_io io, float glb, const float* Q0) {
+void flush4_kernel(lq_state st, StepIo io, float glb, const float* Q0) {
   __shared__ KdaLds<W> lds;
   const int n = blockIdx.x / (st.HV / W), hv0 = (blockIdx.x - n * (st.HV / W)) * W;
   int slot;
@@ -1229,32 +1275,13 @@ void flush4_kernel(lq_state st, lq_step_io io, float glb, const float* Q0) {
 
 }  // namespace
 
-// head dims of the GDN step (kernels.py:62); the KDA step is K = V = 128 only (kernels.py:727)
-static bool gdn_dims(int K, int V) { return (K == 128 && V == 128) || (K == 64 && (V == 128 || V == 64)); }
-
-int lq_check_step(const lq_state* st, const lq_step_io* io) {
-  if (!st || !io) return LQ_ERR_ARG;
-  if (!gdn_dims(st->K, st->V) || st->L < 1 || st->L > LMAX || st->R < 1) return LQ_ERR_ARG;
-  if (st->R > (st->K == 128 && st->V == 128 ? LQ_STEP_RMAX : 4)) return LQ_ERR_ARG;   // kernels.py:63-64
-  if (st->H <= 0 || st->HV <= 0 || st->HV % st->H != 0 || st->NS <= 0 || io->N < 0) return LQ_ERR_ARG;
-  if (!st->ssm || !st->Kbuf || !st->Ubuf || !st->Wbuf || !st->Pbuf || !st->hcnt) return LQ_ERR_ARG;
-  // 16-byte loads of the int8 rows and of the scale / factor block need a 16-byte aligned block start
-  if (st->slot_stride < (long long)st->HV * st->V * st->K || (st->slot_stride & 3) || ((uintptr_t)st->ssm & 15))
-    return LQ_ERR_ARG;
-  if (!buffers_aligned(st)) return LQ_ERR_ARG;
-  if (!(st->qmax == 0.f || (st->qmax >= 1.f && st->qmax <= 127.f))) return LQ_ERR_ARG;
-  if (io->N > 0 && (!io->mixed || !io->a || !io->b || !io->A_log || !io->dt_bias || !io->idx || !io->out))
-    return LQ_ERR_ARG;
-  return LQ_OK;
-}
-
 template <int K_, int V_, bool CONV, int RM = 4>
 static int launch_gdn(const lq_state* st, const lq_step_io* io, const lq_conv& cv, int* dlist, hipStream_t s) {
   dim3 grid((unsigned)(io->N * st->H));
   switch (st->HV / st->H) {
-    case 1: gdn_step_kernel<K_, V_, 1, CONV, false, RM><<<grid, 64 * step_wph<V_>(), 0, s>>>(*st, *io, cv, dlist, nullptr); break;
-    case 2: gdn_step_kernel<K_, V_, 2, CONV, false, RM><<<grid, 128 * step_wph<V_>(), 0, s>>>(*st, *io, cv, dlist, nullptr); break;
-    case 4: gdn_step_kernel<K_, V_, 4, CONV, false, RM><<<grid, 256 * step_wph<V_>(), 0, s>>>(*st, *io, cv, dlist, nullptr); break;
+    case 1: gdn_step_kernel<K_, V_, 1, CONV, false, RM><<<grid, 64 * step_wph<V_>(), 0, s>>>(*st, step_io(io), cv, dlist, nullptr); break;
+    case 2: gdn_step_kernel<K_, V_, 2, CONV, false, RM><<<grid, 128 * step_wph<V_>(), 0, s>>>(*st, step_io(io), cv, dlist, nullptr); break;
+    case 4: gdn_step_kernel<K_, V_, 4, CONV, false, RM><<<grid, 256 * step_wph<V_>(), 0, s>>>(*st, step_io(io), cv, dlist, nullptr); break;
     default: return LQ_ERR_ARG;
   }
   return hipGetLastError() == hipSuccess ? LQ_OK : LQ_ERR_HIP;
@@ -1274,15 +1301,14 @@ static int launch_gdn_dims(const lq_state* st, const lq_step_io* io, const lq_co
 // rotated by three more each: rows at different fills, W = 16, us per call, in order -> rotated: 61 rows with conv and
 // deferred flushes 31.7 -> 26.1, without conv 28.3 -> 22.9; 100 rows of 8 key heads 25.0 -> 21.0.  Elsewhere the rows stay in
 // order (64 such rows at W = 64 24.4 us in order, 24.8 rotated).
-static lq_step_io rotated_rows(const lq_state* st, const lq_step_io* io, int per, bool deferred = false) {
-  lq_step_io r = *io;
-  r.N = 0;                                            // the kernels' N: the rows that the rotation covers
+static StepIo rotated_rows(const lq_state* st, const lq_step_io* io, int per, bool deferred = false) {
+  int rows = 0;                                       // the rows that the rotation covers
   if (per <= CUS && (per & (per - 1)) == 0)
     for (int k = 1; k <= 3; ++k) {
       const int d = k * (CUS / per) % st->L;
-      if (d == 0 || (deferred && (d == 1 || d == st->L - 1))) r.N = io->N;
+      if (d == 0 || (deferred && (d == 1 || d == st->L - 1))) rows = io->N;
     }
-  return r;
+  return step_io(io, rows);
 }
 
 // Small launches, up to four heads per CU, take the kernels with helper waves: their workgroups flush their heads side by
@@ -1304,7 +1330,7 @@ static int launch_decode(const lq_state* st, const lq_step_io* io, const lq_conv
   const int G = st->HV / st->H;
   const dim3 grid((unsigned)(io->N * (G == 1 ? st->H / 2 : st->H)));
   const bool wide = helper_waves(st, io->N);
-  const lq_step_io rio = rotated_rows(st, io, G == 1 ? st->H / 2 : st->H);
+  const StepIo rio = rotated_rows(st, io, G == 1 ? st->H / 2 : st->H);
   switch (G) {
     case 1:
       if (wide) launch_wide<K_, V_, CONV, 1>(st, io, cv, Q0, s);
@@ -1337,7 +1363,7 @@ static int launch_decode(const lq_state* st, const lq_step_io* io, const lq_conv
 template <bool CONV>
 static int launch_decode8(const lq_state* st, const lq_step_io* io, const lq_conv& cv, const float* Q0, hipStream_t s) {
   const dim3 grid((unsigned)(io->N * st->H));
-  const lq_step_io rio = rotated_rows(st, io, st->H);
+  const StepIo rio = rotated_rows(st, io, st->H);
   if (st->HV == 2 * st->H) gdn_step_kernel<128, 128, 2, CONV, true, 16><<<grid, 256, 0, s>>>(*st, rio, cv, nullptr, Q0);
   else gdn_step_kernel<128, 128, 4, CONV, true, 16><<<grid, 512, 0, s>>>(*st, rio, cv, nullptr, Q0);
   return hipGetLastError() == hipSuccess ? LQ_OK : LQ_ERR_HIP;
@@ -1366,16 +1392,67 @@ static bool one_launch(const lq_state* st, int N, bool conv, bool deferred) {
   return G == 1 || G == 2 || G == 4;
 }
 
+int LQ_LAUNCH(step)(const lq_state* st, const lq_step_io* io, const lq_conv* cv, int kda, float glb, int* dlist,
+                    hipStream_t s) {
+  if (!kda) return cv ? launch_gdn_dims<true>(st, io, *cv, dlist, s) : launch_gdn_dims<false>(st, io, lq_conv{}, dlist, s);
+  if (st->R > 4) return LQ_ERR_ARG;           // the KDA step holds four factors (kernels.py:1036)
+  kda_step_kernel<<<dim3((unsigned)(io->N * st->HV)), 128, 0, s>>>(*st, step_io(io), glb, dlist);
+  return hipGetLastError() == hipSuccess ? LQ_OK : LQ_ERR_HIP;
+}
+
+int LQ_LAUNCH(gdn_decode)(const lq_state* st, const lq_step_io* io, const lq_conv* cv, const float* Q0, bool deferred,
+                          hipStream_t s) {
+  if (deferred && st->K == 128 && st->V == 128 && st->HV == 2 * st->H && st->R <= 4) {
+    const dim3 grid((unsigned)(io->N * st->H));
+    const StepIo rio = rotated_rows(st, io, st->H, true);
+    if (cv) gdn_step_kernel<128, 128, 2, true, true, 4, true><<<grid, 256, 0, s>>>(*st, rio, *cv, nullptr, Q0);
+    else gdn_step_kernel<128, 128, 2, false, true, 4, true><<<grid, 256, 0, s>>>(*st, rio, lq_conv{}, nullptr, Q0);
+    return hipGetLastError() == hipSuccess ? LQ_OK : LQ_ERR_HIP;
+  }
+  if (one_launch(st, io->N, cv != nullptr, deferred))
+    return cv ? launch_decode_dims<true>(st, io, *cv, Q0, s) : launch_decode_dims<false>(st, io, lq_conv{}, Q0, s);
+  const int rc = LQ_LAUNCH(step)(st, io, cv, 0, 0.f, nullptr, s);
+  return rc ? rc : lq_launch_flush(st, Q0, io->idx, io->N, 0, st->qmax > 0.f ? st->qmax : LQ_QMAX, nullptr, s);
+}
+
+int LQ_LAUNCH(kda_decode)(const lq_state* st, const lq_step_io* io, float glb, const float* Q0, hipStream_t s) {
+  const unsigned heads = (unsigned)io->N * (unsigned)st->HV;
+  switch (lq_kda_decode_heads(io->N, st->HV, st->H, st->L, lq_num_cus())) {
+    case 1: flush4_kernel<1><<<dim3(heads), 256, 0, s>>>(*st, step_io(io), glb, Q0); break;
+    case 2: flush4_kernel<2><<<dim3(heads / 2), 256, 0, s>>>(*st, step_io(io), glb, Q0); break;
+    default: {
+      const int rc = LQ_LAUNCH(step)(st, io, nullptr, 1, glb, nullptr, s);
+      return rc ? rc : lq_launch_flush(st, Q0, io->idx, io->N, 1, st->qmax > 0.f ? st->qmax : LQ_QMAX, nullptr, s);
+    }
+  }
+  return hipGetLastError() == hipSuccess ? LQ_OK : LQ_ERR_HIP;
+}
+
+#if !LQ_GATE_BF16
+// ---- entry points: checks, then the launches for the gate parameters' dtypes ------------------------------------------
+// head dims of the GDN step (kernels.py:62); the KDA step is K = V = 128 only (kernels.py:727)
+static bool gdn_dims(int K, int V) { return (K == 128 && V == 128) || (K == 64 && (V == 128 || V == 64)); }
+
+int lq_check_step(const lq_state* st, const lq_step_io* io) {
+  if (!st || !io) return LQ_ERR_ARG;
+  if (!gdn_dims(st->K, st->V) || st->L < 1 || st->L > LMAX || st->R < 1) return LQ_ERR_ARG;
+  if (st->R > (st->K == 128 && st->V == 128 ? LQ_STEP_RMAX : 4)) return LQ_ERR_ARG;   // kernels.py:63-64
+  if (st->H <= 0 || st->HV <= 0 || st->HV % st->H != 0 || st->NS <= 0 || io->N < 0) return LQ_ERR_ARG;
+  if (!st->ssm || !st->Kbuf || !st->Ubuf || !st->Wbuf || !st->Pbuf || !st->hcnt) return LQ_ERR_ARG;
+  // 16-byte loads of the int8 rows and of the scale / factor block need a 16-byte aligned block start
+  if (st->slot_stride < (long long)st->HV * st->V * st->K || (st->slot_stride & 3) || ((uintptr_t)st->ssm & 15))
+    return LQ_ERR_ARG;
+  if (!buffers_aligned(st)) return LQ_ERR_ARG;
+  if (!(st->qmax == 0.f || (st->qmax >= 1.f && st->qmax <= 127.f)) || (io->gate_bf16 & ~3)) return LQ_ERR_ARG;
+  if (io->N > 0 && (!io->mixed || !io->a || !io->b || !io->A_log || !io->dt_bias || !io->idx || !io->out))
+    return LQ_ERR_ARG;
+  return LQ_OK;
+}
+
 // the plain GDN / KDA step of every row, arguments already checked
 int lq_launch_step(const lq_state* st, const lq_step_io* io, int kda, float glb, int* dlist, hipStream_t s) {
   if (io->N == 0) return LQ_OK;
-  if (!kda) {
-    const lq_conv none = {};
-    return launch_gdn_dims<false>(st, io, none, dlist, s);
-  }
-  if (st->R > 4) return LQ_ERR_ARG;           // the KDA step holds four factors (kernels.py:1036)
-  kda_step_kernel<<<dim3((unsigned)(io->N * st->HV)), 128, 0, s>>>(*st, *io, glb, dlist);
-  return hipGetLastError() == hipSuccess ? LQ_OK : LQ_ERR_HIP;
+  return (io->gate_bf16 ? lq_bf16_step : lq_f32_step)(st, io, nullptr, kda, glb, dlist, s);
 }
 
 extern "C" int lq_gdn_step(const lq_state* st, const lq_step_io* io, void* stream) {
@@ -1400,7 +1477,7 @@ extern "C" int lq_gdn_step_conv(const lq_state* st, const lq_step_io* io, const 
   if (rc) return rc;
   if ((rc = check_conv(st, cv))) return rc;
   if (io->N == 0) return LQ_OK;
-  return launch_gdn_dims<true>(st, io, *cv, nullptr, (hipStream_t)stream);
+  return (io->gate_bf16 ? lq_bf16_step : lq_f32_step)(st, io, cv, 0, 0.f, nullptr, (hipStream_t)stream);
 }
 
 static int gdn_decode(const lq_state* st, const lq_step_io* io, const lq_conv* cv, const float* Q0, bool deferred,
@@ -1411,19 +1488,7 @@ static int gdn_decode(const lq_state* st, const lq_step_io* io, const lq_conv* c
   const float qmax = st->qmax > 0.f ? st->qmax : LQ_QMAX;
   if ((rc = lq_check_flush(st, Q0, io->idx, io->N, 0, qmax))) return rc;
   if (io->N == 0) return LQ_OK;
-  if (deferred && st->K == 128 && st->V == 128 && st->HV == 2 * st->H && st->R <= 4) {
-    const dim3 grid((unsigned)(io->N * st->H));
-    const lq_conv none = {};
-    const lq_step_io rio = rotated_rows(st, io, st->H, true);
-      if (cv) gdn_step_kernel<128, 128, 2, true, true, 4, true><<<grid, 256, 0, s>>>(*st, rio, *cv, nullptr, Q0);
-    else gdn_step_kernel<128, 128, 2, false, true, 4, true><<<grid, 256, 0, s>>>(*st, rio, none, nullptr, Q0);
-    return hipGetLastError() == hipSuccess ? LQ_OK : LQ_ERR_HIP;
-  }
-  if (one_launch(st, io->N, cv != nullptr, deferred))
-    return cv ? launch_decode_dims<true>(st, io, *cv, Q0, s) : launch_decode_dims<false>(st, io, lq_conv{}, Q0, s);
-  rc = cv ? launch_gdn_dims<true>(st, io, *cv, nullptr, s) : lq_launch_step(st, io, 0, 0.f, nullptr, s);
-  if (rc) return rc;
-  return lq_launch_flush(st, Q0, io->idx, io->N, 0, qmax, nullptr, s);
+  return (io->gate_bf16 ? lq_bf16_gdn_decode : lq_f32_gdn_decode)(st, io, cv, Q0, deferred, s);
 }
 
 extern "C" int lq_gdn_decode(const lq_state* st, const lq_step_io* io, const lq_conv* cv, const float* Q0,
@@ -1450,16 +1515,8 @@ extern "C" int lq_kda_decode(const lq_state* st, const lq_step_io* io, float glb
   const float qmax = st->qmax > 0.f ? st->qmax : LQ_QMAX;
   if ((rc = lq_check_flush(st, Q0, io->idx, io->N, 1, qmax))) return rc;
   if (io->N == 0) return LQ_OK;
-  hipStream_t s = (hipStream_t)stream;
-  const unsigned heads = (unsigned)io->N * (unsigned)st->HV;
-  switch (lq_kda_decode_heads(io->N, st->HV, st->H, st->L, lq_num_cus())) {
-    case 1: flush4_kernel<1><<<dim3(heads), 256, 0, s>>>(*st, *io, glb, Q0); break;
-    case 2: flush4_kernel<2><<<dim3(heads / 2), 256, 0, s>>>(*st, *io, glb, Q0); break;
-    default:
-      if ((rc = lq_launch_step(st, io, 1, glb, nullptr, s))) return rc;
-      return lq_launch_flush(st, Q0, io->idx, io->N, 1, qmax, nullptr, s);
-  }
-  return hipGetLastError() == hipSuccess ? LQ_OK : LQ_ERR_HIP;
+  return (io->gate_bf16 ? lq_bf16_kda_decode : lq_f32_kda_decode)(st, io, glb, Q0, (hipStream_t)stream);
 }
 
 extern "C" int lq_abi_version(void) { return LQ_ABI_VERSION; }
+#endif  // !LQ_GATE_BF16

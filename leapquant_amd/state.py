@@ -54,6 +54,9 @@ def state_views(ssm, R):
         uq=_alias(ssm, torch.float16, (NS, HV, R, K + V), (2 * SS, 2 * V * K, K + V, 1), 2 * (sc + K + V)))
 
 
+_F32, _BF16 = torch.float32, torch.bfloat16
+
+
 class LeapQuantState:
     """Window buffers + kernels of one linear-attention layer.
 
@@ -108,25 +111,21 @@ class LeapQuantState:
         self._vkey = None
         self._skey = None
         self._scan_src = None
-        self._param_f32 = {}
 
-    def _as_f32(self, t):
-        """A gate parameter (A_log, dt_bias) as the fp32 tensor the kernels read.  A parameter in another dtype is
-        converted once and the copy kept, keyed by the parameter's address and dtype (a state tensor may be shared by
-        layers that each bring their own parameters)."""
-        if t.dtype == torch.float32:
-            return t
-        key = (t.data_ptr(), t.dtype)
-        if key not in self._param_f32:
-            self._param_f32[key] = t.detach().float().contiguous()
-        return self._param_f32[key]
+    @staticmethod
+    def _param(t, n):
+        """A gate parameter (A_log, dt_bias) as n contiguous values, in its own dtype if the kernels read it (fp32, bf16),
+        else converted here on every call: a copy kept from one call to the next would outlive an update of the parameter
+        in place.  Only the address goes to the kernels, so a tensor of as many contiguous values is taken as it is (a
+        reshape costs the host ~2 us, three of them 6 of a decode call's 12)."""
+        if t.dtype is not _F32 and t.dtype is not _BF16:
+            t = t.detach().float()
+        return t if t.numel() == n and t.is_contiguous() else t.reshape(n).contiguous()
 
-    def _param(self, t, shape):
-        """A gate parameter as contiguous fp32 values of `shape`.  Only the address goes to the kernels, so a tensor of as
-        many contiguous values is taken as it is (a reshape costs the host ~2 us, three of them 6 of a decode call's 12)."""
-        t = self._as_f32(t)
-        n = shape[0] * shape[1] if len(shape) == 2 else shape[0]
-        return t if t.numel() == n and t.is_contiguous() else t.reshape(shape).contiguous()
+    @staticmethod
+    def _gate_bf16(A_log, dt_bias):
+        """lq_step_io.gate_bf16 of two parameters as _param returns them, one of them not fp32."""
+        return (A_log.dtype is _BF16) + 2 * (dt_bias.dtype is _BF16)
 
     def views(self, ssm):
         k = _ident(ssm)
@@ -155,8 +154,8 @@ class LeapQuantState:
         N = idx.shape[0]
         self._check_gate(a, N, KA)
         a = a.contiguous()
-        dt_bias = self._param(dt_bias, (self.HV, KA))
-        A_log = self._param(A_log, (self.HV,))
+        dt_bias = self._param(dt_bias, self.HV * KA)
+        A_log = self._param(A_log, self.HV)
         idx = idx if idx.dtype == torch.int32 else idx.to(torch.int32)
         idx = idx.contiguous()
         if (mixed.dtype != torch.bfloat16 or not mixed.is_contiguous()
@@ -169,7 +168,8 @@ class LeapQuantState:
         b = b.contiguous()
         st = self._struct(ssm)
         dev = KN._dev
-        io = _lib.LqStepIO(dev(mixed), dev(a), dev(b), dev(A_log), dev(dt_bias), dev(idx), dev(out), N, self._scale)
+        io = _lib.LqStepIO(dev(mixed), dev(a), dev(b), dev(A_log), dev(dt_bias), dev(idx), dev(out), N, self._scale,
+                           0 if A_log.dtype is dt_bias.dtype is _F32 else self._gate_bf16(A_log, dt_bias))
         stream = KN._raw_stream(mixed)
         L = self._lib
         if self.kda:                 # step + flush of the heads it fills (one launch for small batches)
@@ -198,8 +198,8 @@ class LeapQuantState:
         N = idx.shape[0]
         self._check_gate(a, N, 1)
         a = a.contiguous()
-        dt_bias = self._param(dt_bias, (self.HV,))
-        A_log = self._param(A_log, (self.HV,))
+        dt_bias = self._param(dt_bias, self.HV)
+        A_log = self._param(A_log, self.HV)
         idx = idx if idx.dtype == torch.int32 else idx.to(torch.int32)
         idx = idx.contiguous()
         if x.dtype != torch.bfloat16 or not x.is_contiguous() or x.shape != (N, C):
@@ -211,7 +211,8 @@ class LeapQuantState:
         b = b.contiguous()
         st = self._struct(ssm)
         dev = KN._dev
-        io = _lib.LqStepIO(dev(x), dev(a), dev(b), dev(A_log), dev(dt_bias), dev(idx), dev(out), N, self._scale)
+        io = _lib.LqStepIO(dev(x), dev(a), dev(b), dev(A_log), dev(dt_bias), dev(idx), dev(out), N, self._scale,
+                           0 if A_log.dtype is dt_bias.dtype is _F32 else self._gate_bf16(A_log, dt_bias))
         cv = KN.conv_struct(conv_state, w, conv_bias, silu)
         stream = KN._raw_stream(x)
         fn = self._lib.lq_gdn_decode_deferred if self.defer_flush else self._lib.lq_gdn_decode
