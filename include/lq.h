@@ -117,8 +117,8 @@ int lq_gdn_step_conv(const lq_state* st, const lq_step_io* io, const lq_conv* cv
  * qmax = st->qmax, 0 meaning 127) -- what lq_gdn_step (or lq_gdn_step_conv) followed by lq_flush computes, in one
  * call.  Replaces make_gdn_step(...)(...) followed by make_flush(...)(...) as LeapQuantState.decode launches them
  * (/root/reference/leapquant/state.py:99-116; kernels.py:27-692, 1077-2033).  It is one launch, in which each workgroup
- * flushes the heads it has just filled (or found full) on the same threads; an odd H and ranks above 4 at HV = H, and large
- * (64, 64) batches at HV = 4 H, run the step and the flush as two launches.  Same limits as lq_gdn_step and lq_flush. */
+ * flushes the heads it has just filled (or found full); an odd H or ranks above 4 at HV = H, and large (64, 64) batches at
+ * HV = 4 H, run the step and the flush as two launches.  Same limits as lq_gdn_step and lq_flush. */
 int lq_gdn_decode(const lq_state* st, const lq_step_io* io, const lq_conv* cv, const float* Q0, void* stream);
 
 /* lq_gdn_decode with the flush of a key head's second value head deferred: no counterpart in the reference (whose
@@ -129,7 +129,8 @@ int lq_gdn_decode(const lq_state* st, const lq_step_io* io, const lq_conv* cv, c
  * (a full head is flushed before any step reads it); between calls a slot may hold a full head, so a reader of the
  * checkpoint other than these two calls runs lq_flush on its slots first (LeapQuantState.dequantize does).  A filling
  * call costs one head's flush instead of two: the latency that a due row adds to the call halves.  Other shapes: as
- * lq_gdn_decode. */
+ * lq_gdn_decode, with the flush in a launch of its own where rows at different fills are faster that way (HV = 4 H: ranks
+ * above 4; V = 128 with few heads, or with the conv above four heads per CU). */
 int lq_gdn_decode_deferred(const lq_state* st, const lq_step_io* io, const lq_conv* cv, const float* Q0,
                            void* stream);
 

@@ -1311,14 +1311,6 @@ static StepIo rotated_rows(const lq_state* st, const lq_step_io* io, int per, bo
   return step_io(io, rows);
 }
 
-// Small launches, up to four heads per CU, take the kernels with helper waves: their workgroups flush their heads side by
-// side, and all stay resident.  A flush call of one row (us, in turn -> side by side): two GQA 1 heads 21.6 -> 14.6, two of
-// a key head 21.6 -> 16.8, four 29.2 -> 25.4, two KDA heads 24.6 -> 15.2.  Window 16, us per call without -> with: GQA 1,
-// 16 heads, B = 16 7.5 -> 6.5, B = 64 (4 heads per CU) 9.7 -> 9.6; GQA 2, B = 16 (2) 7.4 -> 7.3, B = 64 (8) 15.3 -> 17.4;
-// GQA 4, B = 16 (4) 9.4 -> 9.2, B = 32 (8) 15.7 -> 17.7; KDA, 32 heads, B = 1 8.2 -> 6.9, B = 32 (4) 13.0 -> 11.9,
-// B = 48 (6) 16.7 -> 18.6.
-static bool helper_waves(const lq_state* st, int N) { return lq_helper_waves(N, st->HV, lq_num_cus()); }
-
 // the decode call in one launch: each workgroup flushes the heads whose window it fills
 template <int K_, int V_, bool CONV, int G>
 static void launch_wide(const lq_state* st, const lq_step_io* io, const lq_conv& cv, const float* Q0, hipStream_t s) {
@@ -1326,10 +1318,10 @@ static void launch_wide(const lq_state* st, const lq_step_io* io, const lq_conv&
       *st, rotated_rows(st, io, st->H), cv, Q0);
 }
 template <int K_, int V_, bool CONV>
-static int launch_decode(const lq_state* st, const lq_step_io* io, const lq_conv& cv, const float* Q0, hipStream_t s) {
+static int launch_decode(const lq_state* st, const lq_step_io* io, const lq_conv& cv, const float* Q0, bool wide,
+                         hipStream_t s) {
   const int G = st->HV / st->H;
   const dim3 grid((unsigned)(io->N * (G == 1 ? st->H / 2 : st->H)));
-  const bool wide = helper_waves(st, io->N);
   const StepIo rio = rotated_rows(st, io, G == 1 ? st->H / 2 : st->H);
   switch (G) {
     case 1:
@@ -1369,29 +1361,13 @@ static int launch_decode8(const lq_state* st, const lq_step_io* io, const lq_con
   return hipGetLastError() == hipSuccess ? LQ_OK : LQ_ERR_HIP;
 }
 template <bool CONV>
-static int launch_decode_dims(const lq_state* st, const lq_step_io* io, const lq_conv& cv, const float* Q0,
+static int launch_decode_dims(const lq_state* st, const lq_step_io* io, const lq_conv& cv, const float* Q0, bool wide,
                               hipStream_t s) {
   if (st->R > 4) return launch_decode8<CONV>(st, io, cv, Q0, s);
-  if (st->K == 128) return launch_decode<128, 128, CONV>(st, io, cv, Q0, s);
-  return st->V == 128 ? launch_decode<64, 128, CONV>(st, io, cv, Q0, s) : launch_decode<64, 64, CONV>(st, io, cv, Q0, s);
+  if (st->K == 128) return launch_decode<128, 128, CONV>(st, io, cv, Q0, wide, s);
+  return st->V == 128 ? launch_decode<64, 128, CONV>(st, io, cv, Q0, wide, s)
+                      : launch_decode<64, 64, CONV>(st, io, cv, Q0, wide, s);
 }
-// Which calls take one launch.  The second launch, the flush, costs a call ~2 us also when nothing is due.  Window 16,
-// us per call, two launches -> one: 128 x 128 at GQA 4, B = 24, 16 key heads 16.5 -> 12.5, B = 200 78.2 -> 71.8; at GQA 1,
-// B = 64, 32 heads 21.0 -> 16.4, B = 200 45.8 -> 41.7; (64, 128) at GQA 2, B = 64 13.0 -> 10.4; (64, 64) at GQA 1,
-// B = 64 10.9 -> 8.5.  GQA 1 pairs two key heads of a row in a workgroup, so an odd H takes two launches.  So do large
-// (64, 64) batches at GQA 4, whose flush needs more LDS and registers than the step: us per call at 8 rows x H per CU 25.2 ->
-// 23.7, at 10 29.8 -> 29.0, at 12.5 35.7 -> 35.1 in two launches, 37.4 in one.  With the conv a key head's four value heads
-// stay in one workgroup (they share its conv state), 16.6 -> 14.3 at 4, 20.9 -> 20.0 at 6, 25.2 -> 25.6 at 8; and its V = 128
-// heads take two flushes in turn, so that a batch whose rows are due on different calls (which is what the deferred entry is
-// for) flushes them sooner in a launch of its own, over all CUs: 24 rows 38.8 us per call, in one launch 43.2.
-static bool one_launch(const lq_state* st, int N, bool conv, bool deferred) {
-  const int G = st->HV / st->H;
-  if (G == 1 && (st->R > 4 || st->H % 2 != 0)) return false;
-  if (G == 4 && conv && deferred && st->V == 128 && !helper_waves(st, N)) return false;
-  if (G == 4 && st->V == 64) return (long long)N * st->H <= (conv ? 6ll : 10ll) * lq_num_cus();
-  return G == 1 || G == 2 || G == 4;
-}
-
 int LQ_LAUNCH(step)(const lq_state* st, const lq_step_io* io, const lq_conv* cv, int kda, float glb, int* dlist,
                     hipStream_t s) {
   if (!kda) return cv ? launch_gdn_dims<true>(st, io, *cv, dlist, s) : launch_gdn_dims<false>(st, io, lq_conv{}, dlist, s);
@@ -1409,8 +1385,13 @@ int LQ_LAUNCH(gdn_decode)(const lq_state* st, const lq_step_io* io, const lq_con
     else gdn_step_kernel<128, 128, 2, false, true, 4, true><<<grid, 256, 0, s>>>(*st, rio, lq_conv{}, nullptr, Q0);
     return hipGetLastError() == hipSuccess ? LQ_OK : LQ_ERR_HIP;
   }
-  if (one_launch(st, io->N, cv != nullptr, deferred))
-    return cv ? launch_decode_dims<true>(st, io, *cv, Q0, s) : launch_decode_dims<false>(st, io, lq_conv{}, Q0, s);
+  const lq_form form = lq_gdn_decode_form(io->N, st->HV, st->H, st->K, st->V, st->R, st->L, cv != nullptr, deferred,
+                                          lq_num_cus());
+  if (form != LQ_TWO_LAUNCHES) {
+    const bool wide = form == LQ_HELPER_WAVES;
+    return cv ? launch_decode_dims<true>(st, io, *cv, Q0, wide, s)
+              : launch_decode_dims<false>(st, io, lq_conv{}, Q0, wide, s);
+  }
   const int rc = LQ_LAUNCH(step)(st, io, cv, 0, 0.f, nullptr, s);
   return rc ? rc : lq_launch_flush(st, Q0, io->idx, io->N, 0, st->qmax > 0.f ? st->qmax : LQ_QMAX, nullptr, s);
 }

@@ -1,8 +1,8 @@
 """GPU: the one-launch decodes (lq_gdn_decode, lq_kda_decode: the step's workgroups flush the heads whose window they
 fill) against the step followed by the standalone flush on a copy of the state, byte for byte: every head-dim pair and
 GQA factor, window lengths on both sides of a staged half (32 entries), rows whose heads are due together and rows where
-they stand at different fills (one head of a pair due, a head found full, none due), padding rows; launches of up to four
-heads per CU, whose workgroups have helper waves, and larger ones."""
+they stand at different fills (one head of a pair due, a head found full, none due), padding rows; launches of up to two
+and up to four heads per CU, some of whose workgroups have helper waves, and larger ones."""
 import pytest
 import torch
 
@@ -76,7 +76,7 @@ def _check(g, lq, ssm, H, N, rest):
 @pytest.mark.parametrize("K,V", [(128, 128), (64, 128), (64, 64)])
 @pytest.mark.parametrize("GQA", [1, 2, 4])
 @pytest.mark.parametrize("L,R,qmax", [(16, 4, 127.0), (33, 3, 31.0), (64, 4, 127.0), (1, 1, 127.0)])
-@pytest.mark.parametrize("heads", [100, 1100])
+@pytest.mark.parametrize("heads", [100, 700, 1100])
 def test_gdn_one_launch_equals_step_then_flush(K, V, GQA, L, R, qmax, heads):
     g = torch.Generator(device=G.DEV)
     g.manual_seed(K + V + GQA + L + heads)
