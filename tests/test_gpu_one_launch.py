@@ -107,6 +107,16 @@ def test_kda_one_launch_equals_step_then_flush(HV, H, heads, L, R, glb):
     _check(g, lq, ssm, H, N, dict(R=R, kda=True, gate_lower_bound=glb))
 
 
+@pytest.mark.parametrize("N", [64, 70, 130])
+def test_kda_rows_rotated(N):
+    """Two heads per workgroup and 16 workgroups a row at a window of 16: the rounds of 256 workgroups take their rows
+    rotated, with whole and partial rounds."""
+    g = torch.Generator(device=G.DEV)
+    g.manual_seed(N)
+    ssm, lq = _state(g, N + 4, 32, 32, 128, 128, 16, 4, 127.0, kda=True)
+    _check(g, lq, ssm, 32, N, dict(R=4, kda=True))
+
+
 def test_deferred_decode_of_a_large_batch():
     """More than a round of 256 workgroups at a window whose rows are taken rotated: the deferred decode's outputs are the
     immediate one's, and the states agree once the deferred heads are flushed."""
