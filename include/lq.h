@@ -145,10 +145,10 @@ int lq_kda_step(const lq_state* st, const lq_step_io* io, float glb, void* strea
  * it filled (codes in [-qmax, qmax], qmax = st->qmax, 0 meaning 127) -- what lq_kda_step followed by lq_flush (kda = 1)
  * computes, in one call.  Replaces make_kda_step(...)(...) followed by make_flush(..., KDA=True)(...) as
  * LeapQuantState.decode launches them (/root/reference/leapquant/state.py:99-116; kernels.py:694-1075, 1077-2033).
- * One launch, whose workgroups flush the heads they have filled, for small batches: at HV = H up to four heads (rows x
- * HV) per CU; with an even HV of H or 2 H up to eight, and below 16 for windows up to 32.  Everything else (more heads,
- * an odd HV above four per CU, HV / H above 2) runs the step, then the persistent flush (which returns at once when no
- * step raised the due flag st->ctl).  Same limits as lq_kda_step and lq_flush. */
+ * One launch, whose workgroups flush the heads they have filled: at HV = H up to four heads (rows x
+ * HV) per CU; with an even HV of H or 2 H up to eight, and any number for windows up to 32.  Everything else (more
+ * heads, an odd HV above four per CU, HV / H above 2) runs the step, then the persistent flush (which returns at once
+ * when no step raised the due flag st->ctl).  Same limits as lq_kda_step and lq_flush. */
 int lq_kda_decode(const lq_state* st, const lq_step_io* io, float glb, const float* Q0, void* stream);
 
 /* End-of-window flush of every (idx[n] > 0, hv) head whose window is full (hcnt == L): rebuild, one subspace

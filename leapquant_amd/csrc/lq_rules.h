@@ -55,12 +55,14 @@ static inline lq_form lq_gdn_decode_form(int N, int HV, int H, int K, int V, int
 // A token's key is appended once per key head, by its first value head, and the flush of each of the key head's value
 // heads reads it: with the flush in the step's launch, a workgroup therefore holds whole key heads (workgroups of one
 // launch are not ordered, and their XCDs' L2s not coherent), so HV = H for one head per workgroup, and HV / H <= 2 for
-// two.  Sizes, two launches -> one, 32 heads, in step: B = 48 18.6 -> 16.7, B = 64 21.7 -> 20.0, B = 96 27.9 -> 27.3,
-// B = 120 32.7 -> 31.7; W = 64, whose units also meet at each chunk's barriers: B = 48 21.9 -> 21.4, B = 64
-// 25.6 -> 25.7, B = 96 33.9 -> 35.1.  An odd HV above four heads per CU takes two launches.
+// two.  Sizes, two launches -> one, 32 heads, in step [at random fills]: windows of one chunk of the step (32 entries), W = 16:
+// B = 48 17.5 -> 16.0, B = 64 21.1 -> 19.1 [43.4 -> 36.1], B = 128 33.6 -> 33.0 [56.7 -> 50.5], B = 256 58.7 -> 57.8 [81.2 ->
+// 73.0]; W = 32: B = 128 34.6 -> 34.4 [62.0 -> 51.3], B = 256 61.1 -> 60.8 [89.4 -> 75.3]; W = 8: B = 256 63.5 -> 61.9
+// [81.8 -> 79.3].  W = 64, whose units also meet at each chunk's barriers, up to eight heads per CU: B = 48 21.9 -> 21.4,
+// B = 64 25.6 -> 25.7 [44.1 -> 40.3], B = 96 33.9 -> 35.1.  An odd HV above four heads per CU takes two launches.
 static inline int lq_kda_decode_heads(int N, int HV, int H, int L, int cus) {
   const long long heads = (long long)N * HV;
   if (HV == H && heads <= 4ll * cus) return 1;
-  if (HV % 2 == 0 && HV / H <= 2 && (heads <= 8ll * cus || (L <= 32 && heads < 16ll * cus))) return 2;
+  if (HV % 2 == 0 && HV / H <= 2 && (L <= 32 || heads <= 8ll * cus)) return 2;
   return 0;
 }

@@ -83,3 +83,10 @@ def test_wide_ranks_defer_to_a_flush_launch_at_gqa4(rules):
     assert rules.gdn_decode_form(32, 64, 16, 128, 128, 8, 16, 0, 1, 256) == TWO
     assert rules.gdn_decode_form(32, 64, 16, 128, 128, 8, 16, 0, 0, 256) == ONE
     assert rules.gdn_decode_form(32, 32, 16, 128, 128, 8, 16, 0, 1, 256) == ONE
+
+
+@pytest.mark.parametrize("N,HV,H,L,heads", [
+    (32, 32, 32, 16, 1), (33, 32, 32, 16, 2), (64, 32, 32, 64, 2), (65, 32, 32, 64, 0), (65, 32, 32, 33, 0),
+    (256, 32, 32, 32, 2), (1024, 32, 32, 16, 2), (60, 17, 17, 16, 1), (61, 17, 17, 16, 0), (9, 32, 16, 16, 2), (9, 32, 8, 16, 0)])
+def test_kda_lines(rules, N, HV, H, L, heads):
+    assert rules.kda_decode_heads(N, HV, H, L, 256) == heads
