@@ -2,10 +2,15 @@
 fill) against the step followed by the standalone flush on a copy of the state, byte for byte: every head-dim pair and
 GQA factor, window lengths on both sides of a staged half (32 entries), rows whose heads are due together and rows where
 they stand at different fills (one head of a pair due, a head found full, none due), padding rows; launches of up to two
-and up to four heads per CU, some of whose workgroups have helper waves, and larger ones."""
+and up to four heads per CU, some of whose workgroups have helper waves, and larger ones; the same with the conv1d update
+in the step."""
+import ctypes
+
 import pytest
 import torch
 
+from leapquant_amd import _lib
+from leapquant_amd import kernels as KN
 from tests import lqgpu as G
 
 pytestmark = pytest.mark.gpu
@@ -40,9 +45,22 @@ def _state(g, NS, HV, H, K, V, L, R, qmax, kda=False, glb=0.0):
     return ssm, lq
 
 
-def _check(g, lq, ssm, H, N, rest):
+def _step(lq, ssm, mixed, a, b, A_log, dt_bias, idx, out, conv):
+    """The step alone, with the conv update in it if conv = (conv_state, weight, bias)."""
+    if conv is None:
+        v = lq.views(ssm)
+        lq.kstep(v["q32"], v["Sk"], v["Sv"], v["skv"], lq.Kbuf, lq.Ubuf, lq.Wbuf, lq.Pbuf,
+                 *((lq.Gbuf,) if lq.kda else ()), lq.hcnt, mixed, a, b, A_log, dt_bias, v["uq"], idx, out)
+        return
+    st, cv = lq._struct(ssm), KN.conv_struct(*conv)
+    io = KN._step_io(mixed, a, b, A_log, dt_bias, idx, out, lq.kstep_scale)
+    _lib.check(_lib.lib().lq_gdn_step_conv(ctypes.byref(st), ctypes.byref(io), ctypes.byref(cv), KN._stream(mixed)),
+               "lq_gdn_step_conv")
+
+
+def _check(g, lq, ssm, H, N, rest, with_conv=False):
     """Two decode calls (the second steps the windows that the first has reset) of N rows, padding rows among them,
-    against step + flush on a copy of the state."""
+    against step + flush on a copy of the state; with_conv: decode_conv, the conv states compared as well."""
     NS, HV, K, V, L = lq.NS, lq.HV, lq.K, lq.V, lq.L
     ssm2 = ssm.clone()
     lq2 = G.LeapQuantState(ssm2, H, L=L, **rest)
@@ -56,17 +74,24 @@ def _check(g, lq, ssm, H, N, rest):
     bf = lambda *s: torch.randn(*s, device=G.DEV, generator=g).bfloat16()
     KA = K if lq.kda else 1
     A_log, dt_bias = torch.zeros(HV, device=G.DEV), torch.zeros(HV * KA, device=G.DEV)
+    C = 2 * H * K + HV * V
+    conv = conv2 = None
+    if with_conv:                                       # [NS, C, 3] as vLLM's transposed layout holds it
+        conv = (bf(NS, 3, C).transpose(1, 2), bf(C, 4) * 0.5, bf(C) * 0.1)
+        conv2 = (conv[0].clone(),) + conv[1:]
     for _ in range(2):
-        mixed, a, b = bf(N, 2 * H * K + HV * V), bf(N, HV, KA), bf(N, HV)
+        mixed, a, b = bf(N, C), bf(N, HV, KA), bf(N, HV)
         o1 = torch.empty(N, HV, V, device=G.DEV, dtype=torch.bfloat16)
         o2 = torch.empty_like(o1)
-        lq.decode(ssm, mixed, a, b, A_log, dt_bias, idx, o1)
-        v = lq2.views(ssm2)
-        lq2.kstep(v["q32"], v["Sk"], v["Sv"], v["skv"], lq2.Kbuf, lq2.Ubuf, lq2.Wbuf, lq2.Pbuf,
-                  *((lq2.Gbuf,) if lq.kda else ()), lq2.hcnt, mixed, a, b, A_log, dt_bias, v["uq"], idx, o2)
+        if with_conv:
+            lq.decode_conv(ssm, mixed, *conv, True, a, b, A_log, dt_bias, idx, o1)
+        else:
+            lq.decode(ssm, mixed, a, b, A_log, dt_bias, idx, o1)
+        _step(lq2, ssm2, mixed, a, b, A_log, dt_bias, idx, o2, conv2)
         lq2.flush(ssm2, idx)
         torch.cuda.synchronize()
         assert torch.equal(o1, o2)
+        assert not with_conv or torch.equal(conv[0], conv2[0])
         assert torch.equal(ssm.view(torch.int32), ssm2.view(torch.int32))
         for k in bufs:
             assert torch.equal(getattr(lq, k), getattr(lq2, k)), k
@@ -86,13 +111,39 @@ def test_gdn_one_launch_equals_step_then_flush(K, V, GQA, L, R, qmax, heads):
     _check(g, lq, ssm, H, N, dict(R=R, qmax=qmax))
 
 
+@pytest.mark.parametrize("K,V", [(128, 128), (64, 128), (64, 64)])
+@pytest.mark.parametrize("GQA", [1, 2, 4])
+@pytest.mark.parametrize("L,R,qmax", [(16, 4, 127.0), (33, 3, 31.0)])
+@pytest.mark.parametrize("heads", [100, 700, 1100])
+def test_gdn_one_launch_with_conv_equals_step_then_flush(K, V, GQA, L, R, qmax, heads):
+    g = torch.Generator(device=G.DEV)
+    g.manual_seed(K + V + GQA + L + heads + 1)
+    H = 3 if (GQA, heads) == (1, 100) else 4
+    N = max(9, heads // (H * GQA) + 1)
+    ssm, lq = _state(g, N + 4, H * GQA, H, K, V, L, R, qmax)
+    _check(g, lq, ssm, H, N, dict(R=R, qmax=qmax), with_conv=True)
+
+
+@pytest.mark.parametrize("conv", [False, True])
+@pytest.mark.parametrize("R,V,heads", [(4, 128, 100), (4, 128, 700), (4, 128, 1100), (4, 64, 1100), (8, 128, 400)])
+def test_deferred_entry_at_gqa4(R, V, heads, conv):
+    """HV = 4 H: the deferred entry leaves no head full; its calls, in one launch or two, equal step then flush."""
+    g = torch.Generator(device=G.DEV)
+    g.manual_seed(R + V + heads)
+    H, N, K = 4, heads // 16 + 1, 64 if V == 64 else 128
+    ssm, lq = _state(g, N + 4, 4 * H, H, K, V, 16, R, 127.0)
+    lq.defer_flush = True
+    _check(g, lq, ssm, H, N, dict(R=R), with_conv=conv)
+
+
+@pytest.mark.parametrize("conv", [False, True])
 @pytest.mark.parametrize("GQA,L,R", [(1, 16, 8), (2, 16, 8), (2, 33, 8), (2, 64, 8), (4, 16, 8), (4, 64, 8)])
-def test_rank8_one_launch_equals_step_then_flush(GQA, L, R):
+def test_rank8_one_launch_equals_step_then_flush(GQA, L, R, conv):
     g = torch.Generator(device=G.DEV)
     g.manual_seed(GQA + L + R)
     H, N = 3, 30
     ssm, lq = _state(g, N + 4, H * GQA, H, 128, 128, L, R, 127.0)
-    _check(g, lq, ssm, H, N, dict(R=R))
+    _check(g, lq, ssm, H, N, dict(R=R), with_conv=conv)
 
 
 @pytest.mark.parametrize("L,R,glb", [(16, 4, 0.0), (33, 2, -5.0), (64, 4, 0.0), (1, 1, 0.0)])
