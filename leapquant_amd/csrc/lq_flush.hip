@@ -174,11 +174,10 @@ void flush4_kernel(lq_state st, const float* __restrict__ Q0, const int* __restr
 }
 
 // ranks 5 to 8 (GDN 128 x 128 heads)
-template <int RA, int MODE>
+template <int MODE>
 __global__ __launch_bounds__(FT4) __attribute__((amdgpu_waves_per_eu(4)))
-void flush4_kernel(lq_state st, const float* __restrict__ Q0, const int* __restrict__ idx, int N, int* dlist,
-                   float qmax) {
-  static_assert(RA == R8, "eight factor columns");
+void flush8_kernel(lq_state st, const float* __restrict__ Q0, const int* __restrict__ idx, int N, float qmax,
+                   int* dlist) {
   __shared__ FlushShared8 sh;
   auto head = [&](int slot, int hv, unsigned, int* sched) { flush_head8(sh, st, Q0, slot, hv, qmax, sched); };
   if constexpr (MODE == FS_LISTED) flush_listed(sh.due, st, idx, N, dlist, head);
@@ -1021,7 +1020,7 @@ int lq_launch_flush(const lq_state* st, const float* Q0, const int* idx, int N, 
     });
   } else if (st->K == KD && st->R > 4) {
     with_mode(st, dlist, total, g4.x, [&](auto m) {
-      flush4_kernel<8, decltype(m)::value><<<g4, FT4, 0, s>>>(*st, Q0, idx, N, dlist, qmax);
+      flush8_kernel<decltype(m)::value><<<g4, FT4, 0, s>>>(*st, Q0, idx, N, qmax, dlist);
     });
   } else if (st->K == KD) {
     with_mode(st, dlist, total, g4.x, [&](auto m) {

@@ -210,14 +210,11 @@ __device__ __forceinline__ void flush_due(LDS& lds, const lq_state& st, const fl
   }
 }
 
-// RM: factors held per head.  4 (R <= 4): the G R <= 16 factor rows of the workgroup's heads are one MFMA tile, taken
-// by the last wave.  16 (the rank ablation R <= 16, K = V = 128; kernels.py:63, 457-469): up to G tiles, tile g taken
-// by the second wave of head g.
 // The row, and the unit in it, of a one-launch decode's workgroup: block b of `per` blocks a row.  Of the first `rot` rows
 // (rotated_rows; their number is in StepIo, beside the first thing that a workgroup reads), each full round of 256
 // blocks (one per CU) takes its rows rotated by three more than the round before.  `per` a power of two: shifts and masks
 // (four divisions in their place cost config 1 0.6 us a call).
-constexpr int CUS = 256;
+constexpr int CUS = 256;            // a constant, for the shifts; a device with another count only permutes its rows
 struct RowUnit { int n, u; };
 __device__ __forceinline__ RowUnit decode_row(int b, int per, int rot) {
   constexpr int SKEW = 3;
@@ -232,6 +229,9 @@ __device__ __forceinline__ RowUnit decode_row(int b, int per, int rot) {
 
 // Steps the UW units of a workgroup, and returns the mask of its value heads whose window is now full (bit i: value head
 // hk0 G + i of the row), 0 for a padding row; `slot_` is the row's slot.
+// RM: factors held per head.  4 (R <= 4): the G R <= 16 factor rows of the workgroup's heads are one MFMA tile, taken
+// by the last wave.  16 (the rank ablation R <= 16, K = V = 128; kernels.py:63, 457-469): up to G tiles, tile g taken
+// by the second wave of head g.
 // KSH: the key head's value heads are 2^KSH units of G, each a workgroup of its own (FL only).  Each unit with a head to
 // step appends the key, the same bytes to the same row (the heads of a key head that are not full share one fill), so that
 // its own flush finds it whatever the other's workgroup has written.
@@ -735,10 +735,11 @@ void gdn_step_kernel(lq_state st, StepIo io, lq_conv cv, int* dlist, const float
   }
 }
 // the one-launch decode at GQA 1: W = 2 value heads, of two key heads, per workgroup
-template <int K_, int V_, int W, bool CONV>
-__global__ __launch_bounds__(64 * step_wph<V_>() * W) __attribute__((amdgpu_waves_per_eu(4)))
-void gdn_step_kernel(lq_state st, StepIo io, lq_conv cv, const float* Q0) {
-  static_assert(W == step_units<1, true>(), "value heads of a workgroup");
+template <int K_, int V_, bool CONV>
+__global__ __launch_bounds__(128 * step_wph<V_>()) __attribute__((amdgpu_waves_per_eu(4)))
+void gdn_decode_pair_kernel(lq_state st, StepIo io, lq_conv cv, const float* Q0) {
+  constexpr int W = step_units<1, true>();
+  static_assert(W == 2, "value heads of a workgroup");
   __shared__ StepLds<K_, V_, 1, true, 4> lds;
   int slot;
   const unsigned due = gdn_step<K_, V_, 1, CONV, true, W, 4, false>(lds, st, io, cv, nullptr, Q0, slot);
@@ -748,10 +749,11 @@ void gdn_step_kernel(lq_state st, StepIo io, lq_conv cv, const float* Q0) {
     flush_due<K_, V_, 1, W, 1>(lds, st, Q0, slot, hv0, due, code_range(st));
   }
 }
-// the one-launch decode at GQA 4: G = 2 value heads per workgroup, 2^KSH workgroups per key head
-template <int K_, int V_, int G, int KSH>
-__global__ __launch_bounds__(64 * step_wph<V_>() * G) __attribute__((amdgpu_waves_per_eu(4)))
-void gdn_step_kernel(lq_state st, StepIo io, const float* Q0) {
+// the one-launch decode at GQA 4 without conv: G = 2 value heads per workgroup, 2^KSH = 2 workgroups per key head
+template <int K_, int V_>
+__global__ __launch_bounds__(128 * step_wph<V_>()) __attribute__((amdgpu_waves_per_eu(4)))
+void gdn_decode_split_kernel(lq_state st, StepIo io, const float* Q0) {
+  constexpr int G = 2, KSH = 1;
   __shared__ StepLds<K_, V_, G, true, 4> lds;
   int slot;
   const unsigned due = gdn_step<K_, V_, G, false, true, 1, 4, false, KSH>(lds, st, io, lq_conv{}, nullptr, Q0, slot);
@@ -760,12 +762,12 @@ void gdn_step_kernel(lq_state st, StepIo io, const float* Q0) {
     flush_due<K_, V_, G, G, 1>(lds, st, Q0, slot, decode_row(blockIdx.x, st.H << KSH, io.rotated()).u * G, due, code_range(st));
   }
 }
-// the one-launch decode with helper waves: one key head per workgroup, G value heads, 256 G = 128 W threads.  The waves
-// past the step's pass its barriers, and then each group of 256 threads flushes a head.
-template <int K_, int V_, int W, bool CONV, int G>
-__global__ __launch_bounds__(128 * W) __attribute__((amdgpu_waves_per_eu(4)))
-void gdn_step_kernel(lq_state st, StepIo io, lq_conv cv, const float* Q0) {
-  static_assert(W == 2 * G && step_wph<V_>() == 2, "two step waves and two helpers per value head");
+// the one-launch decode with helper waves: one key head per workgroup, G value heads, 256 G threads.  The waves past the
+// step's pass its barriers, and then each group of 256 threads flushes a head.
+template <int K_, int V_, int G, bool CONV>
+__global__ __launch_bounds__(256 * G) __attribute__((amdgpu_waves_per_eu(4)))
+void gdn_decode_wide_kernel(lq_state st, StepIo io, lq_conv cv, const float* Q0) {
+  static_assert(step_wph<V_>() == 2, "two step waves and two helpers per value head");
   __shared__ WideLds<K_, V_, G> lds;
   const RowUnit ru = decode_row(blockIdx.x, st.H, io.rotated());
   const int n = ru.n, hv0 = ru.u * G;
@@ -1251,11 +1253,11 @@ void kda_step_kernel(lq_state st, StepIo io, float glb, int* dlist) {
   unsigned due;
   kda_step<1, false>(nullptr, st, io, glb, dlist, slot, due);
 }
-// the four-wave flush of KDA heads behind their own step: W = 2 heads per workgroup, or (W = 1) one head with two waves
-// that pass the step's barriers and only flush
+// the one-launch KDA decode: the four-wave flush of heads behind their own step, W = 2 heads per workgroup, or (W = 1) one
+// head with two waves that pass the step's barriers and only flush
 template <int W>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
-void flush4_kernel(lq_state st, StepIo io, float glb, const float* Q0) {
+void kda_decode_kernel(lq_state st, StepIo io, float glb, const float* Q0) {
   __shared__ KdaLds<W> lds;
   const RowUnit ru = kda_row<W>(st.HV, io);
   const int n = ru.n, hv0 = ru.u * W;
@@ -1310,9 +1312,11 @@ static int launch_gdn_dims(const lq_state* st, const lq_step_io* io, const lq_co
 // that were admitted one per call fill their windows L calls apart.  Where the two coincide -- at 16 blocks a row and the
 // default window of 16 -- the rows of a CU all flush in the same call, one CU with four flushes beside fifteen with none; the
 // same holds for rows one call apart where a flush is deferred by one.  There the rounds of 256 blocks take their rows
-// rotated by three more each: rows at different fills, W = 16, us per call, in order -> rotated: 61 rows with conv and
+// rotated by three more each: rows one call apart, W = 16, us per call, in order -> rotated: 61 rows with conv and
 // deferred flushes 31.7 -> 26.1, without conv 28.3 -> 22.9; 100 rows of 8 key heads 25.0 -> 21.0.  Elsewhere the rows stay in
-// order (64 such rows at W = 64 24.4 us in order, 24.8 rotated).
+// order (64 such rows at W = 64 24.4 us in order, 24.8 rotated).  Rows at random fills take no harm (61 with conv 25.5 to
+// 26.1 for any rotation, 64 without 23.1 to 23.4).  By 1, 2, 3, 5 or 7 a round: 25.7, 25.7, 25.6, 26.5, 25.4 with conv;
+// 24.4, 23.1, 23.0, 22.6, 22.9 without (two rounds one call apart again meet in a deferred flush at 1).
 static StepIo rotated_rows(const lq_state* st, const lq_step_io* io, int per, bool deferred = false) {
   int rows = 0;                                       // the rows that the rotation covers
   if (per <= CUS && (per & (per - 1)) == 0)
@@ -1326,7 +1330,7 @@ static StepIo rotated_rows(const lq_state* st, const lq_step_io* io, int per, bo
 // the decode call in one launch: each workgroup flushes the heads whose window it fills
 template <int K_, int V_, bool CONV, int G>
 static void launch_wide(const lq_state* st, const lq_step_io* io, const lq_conv& cv, const float* Q0, hipStream_t s) {
-  gdn_step_kernel<K_, V_, 2 * G, CONV, G><<<dim3((unsigned)(io->N * st->H)), 256 * G, 0, s>>>(
+  gdn_decode_wide_kernel<K_, V_, G, CONV><<<dim3((unsigned)(io->N * st->H)), 256 * G, 0, s>>>(
       *st, rotated_rows(st, io, st->H), cv, Q0);
 }
 template <int K_, int V_, bool CONV>
@@ -1338,7 +1342,7 @@ static int launch_decode(const lq_state* st, const lq_step_io* io, const lq_conv
   switch (G) {
     case 1:
       if (wide) launch_wide<K_, V_, CONV, 1>(st, io, cv, Q0, s);
-      else gdn_step_kernel<K_, V_, 2, CONV><<<grid, 128 * step_wph<V_>(), 0, s>>>(*st, rio, cv, Q0);
+      else gdn_decode_pair_kernel<K_, V_, CONV><<<grid, 128 * step_wph<V_>(), 0, s>>>(*st, rio, cv, Q0);
       break;
     case 2:
       if constexpr (V_ == 128) {
@@ -1356,8 +1360,11 @@ static int launch_decode(const lq_state* st, const lq_step_io* io, const lq_conv
           break;
         }
       }
-      if constexpr (CONV) gdn_step_kernel<K_, V_, 4, true, true><<<grid, 256 * step_wph<V_>(), 0, s>>>(*st, rio, cv, nullptr, Q0);
-      else gdn_step_kernel<K_, V_, 2, 1><<<dim3(2u * grid.x), 128 * step_wph<V_>(), 0, s>>>(*st, rotated_rows(st, io, 2 * st->H), Q0);
+      if constexpr (CONV)
+        gdn_step_kernel<K_, V_, 4, true, true><<<grid, 256 * step_wph<V_>(), 0, s>>>(*st, rio, cv, nullptr, Q0);
+      else
+        gdn_decode_split_kernel<K_, V_><<<dim3(2u * grid.x), 128 * step_wph<V_>(), 0, s>>>(
+            *st, rotated_rows(st, io, 2 * st->H), Q0);
       break;
     default: return LQ_ERR_ARG;
   }
@@ -1411,8 +1418,8 @@ int LQ_LAUNCH(gdn_decode)(const lq_state* st, const lq_step_io* io, const lq_con
 int LQ_LAUNCH(kda_decode)(const lq_state* st, const lq_step_io* io, float glb, const float* Q0, hipStream_t s) {
   const unsigned heads = (unsigned)io->N * (unsigned)st->HV;
   switch (lq_kda_decode_heads(io->N, st->HV, st->H, st->L, lq_num_cus())) {
-    case 1: flush4_kernel<1><<<dim3(heads), 256, 0, s>>>(*st, step_io(io), glb, Q0); break;
-    case 2: flush4_kernel<2><<<dim3(heads / 2), 256, 0, s>>>(*st, rotated_rows(st, io, st->HV / 2), glb, Q0); break;
+    case 1: kda_decode_kernel<1><<<dim3(heads), 256, 0, s>>>(*st, step_io(io), glb, Q0); break;
+    case 2: kda_decode_kernel<2><<<dim3(heads / 2), 256, 0, s>>>(*st, rotated_rows(st, io, st->HV / 2), glb, Q0); break;
     default: {
       const int rc = LQ_LAUNCH(step)(st, io, nullptr, 1, glb, nullptr, s);
       return rc ? rc : lq_launch_flush(st, Q0, io->idx, io->N, 1, st->qmax > 0.f ? st->qmax : LQ_QMAX, nullptr, s);

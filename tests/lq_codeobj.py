@@ -79,12 +79,16 @@ def _targs(name):
 # kernel family -> workgroup size of its launch sites, from the template arguments
 LAUNCH_BLOCK = {
     "gdn_step_kernel": lambda t: 128 * int(t[2]),                # <K, V, G, ...>: two waves per value head
+    "gdn_decode_pair_kernel": lambda t: 256,                     # two value heads of two waves
+    "gdn_decode_split_kernel": lambda t: 256,
+    "gdn_decode_wide_kernel": lambda t: 256 * int(t[2]),         # <K, V, G, CONV>: four waves per value head
     "kda_step_kernel": lambda t: 128,
+    "kda_decode_kernel": lambda t: 256,
     "dense_step_kernel": lambda t: 128 * int(t[0]),              # <G, F>
     "conv_update_kernel": lambda t: 256,
     "dequant4_kernel": lambda t: 256,
-    "flush_kernel": lambda t: 512,
     "flush4_kernel": lambda t: 256,
+    "flush8_kernel": lambda t: 256,
     "flush64_kernel": lambda t: 256,
     "quantize_kernel": lambda t: 256,
     "quantize64_kernel": lambda t: 256,

@@ -8,7 +8,8 @@ gfx950 code objects, tests/lq_codeobj.py).
     least one, so every launch can make progress;
   * the kernels of the benchmark's hot path (the one-launch GDN decode, the four-wave GDN and KDA flushes, the KDA
     step) keep the residency they are tuned for (four workgroups per CU for the 256-thread ones, eight for the KDA
-    step).
+    step);
+  * so do the other one-launch decodes (GDN and KDA) and the rank-8 flush, whose register spills are bounded.
 """
 import os
 import shutil
@@ -66,3 +67,28 @@ def test_hot_kernels_keep_their_residency(kernels):
         assert _per_cu(k) >= 4 and k["scratch"] <= 64, (k["name"], _per_cu(k), k["scratch"])
     for k in find("kda_step_kernel"):
         assert _per_cu(k) >= 8 and k["scratch"] == 0, (k["name"], _per_cu(k), k["scratch"])
+
+
+# (kernel, workgroups per CU it is launched for, scratch bytes per lane at most)
+ONE_LAUNCH = ([("gdn_decode_pair_kernel<%s>" % d, 4, 0) for d in ("128, 128, false", "128, 128, true", "64, 128, false",
+                                                                 "64, 128, true", "64, 64, false", "64, 64, true")]
+              + [("gdn_decode_split_kernel<%s>" % d, 4, 0) for d in ("128, 128", "64, 128", "64, 64")]
+              + [("gdn_decode_wide_kernel<%s, %d, %s>" % (d, g, c), 4 // g, 0) for d in ("128, 128", "64, 128")
+                 for g in (1, 2, 4) for c in ("false", "true")]
+              + [("gdn_step_kernel<%s, %d, %s, true, 4, false>" % (d, g, c), 8 // g, 0) for d in ("128, 128", "64, 128")
+                 for g, c in ((2, "false"), (2, "true"), (4, "true"))]
+              + [("gdn_step_kernel<128, 128, 2, %s, true, 4, true>" % c, 4, 0) for c in ("false", "true")]   # deferred
+              + [("gdn_step_kernel<128, 128, %d, %s, true, 16, false>" % (g, c), 8 // g, 48) for g in (2, 4)   # rank 8
+                 for c in ("false", "true")]
+              + [("flush8_kernel<%d>" % m, 4, 48) for m in (0, 1, 2)]
+              + [("kda_decode_kernel<%d>" % w, 4, 32) for w in (1, 2)])
+
+
+@pytest.mark.parametrize("name,per_cu,scratch", ONE_LAUNCH)
+def test_one_launch_kernels_keep_their_residency(kernels, name, per_cu, scratch):
+    """The one-launch decodes and the rank-8 flush: the residency their launch rules are drawn for, and the register spills
+    of this build."""
+    hit = [k for k in kernels if name + "(" in k["name"]]
+    assert hit, name
+    for k in hit:
+        assert _per_cu(k) >= per_cu and k["scratch"] <= scratch, (k["name"], _per_cu(k), k["scratch"])
