@@ -103,9 +103,6 @@ class LeapQuantState:
         else:
             self.kstep = KN.make_gdn_step(NS, HV, H, K, V, L, SS, R=R, qmax=qmax)
         self.kflush = KN.make_flush(NS, HV, K, V, L, SS, R=R, ITERS=1, KDA=kda, NMAX=nmax, qmax=qmax, sched=self.sched)
-        if not kda:                          # the KDA prefill round trip has its own entry points
-            self.kdeq = _make_dequant(NS, HV, K, V, L, SS, buf_dtype=KN.BF16, R=R, qmax=qmax)
-            self.kquant = _make_quantize(NS, HV, K, V, L, SS, R=R, ITERS=1, qmax=qmax)
         self._lib = _lib.lib()
         self._scale = self.kstep_scale
         self._vkey = None
@@ -244,6 +241,22 @@ class LeapQuantState:
         st = self._struct_scan(ssm)
         _lib.check(self._lib.lq_flush(ctypes.byref(st), KN._p(self.Q0), KN._p(idx), idx.shape[0], 1 if self.kda else 0,
                                       ctypes.c_float(self.qmax), KN._stream(idx)), "lq_flush")
+
+    # GDN's dequant and quantize as the factories' callables, which the reference keeps on the state (state.py:80-82): for
+    # callers that use a state's kernels directly; dequantize and quantize go through the state's own lq_state
+    @property
+    def kdeq(self):
+        self._gdn_only("kdeq")
+        return _make_dequant(self.NS, self.HV, self.K, self.V, self.L, self.SS, buf_dtype=KN.BF16, R=self.R, qmax=self.qmax)
+
+    @property
+    def kquant(self):
+        self._gdn_only("kquant")
+        return _make_quantize(self.NS, self.HV, self.K, self.V, self.L, self.SS, R=self.R, ITERS=1, qmax=self.qmax)
+
+    def _gdn_only(self, name):
+        if self.kda:                         # the KDA prefill round trip has its own entry points
+            raise AttributeError("%s: GDN states only" % name)
 
     @property
     def kstep_scale(self):
