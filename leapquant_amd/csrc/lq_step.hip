@@ -795,7 +795,7 @@ void gdn_decode_wide_kernel(lq_state st, StepIo io, lq_conv cv, const float* Q0)
 // One workgroup of two waves per (row n, value head hv); wave wi owns tile rows 64 wi .. 64 wi + 63.  The window --
 // values u_j and keys K_j of the key head in registers, the per-entry step decays e_j in LDS by direct global -> LDS
 // loads -- is taken in chunks of up to KCH = 32 entries, newest first (the decay scan runs from the newest entry
-// back), so that one chunk is held at a time: 17.7 KiB of LDS and <= 128 VGPRs, eight workgroups per CU (the whole
+// back), so that one chunk is held at a time: 17.3 KiB of LDS and <= 128 VGPRs, eight workgroups per CU (the whole
 // window at once needs 26 KiB and 148 VGPRs: six, and the step is bound by the workgroups in flight).  The first
 // chunk's loads precede the int8 tile's, so the first scan, the key dots and A4 / A5 run while the tile streams.
 //   * gate (kernels.py:704-712, 802, 887-896): g = glb sigmoid(e^A_log (a + dt_bias)) (glb != 0) or
