@@ -70,7 +70,7 @@ def _arg(x):
 class CheckingLib:
     """Drop-in for the ctypes handle of liblq.so: checks the footprint of every call, launches nothing."""
 
-    ABI = 5
+    ABI = 6
 
     def __init__(self):
         self.storages = Storages()
@@ -117,8 +117,8 @@ class CheckingLib:
         MIX = 2 * H * K + HV * V
         S.check(what + " idx", io.idx, 0, 4 * io.N)
         S.check(what + " out", io.out, 0, 2 * io.N * HV * V)
-        S.check(what + " A_log", io.A_log, 0, 4 * HV)
-        S.check(what + " dt_bias", io.dt_bias, 0, 4 * HV * KA)
+        S.check(what + " A_log", io.A_log, 0, (2 if io.gate_bf16 & 1 else 4) * HV)
+        S.check(what + " dt_bias", io.dt_bias, 0, (2 if io.gate_bf16 & 2 else 4) * HV * KA)
         for n, slot in enumerate(_ints(io.idx, io.N)):
             if slot <= 0 or slot >= st.NS or (conv is not None and slot >= conv.NS):
                 continue

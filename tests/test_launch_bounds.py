@@ -86,8 +86,8 @@ ONE_LAUNCH = ([("gdn_decode_pair_kernel<%s>" % d, 4, 0) for d in ("128, 128, fal
 
 @pytest.mark.parametrize("name,per_cu,scratch", ONE_LAUNCH)
 def test_one_launch_kernels_keep_their_residency(kernels, name, per_cu, scratch):
-    """The one-launch decodes and the rank-8 flush: the residency their launch rules are drawn for, and the register spills
-    of this build."""
+    """The one-launch decodes and the rank-8 flush: the residency their launch rules are drawn for, and no more register
+    spills than they were measured with."""
     hit = [k for k in kernels if name + "(" in k["name"]]
     assert hit, name
     for k in hit:
